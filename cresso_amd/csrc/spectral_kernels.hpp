@@ -979,17 +979,20 @@ __global__ __launch_bounds__(256) void part_reduce_kernel(
 // S1: sum f^2 over contiguous chunks (float4 loads when aligned)
 // ---------------------------------------------------------------------------
 // Each block also clears its slice of the axis density sums (rows, then
-// columns) for this step's sweep 2.
+// columns) for this step's sweep 2.  With weight decay and the matrix-core
+// sweeps it stores the force (fout, the tangent field's place): they then read
+// 4 bytes an element twice, where grad and param together are 4 (16-bit) or 8.
 template <typename PT, typename GT, bool V4>
 __global__ __launch_bounds__(SP_NT) void sweep1_kernel(
     Geom g, const GT* __restrict__ grad, const PT* __restrict__ param, double* __restrict__ part,
     unsigned long long* __restrict__ rowfx, unsigned long long* __restrict__ colfx, Ctrl* __restrict__ ctrl,
-    const float* __restrict__ fr_state, Lanes L, cresso_hyper h) {
+    const float* __restrict__ fr_state, float* __restrict__ fout, Lanes L, cresso_hyper h) {
     if (L.dv) {
         const cresso_spectral_desc& d = lane_desc(L);
         grad = (const GT*)d.grad; param = (const PT*)d.param; fr_state = (const float*)d.force_rms;
     }
     part = lane_at(part, L); rowfx = lane_at(rowfx, L); colfx = lane_at(colfx, L); ctrl = lane_at(ctrl, L);
+    if (fout) fout = lane_at(fout, L);
     __shared__ float red[4];
     if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->fr_prev = *fr_state;   // every block of sweep 2 reads the old value
     {
@@ -1028,6 +1031,11 @@ __global__ __launch_bounds__(SP_NT) void sweep1_kernel(
                 for (int u = 0; u < UN; ++u)
 #pragma unroll
                     for (int c = 0; c < VW; ++c) f[u][c] = sg * f[u][c] + wd * pv[u][c];
+                if (fout)
+#pragma unroll
+                    for (int u = 0; u < UN; ++u)
+#pragma unroll
+                        for (int c = 0; c < VW; c += 4) St4<float>::go(fout, e + u * st + c, f[u] + c);
             }
 #pragma unroll
             for (int u = 0; u < UN; ++u)
@@ -1045,6 +1053,9 @@ __global__ __launch_bounds__(SP_NT) void sweep1_kernel(
                 LdV<PT, VW>::go(param, e, pv);
 #pragma unroll
                 for (int c = 0; c < VW; ++c) f[c] = sg * f[c] + wd * pv[c];
+                if (fout)
+#pragma unroll
+                    for (int c = 0; c < VW; c += 4) St4<float>::go(fout, e + c, f + c);
             }
 #pragma unroll
             for (int c = 0; c < VW; ++c) {
@@ -1066,7 +1077,10 @@ __global__ __launch_bounds__(SP_NT) void sweep1_kernel(
     // scalar elements: the tail of a vectorized chunk, or the whole chunk
     for (int64_t i = vend + threadIdx.x; i < end; i += SP_NT) {
         float f = sg * ld(grad, i);
-        if (wd_on) f = f + wd * ld(param, i);
+        if (wd_on) {
+            f = f + wd * ld(param, i);
+            if (fout) fout[i] = f;
+        }
         a += f * f;
         m = fmaxf(m, fabsf(f));
     }
@@ -1503,7 +1517,7 @@ __device__ __forceinline__ void stage_rows(const Geom& g, const float* __restric
 // global load of a staged table at once (addresses clamped into the table,
 // so that no branch separates them and one wait covers them all), store()
 // writes the values to LDS.  Up to N values per thread; a larger table takes
-// its remainder in a loop (never on the matrix-core path: panels of 32 or 64
+// its remainder in a loop (never on the matrix-core path: panels of at most 64
 // rows, at most 4 tables of 256 bins).
 template <int N>
 struct Staged {
@@ -1595,6 +1609,7 @@ __device__ __forceinline__ float marg_factor(unsigned long long fx, double inv_h
 }
 
 constexpr int SP_U = 8;  // rows whose loads are in flight together
+constexpr int SP_WCOLS = 64;   // columns of one wave of a matrix-core sweep
 
 // Keeps the scheduler from interleaving the arithmetic of consecutive
 // elements (their loads are already in flight): bounds register pressure.
@@ -1605,16 +1620,13 @@ __device__ __forceinline__ void elem_fence() { __builtin_amdgcn_sched_barrier(0)
 // is addressed as (uniform base pointer) + (32-bit lane offset lr * cols +
 // lane); the planner keeps PR * cols below 2^29.
 __device__ __forceinline__ int64_t panel_base(const Geom& g, const Tile& t) { return t.r0 * g.cols + (int64_t)t.slab * SP_NT; }
-// The tangent / drive field after the matrix-core sweeps, 4-row interleaved:
-// element (R, C) at 4 ((R / 4) cols + C) + R % 4 (rows are a multiple of 4 on
-// that path).  A block's elements (r0 + i, c0 + j) then sit at
-// q4_base + 4 ((i / 4) cols + j) + i % 4, and the four rows 4 lg + r of a
+// The tangent / drive field after the matrix-core sweeps of full tiles, 4-row
+// interleaved: element (R, C) at 4 ((R / 4) cols + C) + R % 4 (rows are a
+// multiple of 4 there).  A panel's elements (r0 + i, C) then sit at
+// r0 cols + 4 ((i / 4) cols + C) + i % 4, and the four rows 4 lg + r of a
 // lane's tile column are one float4.
-__device__ __forceinline__ int64_t q4_base(const Geom& g, const Tile& t) {
-    return t.r0 * g.cols + 4 * (int64_t)t.slab * SP_NT;
-}
-__device__ __forceinline__ uint32_t q4_lane_bytes(uint32_t cols, int lg, int wv, int li) {
-    return 16u * ((uint32_t)lg * cols + 64u * (uint32_t)wv + (uint32_t)li);
+__device__ __forceinline__ uint32_t q4_lane_bytes(uint32_t cols, int lg, uint32_t col) {
+    return 16u * ((uint32_t)lg * cols + col);
 }
 __device__ __forceinline__ uint32_t q4_tile_bytes(uint32_t cols, int tr, int tc) {
     return 16u * (4u * (uint32_t)tr * cols + 16u * (uint32_t)tc);
@@ -1662,13 +1674,13 @@ __device__ __forceinline__ HiSplit hi_split(float ds, float hq, float yk, unsign
 
 // Whether a block's elements may include one whose y reached 2^k: sweep 1's
 // maxima of |f| over the chunks that the block's flat index range [base,
-// base + (nr - 1) cols + SP_NT) touches, with hi_on's margin.  A spike thus
+// base + (nr - 1) cols + width) touches, with hi_on's margin.  A spike thus
 // sends the blocks of its panel rows (not every block) through the
 // high-word pass.  Every thread of the block calls it (a barrier).
 __device__ __forceinline__ bool hi_block(const Geom& g, const double* __restrict__ part1, int64_t base, int nr,
-                                         float inv_s, float eps, float pw, float kmf) {
+                                         int width, float inv_s, float eps, float pw, float kmf) {
     const int64_t c0 = base / g.chunk1;
-    int64_t c1 = (base + (int64_t)(nr - 1) * g.cols + SP_NT - 1) / g.chunk1;
+    int64_t c1 = (base + (int64_t)(nr - 1) * g.cols + width - 1) / g.chunk1;
     c1 = c1 < g.nblk1 - 1 ? c1 : g.nblk1 - 1;
     int hit = 0;
     for (int64_t c = c0 + threadIdx.x; c <= c1; c += SP_NT)
@@ -1822,12 +1834,20 @@ inline bool matrix_cores_enabled() {
     }();
     return on;
 }
-// whether a tensor's step can use the matrix-core sweeps (host side): MODE 1's
-// conditions with 2 or 4 tables
+// whether a tensor's step can use the matrix-core sweeps (host side): 2 or 4
+// tables, at least one panel of whole tiles and one wave of columns
 inline bool mfast_mode(const Geom& g, int hash_on, int axes_on, const cresso_hyper& h) {
-    return hash_on && axes_on && mtables(g) && !g.one_d && h.weight_decay == 0.0 && h.local_sharpness == 0.0 &&
-           (float)fmax(h.instant_metric_power, 0.25) == 1.0f && g.rows % g.PR == 0 && g.cols % SP_NT == 0 &&
-           g.PR % (4 * SP_U) == 0 && matrix_cores_enabled();
+    return hash_on && axes_on && mtables(g) && !g.one_d && h.local_sharpness == 0.0 &&
+           (float)fmax(h.instant_metric_power, 0.25) == 1.0f && g.rows >= g.PR && g.cols >= SP_WCOLS &&
+           g.PR % 16 == 0 && matrix_cores_enabled();
+}
+// their form: full tiles throughout and the grad itself as the force, or
+// edges and a stored force (template argument EDGE, struct MTile).  The
+// general sweeps took 1.7 to 1.9 times as long for both: (50257,768) fp32
+// 775 -> 454 us a step, two bf16 transformer layers with weight decay (18
+// matrices of 2048 and 5632) 1910 -> 1022 us.
+inline bool medge_mode(const Geom& g, const cresso_hyper& h) {
+    return h.weight_decay != 0.0 || g.rows % g.PR != 0 || g.cols % SP_NT != 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1988,7 +2008,7 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep2_kernel(
             if (MODE == 0) elem_fence();
         }
     }
-    if (F.hash_on && hi_on && hi_block(g, part1, base, nr, inv_s, eps, pw, kmf) && t.colok) {
+    if (F.hash_on && hi_on && hi_block(g, part1, base, nr, SP_NT, inv_s, eps, pw, kmf) && t.colok) {
         // high-word pass: the thread's elements again
         const unsigned long long lo_k = to_fixed_u(yk);   // what the loop added for y >= 2^k
         for (int lr = 0; lr < nr; ++lr) {
@@ -2084,6 +2104,48 @@ template <int TT> __device__ __forceinline__ uint32_t bin_byte(uint32_t b, int t
 }
 // projection rows of rank RM in 16-row tiles; carriers in chunks of 4
 template <int RM> constexpr int nqt() { return (2 * RM + 15) / 16; }
+
+// A block's panel and a wave's 64 columns of it in the matrix-core sweeps.
+// EDGE = false: every panel and slab is full.  EDGE = true: the last panel
+// moves up to end at the last row and a wave that would pass the last column
+// moves left to end there, so every load stays inside the tensor whatever its
+// sizes (rows >= PR, cols >= 64); the elements that another block or wave
+// owns (panel rows below rsh, wave columns below csh) count for nothing and
+// are not stored.  A wave wholly past the last column (on = false) skips its
+// loops.  A mask costs two selects an element where every bound is tested by
+// the lane; a copy of the loop for the inner tiles would double the code.
+template <bool EDGE>
+struct MTile {
+    int64_t r0, wcol;   // first row of the panel, first column of the wave
+    int64_t cbase;      // wcol = cbase (the part the block's base pointers hold) + lcol
+    uint32_t lcol;
+    int rsh, csh;
+    bool on;
+    __device__ __forceinline__ MTile(const Geom& g, int wv) {
+        const int slab = blockIdx.x % g.slabs, panel = blockIdx.x / g.slabs;
+        r0 = (int64_t)panel * g.PR;
+        cbase = EDGE ? 0 : (int64_t)slab * SP_NT;
+        wcol = (int64_t)slab * SP_NT + SP_WCOLS * wv;
+        rsh = csh = 0;
+        on = true;
+        if constexpr (EDGE) {
+            const int64_t rmax = g.rows - g.PR, cmax = g.cols - SP_WCOLS;
+            on = wcol < g.cols;
+            if (r0 > rmax) {
+                rsh = (int)(r0 - rmax);
+                r0 = rmax;
+            }
+            if (wcol > cmax) {
+                csh = (int)(wcol - cmax < SP_WCOLS ? wcol - cmax : SP_WCOLS);
+                wcol = cmax;
+            }
+        }
+        lcol = (uint32_t)(EDGE ? wcol : (int64_t)SP_WCOLS * wv);
+    }
+    __device__ __forceinline__ bool owns_row(int lr) const { return !EDGE || lr >= rsh; }
+    __device__ __forceinline__ bool owns_col(int c) const { return !EDGE || c >= csh; }
+    __device__ __forceinline__ int first_tile() const { return EDGE ? rsh >> 4 : 0; }
+};
 
 
 // Inputs of a matrix-core sweep's projection finish: lane group lg's modes
@@ -2184,7 +2246,7 @@ template <int RM, int KC> constexpr int occ3m() { return (RM > 8 || kch<KC>() > 
 template <int RM, int KC> constexpr int occ4m() { return (RM > 8 || kch<KC>() > 3) ? 3 : 4; }
 
 // ---------------------------------------------------------------------------
-// S2 on the matrix cores (MODE 1 tiles, RM <= 16, TT = 2 or 4 tables of
+// S2 on the matrix cores (RM <= 16, TT = 2 or 4 tables of
 // one-byte bins): sweep2_kernel's element math in sweep3m_kernel's tile
 // layout (lane l: rows 4 lg + r of column li of each 16 x 16 tile, 4 tile
 // columns per wave).  The log-density projection Z_q(col) = sum_rows a_q(row)
@@ -2193,9 +2255,9 @@ template <int RM, int KC> constexpr int occ4m() { return (RM > 8 || kch<KC>() > 
 // then each 16-lane row group sums its columns with DPP; column sums stay per
 // lane and tile column until the end.
 // ---------------------------------------------------------------------------
-template <int RM, int KC, typename GT, int TT>
+template <int RM, int KC, typename GT, int TT, bool EDGE>
 __global__ __launch_bounds__(SP_NT, (occ2m<RM, KC>())) void sweep2m_kernel(
-    Geom g, const GT* __restrict__ grad, const float* __restrict__ rowtab, const float* __restrict__ coltab,
+    Geom g, const GT* __restrict__ grad, const float* __restrict__ fbuf, const float* __restrict__ rowtab, const float* __restrict__ coltab,
     const ModeMeta* __restrict__ meta, const unsigned char* __restrict__ bins, Ctrl* __restrict__ ctrl,
     double* __restrict__ part, unsigned long long* __restrict__ hist, unsigned long long* __restrict__ hhi,
     unsigned long long* __restrict__ rowfx, unsigned long long* __restrict__ colfx, const double* __restrict__ part1,
@@ -2204,6 +2266,9 @@ __global__ __launch_bounds__(SP_NT, (occ2m<RM, KC>())) void sweep2m_kernel(
         const cresso_spectral_desc& d = lane_desc(L);
         grad = (const GT*)d.grad; fr_state = (float*)d.force_rms; step = d.step;
     }
+    // the force as sweep 1 stored it (weight decay), else the grad itself
+    if constexpr (EDGE && std::is_same<GT, float>::value)
+        if (fbuf) grad = lane_at(fbuf, L);
     ctrl = lane_at(ctrl, L); part = lane_at(part, L); hist = lane_at(hist, L); hhi = lane_at(hhi, L);
     rowfx = lane_at(rowfx, L); colfx = lane_at(colfx, L); part1 = lane_at(part1, L);
     static_assert(RM <= 16, "two 16-row tiles of projection rows at most");
@@ -2211,21 +2276,22 @@ __global__ __launch_bounds__(SP_NT, (occ2m<RM, KC>())) void sweep2m_kernel(
     constexpr int NQ = nqt<RM>();
     extern __shared__ __align__(16) unsigned char dyn[];
     __shared__ float red[4 * NV2];
-    const Tile t = tile_of(g);
     const int B = g.B;
     const int TB = TT * B;
     const int nr = g.PR;
-    const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int l = threadIdx.x & 63, wv = EDGE ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : threadIdx.x >> 6;
     const int li = l & 15, lg = l >> 4;
+    const MTile<EDGE> t(g, wv);
     ProjCols<NQ> pc;
     pc.modes(g, meta, lg, KC);
-    const int64_t base = panel_base(g, t);
+    const int64_t base = t.r0 * g.cols + t.cbase;
     const uint32_t cols = (uint32_t)g.cols;
     const __amdgpu_buffer_rsrc_t rg = make_rsrc(grad + base, (uint32_t)((int64_t)nr * g.cols * (int64_t)sizeof(GT)));
     const __amdgpu_buffer_rsrc_t rb = make_rsrc(bins + (size_t)TT * base, (uint32_t)((int64_t)nr * g.cols * TT));
-    const uint32_t lane_el = 4u * (uint32_t)lg * cols + 64u * (uint32_t)wv + (uint32_t)li;  // element offset
+    const uint32_t lane_el = 4u * (uint32_t)lg * cols + t.lcol + (uint32_t)li;  // element offset
     const uint32_t vg = lane_el * (uint32_t)sizeof(GT), vb = lane_el * (uint32_t)TT;
     auto tile_off = [&](int tr, int tc, int r) -> uint32_t { return (uint32_t)(16 * tr + r) * cols + 16u * tc; };
+    const int tr0 = t.first_tile();
     // one register set, refilled tile by tile (loads three tiles ahead of use)
     float xv[16];
     uint32_t bv[16];
@@ -2238,7 +2304,7 @@ __global__ __launch_bounds__(SP_NT, (occ2m<RM, KC>())) void sweep2m_kernel(
         }
     };
 #pragma unroll
-    for (int tc = 0; tc < 4; ++tc) load_tile(0, tc);
+    for (int tc = 0; tc < 4; ++tc) load_tile(tr0, tc);
     // LDS: histogram copies [TB][NH] u64 (low words) | row-sum partials [4 waves][PR] | row factors [PR][RW]
     constexpr int NH = SP_NHIST;
     const int hc = (int)(threadIdx.x & (SP_NHIST - 1));
@@ -2257,7 +2323,7 @@ __global__ __launch_bounds__(SP_NT, (occ2m<RM, KC>())) void sweep2m_kernel(
     stage_rows_rest<RM, NRW>(g, rowtab, t.r0, nr, s_ar);
     // the projection finish's carriers (their rows come from the mode table,
     // in registers by now); first used after the loop
-    const int64_t colw = (int64_t)t.slab * SP_NT + 64 * wv;
+    const int64_t colw = t.wcol;
     pc.load(g, coltab, colw, li);
     __syncthreads();
     const F1Values f1 = fin1_values<4>(g, f1p, part1, ctrl, fr_state, step, h);
@@ -2288,10 +2354,13 @@ __global__ __launch_bounds__(SP_NT, (occ2m<RM, KC>())) void sweep2m_kernel(
     float aL = 0.f;
     float cD[4] = {0.f, 0.f, 0.f, 0.f};   // column density sums of the lane's 4 tile columns
     // Sums of log(1 + ds) are kept in log2 units (fin2 scales them by ln 2).
-    const int ntr = nr / 16;   // 2 or 4 (panels of 32 or 64 rows)
+    const int ntr = t.on ? nr / 16 : 0;   // 1, 2 or 4 (panels of 16, 32 or 64 rows)
+    if (EDGE && !t.on)
+        for (int lr = l; lr < nr; lr += 64) s_wrow[wv * g.PR + lr] = 0.f;
 #pragma unroll
     for (int tr = 0; tr < 4; ++tr) {
         if (tr >= ntr) break;
+        if (EDGE && tr < tr0) continue;
         if (one_round) progress_prio(4 * tr / ntr);
         float rs[4] = {0.f, 0.f, 0.f, 0.f};   // this row of tiles' density, per lane row
 #pragma unroll
@@ -2303,9 +2372,10 @@ __global__ __launch_bounds__(SP_NT, (occ2m<RM, KC>())) void sweep2m_kernel(
             for (int r = 0; r < 4; ++r) {
                 // full tile: rel >= eps and instant-metric power 1, so the density is rel
                 // (|sign x| = |x|)
-                const float rel = rel_full(x[r], inv_s, eps);
-                const float ds = fexp2(pw * flog2(rel));
-                const float L = flog2(1.0f + ds);
+                float rel = rel_full(x[r], inv_s, eps);
+                float ds = fexp2(pw * flog2(rel));
+                if (EDGE && !(t.owns_row(16 * tr + 4 * lg + r) && t.owns_col(16 * tc + li))) rel = ds = 0.f;
+                const float L = flog2(1.0f + ds);   // (log2(1) = 0)
                 Ls[r] = L;
                 aL += L;
                 rs[r] += rel;
@@ -2334,13 +2404,17 @@ __global__ __launch_bounds__(SP_NT, (occ2m<RM, KC>())) void sweep2m_kernel(
         for (int r = 0; r < 4; ++r) rt[r] = row16_total(rs[r]);
         if (li < 4) s_wrow[wv * g.PR + 16 * tr + 4 * lg + li] = li == 0 ? rt[0] : (li == 1 ? rt[1] : (li == 2 ? rt[2] : rt[3]));
     }
-    if (hi_on && hi_block(g, part1, base, nr, inv_s, eps, pw, kmf)) {
+    // (from the slab's first column, or a wave's width to the left of it)
+    const int64_t slab0 = (int64_t)(blockIdx.x % g.slabs) * SP_NT;
+    if (hi_on && hi_block(g, part1, t.r0 * g.cols + (EDGE && slab0 > 0 ? slab0 - SP_WCOLS : slab0), nr,
+                          EDGE ? SP_NT + SP_WCOLS : SP_NT, inv_s, eps, pw, kmf)) {
         // high-word pass: the lane's elements again
         const unsigned long long lo_k = to_fixed_u(yk);   // what the loop added for y >= 2^k
-        for (int tr = 0; tr < ntr; ++tr)
+        for (int tr = tr0; tr < ntr; ++tr)
             for (int tc = 0; tc < 4; ++tc)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
+                    if (EDGE && !(t.owns_row(16 * tr + 4 * lg + r) && t.owns_col(16 * tc + li))) continue;
                     const uint32_t o = tile_off(tr, tc, r);
                     const float ds = fexp2(pw * flog2(rel_full(ldg_el<GT>(rg, vg, o * (uint32_t)sizeof(GT)), inv_s, eps)));
                     if (ds * hs >= yk) {
@@ -2357,7 +2431,7 @@ __global__ __launch_bounds__(SP_NT, (occ2m<RM, KC>())) void sweep2m_kernel(
     }
     __syncthreads();
     // axis density sums: one fixed-point atomic per row of this slab and per column of this panel
-    for (int lr = threadIdx.x; lr < nr; lr += SP_NT) {
+    for (int lr = t.rsh + (int)threadIdx.x; lr < nr; lr += SP_NT) {
         float sr = 0.f;
         for (int w = 0; w < SP_NT / 64; ++w) sr += s_wrow[w * g.PR + lr];
         atomicAdd(&rowfx[t.r0 + lr], to_fixed_u(sr * (float)g.hs_row));
@@ -2369,7 +2443,7 @@ __global__ __launch_bounds__(SP_NT, (occ2m<RM, KC>())) void sweep2m_kernel(
         float c = cD[tc];
         c += __shfl_xor(c, 16, 64);
         c += __shfl_xor(c, 32, 64);
-        if (lg == 0) atomicAdd(&colfx[colw + 16 * tc + li], to_fixed_u(c * (float)g.hs_col));
+        if (lg == 0 && t.owns_col(16 * tc + li)) atomicAdd(&colfx[colw + 16 * tc + li], to_fixed_u(c * (float)g.hs_col));
         aD += cD[tc];
     }
     for (int i = threadIdx.x; i < TB; i += SP_NT) {
@@ -2920,7 +2994,7 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep3_kernel(
 
 
 // ---------------------------------------------------------------------------
-// S3 on the matrix cores (MODE 1 tiles, RM <= 16, TT = 2 or 4 tables of
+// S3 on the matrix cores (RM <= 16, TT = 2 or 4 tables of
 // one-byte bins).  The element math is sweep3_kernel's; the contractions run
 // as v_mfma_f32_16x16x4f32 on 16 x 16 tiles, each wave owning 64 columns of
 // the panel as 4 tile columns:
@@ -2940,9 +3014,9 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep3_kernel(
 // within the 256 registers of two waves per SIMD).
 // ---------------------------------------------------------------------------
 template <int KC> constexpr bool bq_in_regs() { return kch<KC>() > 3; }
-template <int RM, int KC, typename GT, int TT>
+template <int RM, int KC, typename GT, int TT, bool EDGE>
 __global__ __launch_bounds__(SP_NT, (occ3m<RM, KC>())) void sweep3m_kernel(
-    Geom g, const GT* __restrict__ grad, const float* __restrict__ rowtab, const float* __restrict__ coltab,
+    Geom g, const GT* __restrict__ grad, int stored, const float* __restrict__ rowtab, const float* __restrict__ coltab,
     const ModeMeta* __restrict__ meta, const unsigned char* __restrict__ bins, const Ctrl* __restrict__ ctrl,
     const float* __restrict__ lt, const unsigned long long* __restrict__ rowfx,
     const unsigned long long* __restrict__ colfx, const float* __restrict__ colfac, float* __restrict__ tbuf,
@@ -2959,26 +3033,35 @@ __global__ __launch_bounds__(SP_NT, (occ3m<RM, KC>())) void sweep3m_kernel(
     constexpr bool BQR = bq_in_regs<KC>();
     extern __shared__ __align__(16) unsigned char dyn[];
     __shared__ float red[4 * NV3];
-    const Tile t = tile_of(g);
     const int B = g.B;
     const int TB = TT * B;
     const int nr = g.PR;
-    const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int l = threadIdx.x & 63, wv = EDGE ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : threadIdx.x >> 6;
     const int li = l & 15, lg = l >> 4;
+    const MTile<EDGE> t(g, wv);
     ProjCols<NQ> pc;
     pc.modes(g, meta, lg, KC);
-    const int64_t base = panel_base(g, t);
+    const int64_t base = t.r0 * g.cols + t.cbase;
     const uint32_t cols = (uint32_t)g.cols;
-    const __amdgpu_buffer_rsrc_t rg = make_rsrc(grad + base, (uint32_t)((int64_t)nr * g.cols * (int64_t)sizeof(GT)));
-    // t goes to the field in the 4-row interleaved layout (q4_base): a lane's
-    // four rows of a tile are one float4, and a wave's store writes whole lines
-    const __amdgpu_buffer_rsrc_t rt = make_rsrc(tbuf + q4_base(g, t), (uint32_t)((int64_t)nr * g.cols * 4));
+    // the force as sweep 1 stored it (weight decay), else the grad itself.
+    // The stored force sits where t goes: an element's lane reads it before
+    // it stores the element's t, and no other lane's value of it counts.
+    const GT* src = grad;
+    if constexpr (EDGE && std::is_same<GT, float>::value)
+        if (stored) src = tbuf;
+    const __amdgpu_buffer_rsrc_t rg = make_rsrc(src + base, (uint32_t)((int64_t)nr * g.cols * (int64_t)sizeof(GT)));
+    // t goes to the field in the 4-row interleaved layout (q4_lane_bytes): a
+    // lane's four rows of a tile are one float4, and a wave's store writes
+    // whole lines.  EDGE: row-major, element by element (any row count, and
+    // in place over a stored force).
+    const __amdgpu_buffer_rsrc_t rt = make_rsrc(tbuf + (EDGE ? base : base + 3 * t.cbase), (uint32_t)((int64_t)nr * g.cols * 4));
     const __amdgpu_buffer_rsrc_t rb = make_rsrc(bins + (size_t)TT * base, (uint32_t)((int64_t)nr * g.cols * TT));
-    const uint32_t lane_el = 4u * (uint32_t)lg * cols + 64u * (uint32_t)wv + (uint32_t)li;  // element offset
+    const uint32_t lane_el = 4u * (uint32_t)lg * cols + t.lcol + (uint32_t)li;  // element offset
     const uint32_t vg = lane_el * (uint32_t)sizeof(GT), vb = lane_el * (uint32_t)TT;
-    const uint32_t vt = q4_lane_bytes(cols, lg, wv, li);
+    const uint32_t vt = EDGE ? 4u * lane_el : q4_lane_bytes(cols, lg, t.lcol + (uint32_t)li);
     // tile (tr, tc), lane element r: panel element (16 tr + 4 lg + r, 64 wv + 16 tc + li)
     auto tile_off = [&](int tr, int tc, int r) -> uint32_t { return (uint32_t)(16 * tr + r) * cols + 16u * tc; };
+    const int tr0 = t.first_tile();
     // one register set, refilled tile by tile: the loads of tile (tr + 1, tc)
     // go out as soon as tile (tr, tc) is done, three tiles ahead of their use
     float xv[16];
@@ -2992,7 +3075,7 @@ __global__ __launch_bounds__(SP_NT, (occ3m<RM, KC>())) void sweep3m_kernel(
         }
     };
 #pragma unroll
-    for (int tc = 0; tc < 4; ++tc) load_tile(0, tc);
+    for (int tc = 0; tc < 4; ++tc) load_tile(tr0, tc);
     // LDS as sweep3_kernel: histogram copies [TB][NH] u64 | log hash metric [TB]
     //      | row metric factor [PR] | (16-aligned) alpha [PR][2][KP] | row factors [PR][RW]
     constexpr int NH = SP_NHIST;
@@ -3017,13 +3100,13 @@ __global__ __launch_bounds__(SP_NT, (occ3m<RM, KC>())) void sweep3m_kernel(
     Staged<NRW> srw;
     srw.template load_rows<RM>(g, rowtab, t.r0, nr);
     const unsigned long long rfx = rowfx[t.r0 + ((int)threadIdx.x < nr ? (int)threadIdx.x : nr - 1)];
-    const int64_t colw = (int64_t)t.slab * SP_NT + 64 * wv;
-    const int64_t c_own = (int64_t)t.slab * SP_NT + threadIdx.x;
+    const int64_t colw = t.wcol;
+    const int64_t c_own = colw + l;
     // the column's axis sum (2-D) or factor (more dims): both loads issued,
     // the unused one through an empty buffer range (reads 0, no branch)
     const bool two_d = g.ntrail == 1;
-    const u32x2 cfx2 = bload2u(make_rsrc(colfx + (int64_t)t.slab * SP_NT, two_d ? SP_NT * 8u : 0u), threadIdx.x * 8u, 0);
-    const float cfac = bload1(make_rsrc(colfac + (int64_t)t.slab * SP_NT, two_d ? 0u : SP_NT * 4u), threadIdx.x * 4u, 0);
+    const u32x2 cfx2 = bload2u(make_rsrc(colfx + colw, two_d ? SP_WCOLS * 8u : 0u), l * 8u, 0);
+    const float cfac = bload1(make_rsrc(colfac + colw, two_d ? 0u : SP_WCOLS * 4u), l * 4u, 0);
     const unsigned long long cfx = ((unsigned long long)cfx2[1] << 32) | cfx2[0];
     float bqr[BQR ? 4 : 1][BQR ? KCH : 1];
     if constexpr (BQR) {
@@ -3068,7 +3151,8 @@ __global__ __launch_bounds__(SP_NT, (occ3m<RM, KC>())) void sweep3m_kernel(
     alpha_rows_m<RM, KC>(g, cs, s_ar, nr, s_al);   // ends with a barrier
     const float cM = ctrl->rconst[0], cP = ctrl->rconst[1];
     // the force's sign (maximize) rides on the denominator: f / den = grad / (sign den)
-    const float sg = h.maximize ? -1.f : 1.f;
+    // (a stored force has its sign)
+    const float sg = h.maximize && !stored ? -1.f : 1.f;
     const float scale_s = sg * ctrl->scale, eps_s = sg * eps;
     const float kM = (float)h.metric_coupling * 1.4426950408889634f;   // exp(c x) = exp2((c log2 e) x)
     const float tm = (float)h.transport_mix;
@@ -3115,6 +3199,16 @@ __global__ __launch_bounds__(SP_NT, (occ3m<RM, KC>())) void sweep3m_kernel(
     // tile's reads find the LDS queue drained.  At four waves per SIMD the
     // extra live registers spill, and the reads stay beside their uses.
     constexpr bool GATHER = RM > 8 || kch<KC>() > 3;
+    auto owns = [&](int tr, int tc, int r) { return t.owns_row(16 * tr + 4 * lg + r) && t.owns_col(16 * tc + li); };
+    auto store_t = [&](int tr, int tc, const float* tv) {
+        if constexpr (EDGE) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (owns(tr, tc, r)) bstore1(rt, vt, 4u * tile_off(tr, tc, r), tv[r]);
+        } else {
+            bstore4(rt, vt, q4_tile_bytes(cols, tr, tc), f32x4{tv[0], tv[1], tv[2], tv[3]});
+        }
+    };
     auto tile = [&](int tr, int tc, const float* x, const uint32_t* b, const f32x4m& lm, const f32x4m& pred) {
         if constexpr (GATHER) {
             const float ec = ecl[16 * tc];
@@ -3145,16 +3239,17 @@ __global__ __launch_bounds__(SP_NT, (occ3m<RM, KC>())) void sweep3m_kernel(
                 float den = scale_s * M;
                 den = den * med3f(rfv[r] * ec, 0.08f, 12.0f);
                 den = den * med3f(hmv[r], 0.08f, 12.0f);
-                const float tv = med3f(x[r] * frcp(den + eps_s), -1.0e4f, 1.0e4f);
+                float tv = med3f(x[r] * frcp(den + eps_s), -1.0e4f, 1.0e4f);
+                float err = tv - pred[r];
+                if (EDGE && !owns(tr, tc, r)) tv = err = 0.f;   // (every sum below then adds 0)
                 tvs[r] = tv;
-                const float err = tv - pred[r];
                 const float P = err + tm * tv;
                 m_ee += err * err;
                 m_t += tv;
                 m_tt += tv * tv;
                 vfx[r] = to_fixed_s(P * hs);
             }
-            bstore4(rt, vt, q4_tile_bytes(cols, tr, tc), f32x4{tvs[0], tvs[1], tvs[2], tvs[3]});
+            store_t(tr, tc, tvs);
 #pragma unroll
             for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -3188,9 +3283,10 @@ __global__ __launch_bounds__(SP_NT, (occ3m<RM, KC>())) void sweep3m_kernel(
 #pragma unroll
                 for (int tt = 1; tt < TT; ++tt) hm *= s_lt[tt * B + bin_byte<TT>(b[r], tt)];
                 den = den * med3f(hm, 0.08f, 12.0f);
-                const float tv = med3f(x[r] * frcp(den + eps_s), -1.0e4f, 1.0e4f);
+                float tv = med3f(x[r] * frcp(den + eps_s), -1.0e4f, 1.0e4f);
+                float err = tv - pred[r];
+                if (EDGE && !owns(tr, tc, r)) tv = err = 0.f;   // (every sum below then adds 0)
                 tvs[r] = tv;
-                const float err = tv - pred[r];
                 const float P = err + tm * tv;
                 m_ee += err * err;
                 m_t += tv;
@@ -3204,7 +3300,7 @@ __global__ __launch_bounds__(SP_NT, (occ3m<RM, KC>())) void sweep3m_kernel(
 #pragma unroll
                 for (int tt = 0; tt < TT; ++tt) atomicAdd(&s_hist[(tt * B + bin_byte<TT>(b[r], tt)) * NH + hc], v);
             }
-            bstore4(rt, vt, q4_tile_bytes(cols, tr, tc), f32x4{tvs[0], tvs[1], tvs[2], tvs[3]});
+            store_t(tr, tc, tvs);
             // A of the projection: a_q(row 16 tr + 4 lg + r), q = 16 qt + li
 #pragma unroll
             for (int qt = 0; qt < NQ; ++qt)
@@ -3219,11 +3315,11 @@ __global__ __launch_bounds__(SP_NT, (occ3m<RM, KC>())) void sweep3m_kernel(
         }
         elem_fence();
     };
-    const int ntr = nr / 16;
+    const int ntr = t.on ? nr / 16 : 0;
     f32x4m lmA, prA, lmB, prB;
-    row_alpha(0);
+    row_alpha(tr0);
     recon(0, lmA, prA);
-    for (int tr = 0; tr < ntr; ++tr) {
+    for (int tr = tr0; tr < ntr; ++tr) {
         if (one_round) progress_prio(4 * tr / ntr);
         // the fields of tile (tr, tc + 1), or of (tr + 1, 0), go to the matrix
         // cores before tile (tr, tc)'s element math, which reads the fields
@@ -3836,55 +3932,65 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep4_kernel(
 // writes the drive without the hash term and sums d^2, d hp and hp^2 for
 // sweep 5).
 // ---------------------------------------------------------------------------
-template <int RM, int KC, int TT, bool Q4>
+template <int RM, int KC, int TT, bool Q4, bool EDGE>
 __global__ __launch_bounds__(SP_NT, (occ4m<RM, KC>())) void sweep4m_kernel(
     Geom g, const float* __restrict__ rowtab, const float* __restrict__ coltab, const ModeMeta* __restrict__ meta,
     const unsigned char* __restrict__ bins, Ctrl* __restrict__ ctrl, const float* __restrict__ imp_tab,
     float* __restrict__ tbuf, double* __restrict__ part, int echo_on, Lanes L, cresso_hyper h, int one_round) {
     ctrl = lane_at(ctrl, L); imp_tab = lane_at(imp_tab, L); tbuf = lane_at(tbuf, L); part = lane_at(part, L);
     static_assert(TT == 2 || TT == 4, "two or four tables of one-byte bins");
+    static_assert(!(Q4 && EDGE), "the interleaved field has full tiles");
     extern __shared__ __align__(16) unsigned char dyn[];
     __shared__ float red[4 * NV4];
-    const Tile t = tile_of(g);
     const int B = g.B;
     const int TB = TT * B;
     const int nr = g.PR;
     constexpr int KP = kcp<KC>();
     constexpr int KCH = kch<KC>();
-    const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int l = threadIdx.x & 63, wv = EDGE ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : threadIdx.x >> 6;
     const int li = l & 15, lg = l >> 4;
-    const int64_t base = panel_base(g, t);
-    // the field: 4-row interleaved after sweep 3m (Q4), row-major after the general sweep 3
-    float* __restrict__ tb = tbuf + (Q4 ? q4_base(g, t) : base);
+    const MTile<EDGE> t(g, wv);
+    const int64_t base = t.r0 * g.cols + t.cbase;
+    // the field: 4-row interleaved after a sweep 3m of full tiles (Q4), else row-major
+    float* __restrict__ tb = tbuf + (Q4 ? base + 3 * t.cbase : base);
     const uint32_t cols = (uint32_t)g.cols;
     const __amdgpu_buffer_rsrc_t rt = make_rsrc(tb, (uint32_t)((int64_t)nr * g.cols * 4));
     const __amdgpu_buffer_rsrc_t rb = make_rsrc(bins + (size_t)TT * base, (uint32_t)((int64_t)nr * g.cols * TT));
-    const uint32_t lane_el = 4u * (uint32_t)lg * cols + 64u * (uint32_t)wv + (uint32_t)li;  // element offset
-    const uint32_t vt = Q4 ? q4_lane_bytes(cols, lg, wv, li) : lane_el * 4u, vb = lane_el * (uint32_t)TT;
+    const uint32_t lane_el = 4u * (uint32_t)lg * cols + t.lcol + (uint32_t)li;  // element offset
+    const uint32_t vt = Q4 ? q4_lane_bytes(cols, lg, t.lcol + (uint32_t)li) : lane_el * 4u, vb = lane_el * (uint32_t)TT;
     // tile (tr, tc), lane element r: panel element (16 tr + 4 lg + r, 64 wv + 16 tc + li)
     auto tile_off = [&](int tr, int tc, int r) -> uint32_t { return (uint32_t)(16 * tr + r) * cols + 16u * tc; };
-    // A row of tiles (4 tiles x 4 elements) is in flight while the previous row
-    // is processed; the first row's loads go out before the block's set-up, so
-    // that memory is busy during it.
-    float xa[16], xb[16];
-    uint32_t ba[16], bb[16];
-    auto load_row = [&](int tr, float* x, uint32_t* b) {
+    // DB: two register sets of a row of tiles (4 tiles x 4 elements), the next
+    // row in flight while one is processed.  Else one set, refilled tile by
+    // tile as in sweep 3m (loads three tiles ahead of their use): 40 registers
+    // fewer at rank 8, where the edge form spills 10 with two sets (sweep 4m of
+    // (50257,768) 112 -> 104 us), and 16 fewer at rank 16 ((8192,8192): 220 ->
+    // 210 us).  The full tiles of rank 8 keep two sets: a lone (2048,2048)
+    // tensor has one wave a SIMD and nothing else to hide its loads (16.5 us,
+    // 18.2 with one set).  The first row's loads go out before the block's
+    // set-up, so that memory is busy during it.
+    constexpr bool DB = RM <= 8 && !EDGE;
+    float xv[DB ? 2 : 1][16];
+    uint32_t bv[DB ? 2 : 1][16];
+    auto load_tile = [&](int tr, int tc, float* x, uint32_t* b) {
+        if constexpr (Q4) {
+            const f32x4 v = bload4(rt, vt, q4_tile_bytes(cols, tr, tc));
 #pragma unroll
-        for (int tc = 0; tc < 4; ++tc) {
-            if constexpr (Q4) {
-                const f32x4 v = bload4(rt, vt, q4_tile_bytes(cols, tr, tc));
+            for (int r = 0; r < 4; ++r) x[4 * tc + r] = v[r];
+        }
 #pragma unroll
-                for (int r = 0; r < 4; ++r) x[4 * tc + r] = v[r];
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const uint32_t o = tile_off(tr, tc, r);
-                if constexpr (!Q4) x[4 * tc + r] = bload1(rt, vt, o * 4u);
-                b[4 * tc + r] = ldg_bins<TT>(rb, vb, o * (uint32_t)TT);
-            }
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t o = tile_off(tr, tc, r);
+            if constexpr (!Q4) x[4 * tc + r] = bload1(rt, vt, o * 4u);
+            b[4 * tc + r] = ldg_bins<TT>(rb, vb, o * (uint32_t)TT);
         }
     };
-    load_row(0, xa, ba);
+    auto load_row = [&](int tr, float* x, uint32_t* b) {
+#pragma unroll
+        for (int tc = 0; tc < 4; ++tc) load_tile(tr, tc, x, b);
+    };
+    const int tr0 = t.first_tile();
+    load_row(tr0, xv[0], bv[0]);
     float* s_imp = reinterpret_cast<float*>(dyn);
     float* s_al = reinterpret_cast<float*>(dyn + ((sizeof(float) * (size_t)g.T * g.B + 15) & ~(size_t)15));
     float* s_rows = s_al + 2 * KP * g.PR;   // the block's row factors [PR][2 RM]
@@ -3904,7 +4010,7 @@ __global__ __launch_bounds__(SP_NT, (occ4m<RM, KC>())) void sweep4m_kernel(
     simp.load(imp_tab, TB);
     double hhv = 0.0;   // four tables, closed form: hh4_kernel's partial of this thread
     if constexpr (TT == 4) hhv = (int)threadIdx.x < hh4_blocks(g) ? ctrl->hh_part[threadIdx.x] : 0.0;
-    const int64_t colw = (int64_t)t.slab * SP_NT + 64 * wv;
+    const int64_t colw = t.wcol;
     float bq[4][KCH];
 #pragma unroll
     for (int tc = 0; tc < 4; ++tc)
@@ -3963,18 +4069,27 @@ __global__ __launch_bounds__(SP_NT, (occ4m<RM, KC>())) void sweep4m_kernel(
 #pragma unroll
             for (int tt = 1; tt < TT; ++tt) hp += s_imp[tt * B + bin_byte<TT>(b[r], tt)];
             hp = hp * invT;
-            const float d = fmaf(c5, hp, fmaf(k_nov, nov, core + mixed[r]));
-            if constexpr (Q4)
+            float d = fmaf(c5, hp, fmaf(k_nov, nov, core + mixed[r]));
+            if constexpr (EDGE) {
+                // (another block's element may already hold its drive: not counted, not stored)
+                if (t.owns_row(16 * tr + 4 * lg + r) && t.owns_col(16 * tc + li))
+                    bstore1(rt, vt, tile_off(tr, tc, r) * 4u, d);
+                else
+                    d = 0.f;
+            } else if constexpr (Q4) {
                 dv[r] = d;
-            else
+            } else {
                 bstore1(rt, vt, tile_off(tr, tc, r) * 4u, d);
+            }
             a_dd = fmaf(d, d, a_dd);
         }
         if constexpr (Q4) bstore4(rt, vt, q4_tile_bytes(cols, tr, tc), f32x4{dv[0], dv[1], dv[2], dv[3]});
         pin1(a_dd);
         elem_fence();
     };
-    auto row_tiles = [&](int tr, const float* x, const uint32_t* b) {
+    const int ntr = t.on ? nr / 16 : 0;
+    // a row of tiles; refill(tc) after each tile
+    auto row_tiles = [&](int tr, const float* x, const uint32_t* b, auto&& refill) {
         if (one_round) progress_prio(64 * tr / nr);   // rows of tiles done of nr / 16
         // A operands of this row of tiles: alpha_{4 kc + lg}(row 16 tr + li)
         const float* __restrict__ alr = s_al + (16 * tr + li) * (2 * KP) + lg;
@@ -3985,14 +4100,25 @@ __global__ __launch_bounds__(SP_NT, (occ4m<RM, KC>())) void sweep4m_kernel(
             aX[kc] = alr[KP + 4 * kc];
         }
 #pragma unroll
-        for (int tc = 0; tc < 4; ++tc) tile(tr, tc, x + 4 * tc, b + 4 * tc, aP, aX);
+        for (int tc = 0; tc < 4; ++tc) {
+            tile(tr, tc, x + 4 * tc, b + 4 * tc, aP, aX);
+            refill(tc);
+        }
     };
-    const int ntr = nr / 16;   // even: PR is a multiple of 32 on this path
-    for (int tr = 0; tr < ntr; tr += 2) {
-        load_row(tr + 1, xb, bb);
-        row_tiles(tr, xa, ba);
-        if (tr + 2 < ntr) load_row(tr + 2, xa, ba);
-        row_tiles(tr + 1, xb, bb);
+    if constexpr (DB) {
+        const auto none = [](int) {};
+        for (int tr = 0; tr + 1 < ntr; tr += 2) {
+            load_row(tr + 1, xv[1], bv[1]);
+            row_tiles(tr, xv[0], bv[0], none);
+            if (tr + 2 < ntr) load_row(tr + 2, xv[0], bv[0]);
+            row_tiles(tr + 1, xv[1], bv[1], none);
+        }
+        if (ntr & 1) row_tiles(ntr - 1, xv[0], bv[0], none);
+    } else {
+        for (int tr = tr0; tr < ntr; ++tr)
+            row_tiles(tr, xv[0], bv[0], [&](int tc) {
+                if (tr + 1 < ntr) load_tile(tr + 1, tc, xv[0], bv[0]);
+            });
     }
     Partials P{red, 1, 1};   // sum drive^2 only: rows of one value (sweep4_kernel's rows hold NV4)
     P.add(0, a_dd);
@@ -4445,17 +4571,19 @@ int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, 
         v4 = v4 && ((uintptr_t)hd[i].grad % (4 * sizeof(GT))) == 0;
     }
     v4 = v4 && pv4;
-    if (v4)
-        hipLaunchKernelGGL((sweep1_kernel<PT, GT, true>), grid1, blk, 0, s, g, grad, param, part1, rowfx, colfx, ctrl,
-                           st.force_rms, L, h);
-    else
-        hipLaunchKernelGGL((sweep1_kernel<PT, GT, false>), grid1, blk, 0, s, g, grad, param, part1, rowfx, colfx, ctrl,
-                           st.force_rms, L, h);
     const bool fast = fast_mode(g, hash_on, axes_on, h);    // MODE 1 tiles of the general sweeps (two tables)
     // the matrix-core sweeps (two or four tables; ranks up to 16: two 16-row projection tiles)
     constexpr bool MX = RM <= 16;
     const bool mf = MX && mfast_mode(g, hash_on, axes_on, h);
-    const bool t4 = g.T == 4;
+    const bool edge = medge_mode(g, h);
+    // with weight decay they read the force that sweep 1 leaves in tbuf
+    float* fout = mf && h.weight_decay != 0.0 ? tbuf : nullptr;
+    if (v4)
+        hipLaunchKernelGGL((sweep1_kernel<PT, GT, true>), grid1, blk, 0, s, g, grad, param, part1, rowfx, colfx, ctrl,
+                           st.force_rms, fout, L, h);
+    else
+        hipLaunchKernelGGL((sweep1_kernel<PT, GT, false>), grid1, blk, 0, s, g, grad, param, part1, rowfx, colfx, ctrl,
+                           st.force_rms, fout, L, h);
     // the matrix-core sweeps write per-block histogram partials (hpart),
     // which part_reduce sums into hist; the general sweeps add into hist
     const bool m2 = mf;
@@ -4475,17 +4603,29 @@ int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, 
     // (direct, or part_reduce's row groups), else copy 0 only
     const int prh = pr_hist_rows(g.T * g.B, g.nblk) > 0;
     const int nc2 = (hd2 || (m2 && prh)) ? g.hcopies : 1, nc3 = (hd3 || (m3 && prh)) ? g.hcopies : 1;
-    if (m2) {
-        if constexpr (MX) {
-            if (t4)
-                hipLaunchKernelGGL((sweep2m_kernel<RM, KC, GT, 4>), grid, blk, l2, s, g, grad, rowtab, coltab, meta, bins,
-                                   ctrl, part, hd2 ? hist : hpart, hhi, rowfx, colfx, part1, st.force_rms, step, L, h,
-                                   one_round2, hd2);
+    // tables, form and force type of the matrix-core sweeps 2 and 3
+    auto with_form = [&](auto&& launch) {
+        using F = float;
+        auto tables = [&](auto gt, auto e, const auto* src) {
+            if (g.T == 4)
+                launch(gt, std::integral_constant<int, 4>{}, e, src);
             else
-                hipLaunchKernelGGL((sweep2m_kernel<RM, KC, GT, 2>), grid, blk, l2, s, g, grad, rowtab, coltab, meta, bins,
-                                   ctrl, part, hd2 ? hist : hpart, hhi, rowfx, colfx, part1, st.force_rms, step, L, h,
-                                   one_round2, hd2);
-        }
+                launch(gt, std::integral_constant<int, 2>{}, e, src);
+        };
+        if (fout)
+            tables(F{}, std::true_type{}, (const F*)fout);
+        else if (edge)
+            tables(GT{}, std::true_type{}, grad);
+        else
+            tables(GT{}, std::false_type{}, grad);
+    };
+    if (m2) {
+        if constexpr (MX)
+            with_form([&](auto gt, auto tt, auto e, const auto* src) {
+                hipLaunchKernelGGL((sweep2m_kernel<RM, KC, decltype(gt), decltype(tt)::value, decltype(e)::value>), grid,
+                                   blk, l2, s, g, src, fout, rowtab, coltab, meta, bins, ctrl, part, hd2 ? hist : hpart,
+                                   hhi, rowfx, colfx, part1, st.force_rms, step, L, h, one_round2, hd2);
+            });
     } else if (fast) {
         hipLaunchKernelGGL((sweep2_kernel<RM, KC, PT, GT, 1>), grid, blk, l2, s, g, grad, param, rowtab, coltab, meta, bins,
                            ctrl, part, hist, rowfx, colfx, hash_on, axes_on, part1, st.force_rms, step, L, h);
@@ -4506,15 +4646,12 @@ int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, 
                            0, s, g, terms, colfac, L);
     }
     if (m3) {
-        if constexpr (MX) {
-            const size_t l3m = lds_sweep3m<KC>(g, 2 * RM);
-            if (t4)
-                hipLaunchKernelGGL((sweep3m_kernel<RM, KC, GT, 4>), grid, blk, l3m, s, g, grad, rowtab, coltab, meta, bins,
-                                   ctrl, lt, rowfx, colfx, colfac, tbuf, part, hd3 ? hist : hpart, L, h, one_round3, hd3);
-            else
-                hipLaunchKernelGGL((sweep3m_kernel<RM, KC, GT, 2>), grid, blk, l3m, s, g, grad, rowtab, coltab, meta, bins,
-                                   ctrl, lt, rowfx, colfx, colfac, tbuf, part, hd3 ? hist : hpart, L, h, one_round3, hd3);
-        }
+        if constexpr (MX)
+            with_form([&](auto gt, auto tt, auto e, const auto* src) {
+                hipLaunchKernelGGL((sweep3m_kernel<RM, KC, decltype(gt), decltype(tt)::value, decltype(e)::value>), grid,
+                                   blk, lds_sweep3m<KC>(g, 2 * RM), s, g, src, fout ? 1 : 0, rowtab, coltab, meta, bins, ctrl, lt,
+                                   rowfx, colfx, colfac, tbuf, part, hd3 ? hist : hpart, L, h, one_round3, hd3);
+            });
     } else if (fast) {
         hipLaunchKernelGGL((sweep3_kernel<RM, KC, PT, GT, 1>), grid, blk, l3, s, g, grad, param, rowtab, coltab, meta, bins,
                            ctrl, lt, rowfx, colfx, colfac, tbuf, part, hist, hash_on, L, h);
@@ -4532,9 +4669,9 @@ int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, 
                        cooc, step, hash_on, hard, echo_on, c5c, nc3, L, h);
     if (c5c == 2)
         hipLaunchKernelGGL(hh4_kernel, dim3((unsigned)hh4_blocks(g), ny), dim3(256), 0, s, g, cooc, counts, imp, ctrl, L);
-    // the field is 4-row interleaved when sweep 3m wrote it (then sweep 4m
-    // runs too, in place, and sweep 5q applies it)
-    const bool q4 = m3 && c5c != 0;
+    // the field is 4-row interleaved when sweep 3m wrote it in full tiles (then
+    // sweep 4m runs too, in place, and sweep 5q applies it)
+    const bool q4 = m3 && c5c != 0 && !edge;
     if (!MX || c5c == 0) {
         if (fast)
             hipLaunchKernelGGL((sweep4_kernel<RM, KC, 1>), grid, blk, l4, s, g, rowtab, coltab, meta, bins, ctrl, imp, tbuf,
@@ -4543,18 +4680,22 @@ int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, 
             hipLaunchKernelGGL((sweep4_kernel<RM, KC, 0>), grid, blk, l4, s, g, rowtab, coltab, meta, bins, ctrl, imp, tbuf,
                                part, hash_on, echo_on, L, h);
     } else if constexpr (MX) {
-        if (c5c == 1 && q4)
-            hipLaunchKernelGGL((sweep4m_kernel<RM, KC, 2, true>), grid, blk, l4, s, g, rowtab, coltab, meta, bins, ctrl,
-                               imp, tbuf, part, echo_on, L, h, one_round4);
-        else if (c5c == 1)
-            hipLaunchKernelGGL((sweep4m_kernel<RM, KC, 2, false>), grid, blk, l4, s, g, rowtab, coltab, meta, bins, ctrl,
-                               imp, tbuf, part, echo_on, L, h, one_round4);
-        else if (q4)
-            hipLaunchKernelGGL((sweep4m_kernel<RM, KC, 4, true>), grid, blk, l4, s, g, rowtab, coltab, meta, bins, ctrl,
-                               imp, tbuf, part, echo_on, L, h, one_round4);
+        auto sweep4 = [&](auto tt, auto q, auto e) {
+            hipLaunchKernelGGL((sweep4m_kernel<RM, KC, decltype(tt)::value, decltype(q)::value, decltype(e)::value>), grid,
+                               blk, l4, s, g, rowtab, coltab, meta, bins, ctrl, imp, tbuf, part, echo_on, L, h, one_round4);
+        };
+        auto form = [&](auto tt) {
+            if (edge)
+                sweep4(tt, std::false_type{}, std::true_type{});
+            else if (q4)
+                sweep4(tt, std::true_type{}, std::false_type{});
+            else
+                sweep4(tt, std::false_type{}, std::false_type{});
+        };
+        if (c5c == 1)
+            form(std::integral_constant<int, 2>{});
         else
-            hipLaunchKernelGGL((sweep4m_kernel<RM, KC, 4, false>), grid, blk, l4, s, g, rowtab, coltab, meta, bins, ctrl,
-                               imp, tbuf, part, echo_on, L, h, one_round4);
+            form(std::integral_constant<int, 4>{});
     }
     const bool hash5 = hash_on && !c5c;   // sweep 5 adds the hash term itself
     const size_t l5 = hash5 ? sizeof(float) * (size_t)g.T * g.B : 0;

@@ -157,19 +157,25 @@ int32_t plan_spectral(const int64_t* shape, int32_t ndim, const int64_t* freqs, 
         return fail(CRESSO_E_UNSUPPORTED, "spectral route: column carrier table too large (%d x %lld)", g.K, (long long)g.cols);
     g.KA = 2 * P.rmax + 2;
     g.RW = 2 * P.rmax;
-    // tiling: 256 columns per block, PR rows per block, ~1024 blocks
+    // tiling: 256 columns per block, PR rows per block
     g.slabs = (int32_t)((g.cols + SP_NT - 1) / SP_NT);
     int64_t pr = std::max<int64_t>(16, (g.rows * g.slabs) / 1024);
     pr = std::min<int64_t>(std::min<int64_t>(pr, 64), g.rows);
-    // the matrix-core sweeps take panels of 32 or 64 rows that tile the rows
-    // exactly: prefer those from 256 rows on (C5's (512,256,3,3) and
-    // (256,256,3,3) conv tensors then take the matrix-core sweeps instead of
-    // the general kernels' 16-row panels: C5 1.32 -> 1.28 ms), 64 rows when
-    // they tile the rows (measured: (5632,2048) 0.174 -> 0.166 ms a step; a
-    // lone (2048,2048) tensor, 256 blocks of 64 rows, is slower, 0.098 ->
-    // 0.107 ms, but C4's batches of them fill the GPU and gain: 12.2-12.3 ->
-    // 12.0-12.1 ms)
-    if (pr >= 16 && g.rows >= 256 && g.rows % 32 == 0) pr = (g.rows % 64 == 0) ? 64 : 32;
+    // The matrix-core sweeps take panels of 16, 32 or 64 rows (a last panel of
+    // fewer rows overlaps the one before it).  Fewer rows make more, shorter
+    // blocks: each repeats the set-up of its tables, and a lone tensor fills
+    // the chip sooner.  us a step of one fp32 tensor, rank 8, with panels of
+    // 16 / 32 / 64 rows: (512,512) 57 / 66 / 82, (1024,1024) 69 / 75 / 91,
+    // (3072,768) 85 / 87 / 95, (2048,2048) 102 / 96 / 104, (5632,2048)
+    // 183 / 174 / 167, (4096,4096) 233 / 215 / 207, (50257,768) 556 / 480 /
+    // 467.  16 rows up to 640 blocks of them, then 32, and 64 from 256 blocks
+    // on: there (2048,2048) alone would gain from 32, but batches of them
+    // lose (a transformer's 88 in one group: 2.4 % of its layers' time).
+    if (mtables(g) && !g.one_d && rank <= 16 && g.rows >= 16 && g.cols >= SP_WCOLS) {
+        const int64_t area = g.rows * g.slabs;
+        pr = area <= 16 * 640 ? 16 : area < 64 * 256 ? 32 : 64;
+        while (pr > g.rows) pr /= 2;
+    }
     // ranks above 16 run the general sweeps, whose per-block LDS (row
     // coefficients of 2 * 68 + 64 floats per panel row) fits with 32-row panels
     if (rank > 16) pr = std::min<int64_t>(pr, 32);
