@@ -17,7 +17,10 @@
 //   D: drive; sum drive^2                     -> drive-energy reservoir, gain
 //   E: param -= lr * cast(drive * gain)
 //
-// Three kernels:
+// The kernels:
+//  * scalar_small_kernel: tensors of at most 16 Ki elements (fp32 work), any
+//    shape, every pass from registers; micro_small_kernel the same for the
+//    micro-field route.
 //  * scalar_resident_kernel: 2D tensors of <= 64 Ki elements whose rows map to
 //    lane groups (LoRA-thin (L,16)) or whose rows are exactly one block wide
 //    ((16,4096)); f, then t, then drive stay on chip (half of each thread's
@@ -27,8 +30,8 @@
 //  * scalar_stream_kernel: every other shape/size/dtype; re-reads the grad in
 //    each pass and keeps general-ndim axis sums as 64-bit fixed-point integers
 //    in a global scratch area (integer atomics: order-independent results).
-//  * micro_kernel: the dense micro-field route (descriptor route 1) of
-//    cresso_v5.py:1355-1432, same plan, table and launch grouping.
+//  * micro_kernel: larger tensors of the dense micro-field route (descriptor
+//    route 1) of cresso_v5.py:1355-1432, same plan, table and launch grouping.
 #include "common.hpp"
 
 #include <algorithm>
@@ -176,6 +179,10 @@ __device__ __forceinline__ void shape3(W t, W iclip, W clip, W clip2, W eps, W& 
     root = fsign(t) * fsqrt((at < clip2 ? at : clip2) + eps);
 }
 
+// Square root in the work dtype (correctly rounded in both).
+__device__ __forceinline__ float wsqrt(float x) { return sqrtf(x); }
+__device__ __forceinline__ double wsqrt(double x) { return sqrt(x); }
+
 // Everything a drive evaluation needs after the pass-C reduction.
 template <typename W> struct DriveCoef {
     W q1, cA, cB, cN, cD, cr, cb, co, ct, nscale;
@@ -188,8 +195,9 @@ template <typename W>
 __device__ DriveCoef<W> contact_and_coefs(const double* M, double dn, const cresso_hyper& h, int step, W q0, W& imp,
                                           W& act, W& sur) {
     const W eps = (W)h.eps;
-    sur = reservoir(sur, (W)sqrt((double)(W)(M[1] / dn) + (double)eps), h.surprise_decay, step);
-    const W port = (W)(M[0] / dn);
+    const double in = 1.0 / dn;
+    sur = reservoir(sur, (W)sqrt((double)(W)(M[1] * in) + (double)eps), h.surprise_decay, step);
+    const W port = (W)(M[0] * in);
     const W S = sur;
     const W dt = (W)h.dt;
     const W plast = (W)1 + (W)h.surprise_gain * S / ((W)1 + S);
@@ -203,9 +211,9 @@ __device__ DriveCoef<W> contact_and_coefs(const double* M, double dn, const cres
     W q1 = q0 + dt * imp;
     q1 = q1 < (W)-8 ? (W)-8 : (q1 > (W)8 ? (W)8 : q1);
 
-    const W frms = (W)sqrt((double)((W)(M[3] / dn) + eps));
-    const W prms = (W)sqrt((double)(q1 * q1 + eps));
-    W align = (W)((double)q1 * M[2] / dn) / (frms * prms + eps);
+    const W frms = wsqrt((W)(M[3] * in) + eps);
+    const W prms = wsqrt(q1 * q1 + eps);
+    W align = (W)((double)q1 * M[2] * in) / (frms * prms + eps);
     align = align < (W)-1 ? (W)-1 : (align > (W)1 ? (W)1 : align);
     W agate = (align + (W)1) * (W)0.5;
     agate = agate < 0 ? (W)0 : (agate > 1 ? (W)1 : agate);
@@ -214,8 +222,8 @@ __device__ DriveCoef<W> contact_and_coefs(const double* M, double dn, const cres
     if (!(sqrt((double)q1 * (double)q1 + h.eps) > sqrt(h.eps))) agate = 0;
     const double warm = h.warmup_steps == 0 ? 1.0 : 1.0 - exp(-(double)step / (double)(h.warmup_steps > 1 ? h.warmup_steps : 1));
     const W mix = (W)(h.prediction_mix * warm) * agate / ((W)1 + S);
-    const W rms_rat = (W)sqrt((double)((W)(M[4] / dn) + eps));
-    const W rms_root = (W)sqrt((double)((W)(M[6] / dn) + eps));
+    const W rms_rat = wsqrt((W)(M[4] * in) + eps);
+    const W rms_root = wsqrt((W)(M[6] * in) + eps);
     const W kroot = rms_rat / (rms_root > eps ? rms_root : eps);
     const W spike = (W)h.spike_mix / ((W)1 + S);
     const W rmix = (W)h.root_channel_mix / ((W)1 + (W)0.5 * S);
@@ -225,17 +233,17 @@ __device__ DriveCoef<W> contact_and_coefs(const double* M, double dn, const cres
     const double Srr = M[4], Sbb = M[5], Soo = M[6], Srb = M[7], Sro = M[8], Sbo = M[9];
     const double Stt = M[3], Str = M[10], Stb = M[11], Sto = M[12];
     const double sh2 = ar * ar * Srr + ab * ab * Sbb + ao * ao * Soo + 2.0 * (ar * ab * Srb + ar * ao * Sro + ab * ao * Sbo);
-    const W srms = (W)sqrt((double)((W)(sh2 / dn) + eps));
+    const W srms = wsqrt((W)(sh2 * in) + eps);
     const W dmix = (W)h.direct_force_mix / ((W)1 + (W)0.35 * S);
     const W kdir = srms / (frms > eps ? frms : eps);
     const double cr = (1.0 - (double)dmix) * ar, cb = (1.0 - (double)dmix) * ab, co = (1.0 - (double)dmix) * ao;
     const double ct = (double)(dmix * kdir);
     const double core2 = cr * cr * Srr + cb * cb * Sbb + co * co * Soo + ct * ct * Stt +
                          2.0 * (cr * cb * Srb + cr * co * Sro + cb * co * Sbo + ct * cr * Str + ct * cb * Stb + ct * co * Sto);
-    const W crms = (W)sqrt((double)((W)(core2 / dn) + eps));
+    const W crms = wsqrt((W)(core2 * in) + eps);
     const double delta = (double)q1 - (double)q0;
     const double ee1 = fmax(M[1] - 2.0 * delta * M[0] + dn * delta * delta, 0.0);
-    const W erms = (W)sqrt((double)((W)(ee1 / dn) + eps));
+    const W erms = wsqrt((W)(ee1 * in) + eps);
     const W resmix = (W)h.residual_feedback_mix / ((W)1 + S);
     const W kres = crms / (erms > eps ? erms : eps);
     DriveCoef<W> c;
@@ -1630,12 +1638,467 @@ __global__ __launch_bounds__(SR_NT) void micro_kernel(const ScalarRec* __restric
 }
 
 // ---------------------------------------------------------------------------
+// small tensors: every pass from registers
+// ---------------------------------------------------------------------------
+// Tensors of at most SS_MAX elements (work dtype fp32), any rank: one
+// 1024-thread workgroup a tensor, K elements a thread (tid + 1024 j), read
+// once with the params and kept in registers through the five passes.  What
+// bounds such a tensor is the chain of its block reductions and the scalar
+// math between them, not its elements:
+//   - a reduction goes through LDS transposed (block_sum_t: every value of
+//     every thread, then one wave a value adds them in fp64), instead of a
+//     DPP tree of fp64 adds per value in every wave;
+//   - the densities wait in LDS, where P threads an entry add them per axis
+//     in fp64 in a fixed order: no atomics, no scratch in memory;
+//   - the serial fp64 chains (metric oscillator, contact oscillator) run on
+//     wave 0 alone, the first while the other waves form the axis factors.
+// us a step of 8 x (8,768) + 8 x (768,8) fp32: 88.4 in two launches (46 on
+// scalar_stream_kernel, 43 on the resident kernel) -> 18.6 in one.
+constexpr int SS_NT = 1024;
+constexpr int64_t SS_MAX = 16 * SS_NT;
+constexpr int64_t SS_AXES = 4096;   // axis entries (factors in LDS)
+constexpr size_t ss_lds(int K) { return sizeof(float) * ((size_t)(K > 13 ? K : 13) * SS_NT + 2 * SS_NT + SS_AXES); }
+
+// Sums of V values over the block in fp64, to every thread; lds: V * SS_NT
+// floats, pub: V doubles.  Wave v adds value v (thread j, j + 64, ... per
+// lane, then the lanes).  Two barriers; lds may be reused after the call.
+template <int V>
+__device__ __forceinline__ void block_sum_t(const float (&x)[V], double (&out)[V], float* lds, double* pub) {
+    static_assert(V <= SS_NT / 64, "a wave per value");
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+    for (int v = 0; v < V; ++v) lds[v * SS_NT + tid] = x[v];
+    __syncthreads();
+    if (wave < V) {
+        const float* row = lds + wave * SS_NT + lane;
+        float y[SS_NT / 64];
+#pragma unroll
+        for (int k = 0; k < SS_NT / 64; ++k) y[k] = row[64 * k];
+        double a = 0.0;
+#pragma unroll
+        for (int k = 0; k < SS_NT / 64; ++k) a += (double)y[k];
+        a = wave_total_d(a);
+        if (lane == 63) pub[wave] = a;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < V; ++v) out[v] = pub[v];
+}
+
+// kappa log2(max(axis mean / gden, eps)) of every axis entry, from the
+// densities sd[i] in LDS, into fac (axis after axis).  P lanes (a power of
+// two) share an entry's elements; waves w0 .. take part.
+__device__ __forceinline__ void ss_axis_factors(const ScalarRec& R, const float* __restrict__ sd, float* __restrict__ fac,
+                                                float gden, float kappa, float eps, int tid, int nt) {
+    const int n = (int)R.d.numel, nd = R.d.ndim;
+    int off = 0;
+    for (int ax = 0; ax < nd; ++ax) {
+        const int D = (int)R.d.shape[ax], st = (int)R.stride[ax], M = n / D;
+        const bool contig = st == M;   // the first axis: an entry's elements are one run
+        int P = 1;
+        while (P < 64 && 2 * P <= M && D * 2 * P <= nt) P *= 2;
+        const int q = tid & (P - 1);
+        for (int e = tid / P; e < D; e += nt / P) {
+            double a = 0.0;
+            if (contig) {
+                for (int m = q; m < M; m += P) a += (double)sd[e * st + m];
+            } else if (st == 1) {
+                for (int m = q; m < M; m += P) a += (double)sd[m * D + e];
+            } else {
+                for (int m = q; m < M; m += P) {
+                    const int o = m / st;
+                    a += (double)sd[(o * D + e) * st + (m - o * st)];
+                }
+            }
+            for (int x = P >> 1; x > 0; x >>= 1) a += __shfl_xor(a, x, 64);
+            const float r = (float)(a / (double)M) / gden;
+            if (q == 0) fac[off + e] = kappa * flog2(r > eps ? r : eps);
+        }
+        off += D;
+    }
+}
+
+// A thread's position in a tensor of rank nd, for its axis factors: 2-D rows
+// and columns advance by SS_NT elements without divisions.
+struct SSWalk {
+    int row, col, dR, dC, C;
+    __device__ __forceinline__ SSWalk(const ScalarRec& R, int tid) {
+        C = R.layout == L_2D ? (int)R.cols : 1;
+        row = tid / C;
+        col = tid - row * C;
+        dR = SS_NT / C;
+        dC = SS_NT - dR * C;
+    }
+    __device__ __forceinline__ void next() {
+        col += dC;
+        row += dR;
+        if (col >= C) {
+            col -= C;
+            ++row;
+        }
+    }
+};
+// sum of element i's log2 axis factors (i < n)
+__device__ __forceinline__ float ss_log_inst(const ScalarRec& R, const float* __restrict__ fac, const SSWalk& w, int i) {
+    if (R.layout == L_2D) return fac[w.row] + fac[(int)R.rows + w.col];
+    float acc = 0.f;
+    for (int ax = 0; ax < R.d.ndim; ++ax)
+        acc += fac[(int)R.axis_off[ax] + (i / (int)R.stride[ax]) % (int)R.d.shape[ax]];
+    return acc;
+}
+
+// clamp of a number; a NaN stays one
+__device__ __forceinline__ float clampn(float x, float lo, float hi) { return x < lo ? lo : (x > hi ? hi : x); }
+// Instant-metric density of one element (cresso_v5.py:243-262)
+__device__ __forceinline__ float ss_density(float rel, float eps, float ipw) {
+    const float r = fmaxf(rel, eps);
+    const float d = ipw == 1.0f ? r : fpow(r, ipw);
+    return fminf(d, 1.0e6f);
+}
+
+template <typename PT, typename GT, int K>
+__device__ __forceinline__ void ss_load(const ScalarRec& R, const void* grad, const cresso_hyper& h, int tid, float (&f)[K],
+                                        float (&pv)[K]) {
+    const int n = (int)R.d.numel;
+    const GT* __restrict__ g = reinterpret_cast<const GT*>(grad);
+    const PT* __restrict__ p = reinterpret_cast<const PT*>(R.d.param);
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        const int i = tid + j * SS_NT, c = i < n ? i : n - 1;   // (clamped: no branch between the loads)
+        f[j] = to_f(g[c]);
+        pv[j] = to_f(p[c]);
+    }
+    const float wd = (float)h.weight_decay;
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        if (h.maximize) f[j] = -f[j];
+        if (h.weight_decay != 0.0) f[j] = f[j] + wd * pv[j];
+        if (tid + j * SS_NT >= n) f[j] = 0.f;
+    }
+}
+
+template <typename PT, typename GT, int K>
+__global__ __launch_bounds__(SS_NT) void scalar_small_kernel(const ScalarRec* __restrict__ recs, int32_t* __restrict__ steps,
+                                                             const void* const* __restrict__ grads, int32_t first,
+                                                             cresso_hyper h) {
+    extern __shared__ __align__(16) float ss_dyn[];
+    __shared__ double pub[13];
+    __shared__ float s_sM;
+    __shared__ DriveCoef<float> s_dc;
+    float* const sx = ss_dyn;                                     // [max(K, 13)][SS_NT]: densities, moments
+    float* const sy = ss_dyn + (K > 13 ? K : 13) * SS_NT;         // [2][SS_NT]
+    float* const fac = sy + 2 * SS_NT;                            // [SS_AXES]
+    const int tid = threadIdx.x, wave = tid >> 6;
+    const int ri = first + blockIdx.x;
+    const ScalarRec& R = recs[ri];
+    const int n = (int)R.d.numel, nd = R.d.ndim, layout = R.layout;
+    float f[K], pv[K];
+    ss_load<PT, GT, K>(R, grads[ri], h, tid, f, pv);
+    const float* const* st = reinterpret_cast<const float* const*>(R.d.state);
+    float q0 = ld_uniform(st[0]), imp = ld_uniform(st[1]), mq = ld_uniform(st[2]), mp = ld_uniform(st[3]);
+    float fr = ld_uniform(st[4]), de = ld_uniform(st[5]), sur = ld_uniform(st[6]), act = ld_uniform(st[7]);
+    const int step = steps[ri] + 1;
+    const double dn = (double)n, in = 1.0 / dn;
+    const float eps = (float)h.eps, pw = (float)h.energy_power, ipw = (float)fmax(h.instant_metric_power, 0.25);
+    const float kappa = nd > 0 ? (float)(h.instant_metric_coupling / ((double)nd * fmax(h.instant_metric_power, 0.25))) : 0.f;
+    const float tq = wave == 0 ? (float)tanh((double)mq) : 0.f;
+
+    // ---- A ----
+    {
+        float a[1] = {0.f};
+        double v[1];
+#pragma unroll
+        for (int j = 0; j < K; ++j) a[0] += f[j] * f[j];
+        block_sum_t<1>(a, v, sx, pub);
+        fr = reservoir(fr, sqrtf((float)(v[0] * in) + eps), h.reservoir_decay, step);
+    }
+    if (tid == 0) steps[ri] = step;   // (every thread read it before the barriers above)
+    const float scale = fmaxf(fr, eps), inv_s = 1.0f / scale;
+    // ---- B ----
+    float gden;
+    {
+        float a[2] = {0.f, 0.f};
+        double v[2];
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+            const float r = fabsf(f[j]) * inv_s + eps;
+            const float d = ss_density(fminf(r, 1.0e4f), eps, ipw);
+            if (tid + j * SS_NT < n) {
+                a[0] += flog1p(fpow(r, pw));
+                a[1] += d;
+            }
+            sx[tid + j * SS_NT] = d;   // (entries past n are not read)
+        }
+        block_sum_t<2>(a, v, sy, pub);
+        gden = (float)fmax(v[1] * in, (double)eps);
+        if (wave == 0) {
+            // scalar metric oscillator (cresso_v5.py:1510-1518)
+            const float mport = (float)(v[0] * in) - tq;
+            mp = mp * (float)fmax(0.0, 1.0 - h.metric_dt * h.metric_friction);
+            mp = mp + (float)h.metric_dt * (mport - mq);
+            mq = mq + (float)h.metric_dt * mp;
+            mq = clampn(mq, -3.0f, 3.0f);
+            const float metric = clampn((float)exp((double)((float)h.metric_coupling * mq)), 0.06f, 16.0f);
+            if (tid == 0) s_sM = scale * metric;
+        }
+        if (layout == L_2D || layout == L_GENERIC) ss_axis_factors(R, sx, fac, gden, kappa, eps, tid, SS_NT);
+    }
+    __syncthreads();
+    const float sM = s_sM;
+    // ---- C ----
+    const float clip = (float)h.drive_clip, iclip = 1.0f / clip, clip2 = clip * clip, k2 = -2.8853900817779268f * iclip;
+    const float ls = (float)h.local_sharpness;
+    const bool ls_on = h.local_sharpness != 0.0;
+    {
+        SSWalk w(R, tid);
+        float m[13] = {0.f};
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+            const int i = tid + j * SS_NT;
+            if (i < n) {
+                float den = sM;
+                if (ls_on) den *= clampn(1.0f + ls * fsqrt(fminf(fabsf(f[j]) * inv_s + eps, 100.0f)), 1.0f, 8.0f);
+                float inst = 1.0f;
+                if (layout == L_1D) {
+                    const float d = ss_density(fminf(fabsf(f[j]) * inv_s + eps, 1.0e4f), eps, ipw);
+                    inst = fexp2(kappa * flog2(fmaxf(d / gden, eps)));
+                } else if (layout != L_NONE) {
+                    inst = fexp2(ss_log_inst(R, fac, w, i));
+                }
+                if (layout != L_NONE) inst = clampn(inst, 0.08f, 12.0f);
+                const float t = clampn(f[j] * frcp(den * inst + eps), -1.0e4f, 1.0e4f);
+                f[j] = t;
+                const float e = t - q0, at = fabsf(t);
+                const Shape3A z = shape3a(at, k2, iclip, clip2, eps);
+                m[0] += e; m[1] += e * e; m[2] += t; m[3] += t * t;
+                m[4] += z.rat * z.rat; m[5] += z.th * z.th; m[6] += z.root * z.root;
+                m[7] += z.rat * z.th; m[8] += z.rat * z.root; m[9] += z.th * z.root;
+                m[10] += at * z.rat; m[11] += at * z.th; m[12] += at * z.root;
+            }
+            w.next();
+        }
+        double M[13];
+        block_sum_t<13>(m, M, sx, pub);
+        if (wave == 0) {
+            // bnd = clip tanh(t / clip)
+            M[5] *= (double)clip * (double)clip;
+            M[7] *= (double)clip; M[9] *= (double)clip; M[11] *= (double)clip;
+            const DriveCoef<float> c = contact_and_coefs<float>(M, dn, h, step, q0, imp, act, sur);
+            if (tid == 0) s_dc = c;
+        }
+        __syncthreads();
+    }
+    // ---- D ----
+    const DriveCoef<float> c = s_dc;
+    {
+        const float cbt = c.cb * clip, cn = c.cN * clip, k2n = -2.8853900817779268f * c.nscale;
+        float a[1] = {0.f};
+        double v[1];
+#pragma unroll
+        for (int j = 0; j < K; ++j)
+            if (tid + j * SS_NT < n) {
+                const float t = f[j], e = t - c.q1, at = fabsf(t);
+                Shape3A z;
+                const float nov = shape3a_nov(at, e, k2, k2n, iclip, clip2, eps, z);
+                const float core = xorsign(fmaf(c.ct, at, fmaf(c.co, z.root, fmaf(cbt, z.th, c.cr * z.rat))), t);
+                const float d = c.cA * core + c.cB + cn * nov + c.cD * e;
+                f[j] = d;
+                a[0] += d * d;
+            }
+        block_sum_t<1>(a, v, sx, pub);
+        de = reservoir(de, (float)(v[0] * in), h.reservoir_decay, step);
+    }
+    const float gain = clampn((float)h.target_update_rms / sqrtf(de + eps), (float)h.min_gain, (float)h.max_gain);
+    // ---- E ----
+    const float nlr = (float)update_alpha<PT>(-h.lr);
+    PT* __restrict__ p = reinterpret_cast<PT*>(R.d.param);
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        const int i = tid + j * SS_NT;
+        if (i < n) p[i] = from_w<PT>(pv[j] + nlr * to_f(from_w<PT>(f[j] * gain)));
+    }
+    if (tid == 0) {
+        float* const* so = reinterpret_cast<float* const*>(R.d.state);
+        *so[0] = c.q1; *so[1] = imp; *so[2] = mq; *so[3] = mp;
+        *so[4] = fr; *so[5] = de; *so[6] = sur; *so[7] = act;
+    }
+}
+
+// The micro-field route of small tensors (at most SS_MAX elements): as
+// scalar_small_kernel, with the three dense fields in registers too (each is
+// read once and written once).  us a step of a coordinate network's 18
+// tensors of up to 64 x 64: 47.0 on micro_kernel -> 18.6; 200 tensors of
+// (126,126) (sixteen elements a thread): 262 -> 46.
+template <typename PT, typename GT, int K>
+__global__ __launch_bounds__(SS_NT) void micro_small_kernel(const ScalarRec* __restrict__ recs, int32_t* __restrict__ steps,
+                                                            const void* const* __restrict__ grads, int32_t first,
+                                                            cresso_hyper h) {
+    extern __shared__ __align__(16) float ss_dyn[];
+    __shared__ double pub[6];
+    float* const sx = ss_dyn;
+    float* const sy = ss_dyn + (K > 13 ? K : 13) * SS_NT;
+    float* const fac = sy + 2 * SS_NT;
+    const int tid = threadIdx.x;
+    const int ri = first + blockIdx.x;
+    const ScalarRec& R = recs[ri];
+    const int n = (int)R.d.numel, nd = R.d.ndim, layout = R.layout;
+    float* __restrict__ gen = reinterpret_cast<float*>(R.d.state[0]);   // micro_energy
+    float* __restrict__ gim = reinterpret_cast<float*>(R.d.state[1]);   // micro_impulse
+    float* __restrict__ grf = reinterpret_cast<float*>(R.d.state[2]);   // micro_refractory
+    float f[K], pv[K], en[K], im[K], rf[K];
+    ss_load<PT, GT, K>(R, grads[ri], h, tid, f, pv);
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        const int i = tid + j * SS_NT, c = i < n ? i : n - 1;
+        en[j] = gen[c];
+        im[j] = gim[c];
+        rf[j] = grf[c];
+    }
+    const float* const* st = reinterpret_cast<const float* const*>(R.d.state);
+    float fr = ld_uniform(st[3]), de = ld_uniform(st[4]), sur = ld_uniform(st[5]);
+    const int step = steps[ri] + 1;
+    const double dn = (double)n, in = 1.0 / dn;
+    const float eps = (float)h.eps, pw = (float)h.energy_power;
+    const double ipw_d = fmax(h.instant_metric_power, 0.25);
+    const float ipw = (float)ipw_d;
+    // cresso_v5.py:1390-1392: the instant-metric coupling is capped at 0.35
+    const float kappa = nd > 0 ? (float)(fmin(0.35, h.instant_metric_coupling) / ((double)nd * ipw_d)) : 0.f;
+
+    // ---- A ----
+    {
+        float a[1] = {0.f};
+        double v[1];
+#pragma unroll
+        for (int j = 0; j < K; ++j) a[0] += f[j] * f[j];
+        block_sum_t<1>(a, v, sx, pub);
+        fr = reservoir(fr, sqrtf((float)(v[0] * in) + eps), h.reservoir_decay, step);
+    }
+    if (tid == 0) steps[ri] = step;
+    const float scale = fmaxf(fr, eps);
+    // ---- B ----
+    const float md = (float)h.micro_decay, md1 = (float)(1.0 - h.micro_decay);
+    float emean, gden;
+    {
+        float a[2] = {0.f, 0.f};
+        double v[2];
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+            const int i = tid + j * SS_NT;
+            const float rel = fminf(fabsf(f[j]) / scale + eps, 1.0e4f);
+            const float src = pw == 1.0f ? rel : fpow(rel, pw);
+            const float d = layout != L_NONE ? ss_density(rel, eps, ipw) : 0.f;
+            en[j] = step <= 1 ? src : en[j] * md + md1 * src;
+            sx[i] = d;
+            if (i < n) {
+                gen[i] = en[j];
+                a[0] += en[j];
+                a[1] += d;
+            }
+        }
+        block_sum_t<2>(a, v, sy, pub);
+        emean = fmaxf((float)(v[0] * in), eps);
+        gden = fmaxf((float)(v[1] * in), eps);
+    }
+    if (layout == L_GENERIC || layout == L_2D) {
+        ss_axis_factors(R, sx, fac, gden, kappa, eps, tid, SS_NT);
+        __syncthreads();
+    }
+    // ---- C ----
+    const bool metric_on = h.hash_metric_coupling != 0.0;
+    const float mpow = (float)(h.hash_metric_coupling / fmax(0.25, h.energy_power));
+    const float clip = (float)h.drive_clip, iclip = 1.0f / clip, clip2 = clip * clip;
+    const float rd = (float)h.refractory_decay, rd1 = (float)(1.0 - h.refractory_decay), rg = (float)h.refractory_gain;
+    const float idk = (float)h.micro_impulse_decay, idk1 = (float)(1.0 - h.micro_impulse_decay);
+    double M[6];
+    {
+        SSWalk w(R, tid);
+        float m[6] = {0.f};
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+            const int i = tid + j * SS_NT;
+            if (i < n) {
+                float metric = 1.0f;
+                if (metric_on) metric = clampn(fpow(en[j] / emean, mpow), 0.08f, 12.0f);
+                float inst = 1.0f;
+                if (layout == L_1D) {
+                    const float d = ss_density(fminf(fabsf(f[j]) / scale + eps, 1.0e4f), eps, ipw);
+                    inst = fexp2(kappa * flog2(fmaxf(d / gden, eps)));
+                } else if (layout != L_NONE) {
+                    inst = fexp2(ss_log_inst(R, fac, w, i));
+                }
+                if (layout != L_NONE) inst = clampn(inst, 0.08f, 12.0f);
+                const float t = clampn(f[j] / (scale * metric * inst + eps), -1.0e4f, 1.0e4f);
+                f[j] = t;
+                const float r = rf[j] * rd + rd1 * fabsf(t);
+                grf[i] = r;
+                const float pr = im[j] * idk + idk1 * (t * (1.0f / (1.0f + rg * r)));
+                gim[i] = pr;
+                im[j] = pr;
+                const float err = t - pr;
+                float rat, bnd, root;
+                shape3(t, iclip, clip, clip2, eps, rat, bnd, root);
+                m[0] += err * err; m[1] += rat * rat; m[2] += rat * bnd;
+                m[3] += bnd * bnd; m[4] += pr * pr; m[5] += t * t;
+            }
+            w.next();
+        }
+        block_sum_t<6>(m, M, sx, pub);
+    }
+    // cresso_v5.py:1406-1425 with every mean(x^2) taken from the sums above;
+    // mean(shaped^2) expands over rat^2, rat*bnd and bnd^2.
+    const float sur_now = sqrtf((float)(M[0] * in) + eps);
+    sur = reservoir(sur, sur_now, h.surprise_decay, step);
+    const float spike = (float)h.spike_mix / (1.0f + sur);
+    const float a1 = 1.0f - spike;
+    const float ssq = (float)(((double)(a1 * a1) * M[1] + 2.0 * (double)(a1 * spike) * M[2] + (double)(spike * spike) * M[3]) * in);
+    const float target = sqrtf(ssq + eps);
+    const float rms_p = sqrtf((float)(M[4] * in) + eps), rms_t = sqrtf((float)(M[5] * in) + eps);
+    const float kp = target / fmaxf(rms_p, eps), kt = target / fmaxf(rms_t, eps), ke = target / fmaxf(sur_now, eps);
+    const float dmix = (float)h.direct_force_mix / (1.0f + 0.35f * sur);
+    const float mmix = (float)h.micro_drive_mix / (1.0f + 0.25f * sur);
+    const float rmix = (float)h.residual_feedback_mix / (1.0f + sur);
+    const float cw = clampn(1.0f - dmix - 0.5f * mmix, 0.0f, 1.0f);
+    const float cR = cw * a1, cBn = cw * spike, cT = dmix * kt, cP = mmix * kp, cE = rmix * ke;
+    // ---- D ----
+    {
+        float a[1] = {0.f};
+        double v[1];
+#pragma unroll
+        for (int j = 0; j < K; ++j)
+            if (tid + j * SS_NT < n) {
+                const float t = f[j], pr = im[j];
+                float rat, bnd, root;
+                shape3(t, iclip, clip, clip2, eps, rat, bnd, root);
+                const float d = cR * rat + cBn * bnd + cT * t + cP * pr + cE * (t - pr);
+                f[j] = d;
+                a[0] += d * d;
+            }
+        block_sum_t<1>(a, v, sx, pub);
+        de = reservoir(de, (float)(v[0] * in), h.reservoir_decay, step);
+    }
+    const float gain = clampn((float)h.target_update_rms / sqrtf(de + eps), (float)h.min_gain, (float)h.max_gain);
+    // ---- E ----
+    const float nlr = (float)update_alpha<PT>(-h.lr);
+    PT* __restrict__ p = reinterpret_cast<PT*>(R.d.param);
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        const int i = tid + j * SS_NT;
+        if (i < n) p[i] = from_w<PT>(pv[j] + nlr * to_f(from_w<PT>(f[j] * gain)));
+    }
+    if (tid == 0) {
+        float* const* so = reinterpret_cast<float* const*>(R.d.state);
+        *so[3] = fr; *so[4] = de; *so[5] = sur;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
 bool is_pow2(int64_t v) { return v > 0 && (v & (v - 1)) == 0; }
 
 struct Variant {
-    int pt, gt, kind;   // kind: 0 stream, 1 resident (row-group or column-block layout), 2 wide stream, 3 micro field
+    int pt, gt, kind;   // kind: 0 stream, 1 resident (row-group or column-block layout), 2 wide stream, 3 micro field,
+                        // 4 small, 5 small micro field
     bool full;          // resident with numel == SR_RESIDENT_MAX: eligible for the FAST kernel
     bool operator==(const Variant& o) const { return pt == o.pt && gt == o.gt && kind == o.kind && full == o.full; }
 };
@@ -1643,6 +2106,12 @@ struct Variant {
 // The FAST resident kernel skips the per-element work of these options.
 bool fast_hyper(const cresso_hyper& h) {
     return h.weight_decay == 0.0 && h.local_sharpness == 0.0 && (float)fmax(h.instant_metric_power, 0.25) == 1.0f;
+}
+
+// Tensors the small kernels take: fp32 work, elements in registers, axis
+// factors in LDS (sum_dims 0: none).
+bool small_ok(const cresso_scalar_desc& d, int64_t sum_dims) {
+    return d.param_dtype != CRESSO_F64 && d.numel <= SS_MAX && sum_dims <= SS_AXES;
 }
 
 int dtype_bytes(int t) { return t == CRESSO_F64 ? 8 : (t == CRESSO_F32 ? 4 : 2); }
@@ -1697,6 +2166,16 @@ int32_t plan_desc(const cresso_scalar_desc& d, const cresso_hyper& h, ScalarRec&
             if (sum > MF_LDS_AXES) scratch = ((size_t)sum * sizeof(unsigned long long) + 255) & ~(size_t)255;
         }
         v = Variant{d.param_dtype, d.grad_dtype, 3, false};
+        if (small_ok(d, r.sum_dims)) {
+            v.kind = 5;
+            scratch = 0;
+            lds = ss_lds(n <= 8 * SS_NT ? 8 : 16);
+            if (d.ndim == 2 && r.layout == L_GENERIC) {
+                r.layout = L_2D;
+                r.rows = d.shape[0];
+                r.cols = d.shape[1];
+            }
+        }
         return CRESSO_OK;
     }
     int kind = 0;
@@ -1711,14 +2190,18 @@ int32_t plan_desc(const cresso_scalar_desc& d, const cresso_hyper& h, ScalarRec&
         const size_t rg_lds = C0 > 0 ? SR_XLDS + ((sizeof(float) * (size_t)d.shape[0] + 15) & ~(size_t)15) +
                                            sizeof(double) * 16 * (size_t)C0 + sizeof(float) * (size_t)C0
                                      : 0;
-        if (res_ok && is_pow2(C0 / 4) && C0 / 4 <= 64 && rg_lds <= SR_LDS_MAX) {
+        int64_t dims = 0;
+        for (int a = 0; a < d.ndim; ++a) dims += d.shape[a];
+        // (the small kernel takes resident shapes too, up to its size)
+        const bool small = small_ok(d, dims);
+        if (!small && res_ok && is_pow2(C0 / 4) && C0 / 4 <= 64 && rg_lds <= SR_LDS_MAX) {
             r.layout = L_ROWGROUP;
             r.group = (int32_t)(C0 / 4);
             r.rows = d.shape[0];
             r.cols = C0;
             kind = 1;
             lds = rg_lds;
-        } else if (res_ok && C0 == (int64_t)SR_NT * 4) {
+        } else if (!small && res_ok && C0 == (int64_t)SR_NT * 4) {
             r.layout = L_COLBLOCK;
             r.rows = d.shape[0];
             r.cols = C0;
@@ -1747,7 +2230,12 @@ int32_t plan_desc(const cresso_scalar_desc& d, const cresso_hyper& h, ScalarRec&
             scratch = (scratch + 255) & ~(size_t)255;
         }
     }
+    if (kind == 0 && small_ok(d, r.sum_dims)) {
+        kind = 4;
+        scratch = 0;
+    }
     if (kind == 0 && n >= SR_WIDE_MIN) kind = 2;
+    if (kind == 4) lds = ss_lds(n <= 8 * SS_NT ? 8 : 16);
     r.resident = kind == 1;
     v = Variant{d.param_dtype, d.grad_dtype, kind, kind == 1 && n == SR_RESIDENT_MAX};
     return CRESSO_OK;
@@ -1787,6 +2275,32 @@ hipError_t launch_resident(bool fast, const ScalarRec* recs, int32_t* steps, con
     if (lds > SR_LDS_MAX) return hipErrorInvalidValue;
     return fast ? launch_resident_v<PT, GT, true>(recs, steps, grads, first, cnt, lds, h, s)
                 : launch_resident_v<PT, GT, false>(recs, steps, grads, first, cnt, lds, h, s);
+}
+
+// One launch for a group's small tensors: eight elements a thread where the
+// largest has at most 8192, else sixteen.
+template <typename PT, typename GT, int K>
+hipError_t launch_small_k(bool micro, const ScalarRec* recs, int32_t* steps, const void* const* grads, int32_t first,
+                          int32_t cnt, const cresso_hyper& h, hipStream_t s) {
+    static const hipError_t e = [] {
+        const hipError_t a = hipFuncSetAttribute(reinterpret_cast<const void*>(&scalar_small_kernel<PT, GT, K>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)ss_lds(K));
+        const hipError_t b = hipFuncSetAttribute(reinterpret_cast<const void*>(&micro_small_kernel<PT, GT, K>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)ss_lds(K));
+        return a != hipSuccess ? a : b;
+    }();
+    if (e != hipSuccess) return e;
+    if (micro)
+        hipLaunchKernelGGL((micro_small_kernel<PT, GT, K>), dim3(cnt), dim3(SS_NT), ss_lds(K), s, recs, steps, grads, first, h);
+    else
+        hipLaunchKernelGGL((scalar_small_kernel<PT, GT, K>), dim3(cnt), dim3(SS_NT), ss_lds(K), s, recs, steps, grads, first, h);
+    return hipGetLastError();
+}
+template <typename PT, typename GT>
+hipError_t launch_small(bool micro, bool k16, const ScalarRec* recs, int32_t* steps, const void* const* grads, int32_t first,
+                        int32_t cnt, const cresso_hyper& h, hipStream_t s) {
+    return k16 ? launch_small_k<PT, GT, 16>(micro, recs, steps, grads, first, cnt, h, s)
+               : launch_small_k<PT, GT, 8>(micro, recs, steps, grads, first, cnt, h, s);
 }
 
 template <typename W, typename PT, typename GT>
@@ -1836,6 +2350,20 @@ hipError_t dispatch(const Variant& v, const ScalarRec* recs, int32_t* steps, con
         if (v.pt == CRESSO_BF16)
             return launch_resident<__hip_bfloat16, __hip_bfloat16>(fast, recs, steps, grads, first, cnt, lds, h, s);
         if (v.pt == CRESSO_F16) return launch_resident<__half, __half>(fast, recs, steps, grads, first, cnt, lds, h, s);
+        return hipErrorInvalidValue;
+    }
+    if (v.kind >= 4) {
+#define CRESSO_SS_CASE(PC, GC, PT, GT)                                                                               \
+    if (v.pt == PC && v.gt == GC)                                                                                    \
+        return launch_small<PT, GT>(v.kind == 5, lds > ss_lds(8), recs, steps, grads, first, cnt, h, s);
+        CRESSO_SS_CASE(CRESSO_F32, CRESSO_F32, float, float)
+        CRESSO_SS_CASE(CRESSO_BF16, CRESSO_BF16, __hip_bfloat16, __hip_bfloat16)
+        CRESSO_SS_CASE(CRESSO_F16, CRESSO_F16, __half, __half)
+        CRESSO_SS_CASE(CRESSO_BF16, CRESSO_F32, __hip_bfloat16, float)
+        CRESSO_SS_CASE(CRESSO_F16, CRESSO_F32, __half, float)
+        CRESSO_SS_CASE(CRESSO_F32, CRESSO_BF16, float, __hip_bfloat16)
+        CRESSO_SS_CASE(CRESSO_F32, CRESSO_F16, float, __half)
+#undef CRESSO_SS_CASE
         return hipErrorInvalidValue;
     }
 #define CRESSO_SR_CASE(PC, GC, W, PT, GT)                                                                            \

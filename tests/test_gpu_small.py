@@ -1,0 +1,54 @@
+"""The register kernels of small tensors (scalar and micro-field routes) at the
+edges of their range: one element, one past a thread's share, the largest
+tensors of eight and sixteen elements a thread and the first past them, axes
+whose factors just fit in LDS, every rank, against the CPU oracle."""
+
+import pytest
+import torch
+
+from gpu_util import BF16_PARAM_TOL, F32_TOL, announce, compare, needs_gpu, run_pair
+
+pytestmark = [pytest.mark.gpu, needs_gpu]
+
+KW = dict(lr=2e-3, rank=4, hash_bins=64, hash_tables=2, min_spectral_size=1 << 30)
+OPTIONS = dict(KW, weight_decay=0.02, maximize=True, local_sharpness=0.3, instant_metric_power=0.7, warmup_steps=0)
+SHAPES = [(), (1,), (1, 1), (1, 7), (1023,), (1025,), (64, 16), (33, 31), (8, 1024), (8193,), (16384,), (4, 4096),
+          (16385,), (5, 3276), (1, 4095), (1, 4096), (2, 8192), (3, 5, 7), (2, 4, 1000), (16, 8, 3, 3), (2, 3, 2, 5, 3)]
+
+
+@pytest.mark.parametrize("kw", [KW, OPTIONS, dict(KW, instant_metric_coupling=0.0)], ids=["plain", "options", "no_axes"])
+def test_small_scalar_tensors_match_oracle(kw):
+    announce(f"small scalar tensors {sorted(set(kw) - set(KW))}")
+    compare(*run_pair(SHAPES, torch.float32, kw, steps=3, seed=41))
+
+
+@pytest.mark.parametrize("kw", [KW, dict(KW, weight_decay=0.02, maximize=True, instant_metric_power=0.7, energy_power=1.0)],
+                         ids=["plain", "options"])
+def test_small_micro_tensors_match_oracle(kw):
+    announce("small micro tensors")
+    shapes = [s for s in SHAPES if s != ()]
+    compare(*run_pair(shapes, torch.float32, dict(kw, micro_field_max_size=20000), steps=3, seed=42))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("micro", [0, 20000], ids=["scalar", "micro"])
+def test_small_half_dtypes_first_step(dtype, micro):
+    announce(f"small {dtype} micro {micro}")
+    res = run_pair([(1,), (1025,), (33, 31), (4, 4096), (3, 5, 7)], dtype, dict(KW, micro_field_max_size=micro), steps=1,
+                   seed=43, grad_std=0.05, param_std=0.05)
+    compare(*res, param_tol=BF16_PARAM_TOL, state_tol=F32_TOL)
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_small_tensor_with_a_bad_gradient_has_no_number_left(bad):
+    """One NaN or infinite gradient element: the reservoirs and every updated value become NaN, as in the reference."""
+    import cresso_amd
+
+    p = torch.nn.Parameter(0.02 * torch.randn(40, 50, device="cuda"))
+    p.grad = 1e-3 * torch.randn_like(p)
+    p.grad[3, 7] = bad
+    opt = cresso_amd.CRESSO5([p], cuda_ops="required", **KW)
+    opt.step()
+    torch.cuda.synchronize()
+    assert not torch.isfinite(opt.state[p]["force_rms"])
+    assert not torch.isfinite(p).any()
