@@ -72,11 +72,16 @@ __device__ __forceinline__ float uni(float v) {
 __device__ __forceinline__ void sched_fence() { __builtin_amdgcn_sched_barrier(0); }
 // Read of a value that every thread of the block reads at the same address
 // (a 0-dim state tensor): a scalar load through the constant address space.
-// Each value is read once, before this kernel writes it back at its end.
+// One thread writes the state back at the kernel's end, and the compiler may
+// move a constant load down to its use, past every barrier: a wave held up
+// there would read the new value.  hold() the values before the first barrier.
 __device__ __forceinline__ float ld_uniform(const float* p) {
     return *(const __attribute__((address_space(4))) float*)p;
 }
 
+
+// The value is read by here and not read again.
+__device__ __forceinline__ void hold(float& v) { asm volatile("" : "+s"(v)); }
 
 // ---- vector access -------------------------------------------------------
 template <typename T> struct V4;
@@ -366,6 +371,7 @@ __device__ __forceinline__ void resident_body(const ScalarRec* __restrict__ recs
         for (int c = 0; c < 4; ++c) a_ff += v[c] * v[c];
         stx(k, v);
     }
+    hold(q0); hold(imp); hold(mq); hold(mp); hold(fr); hold(de); hold(sur); hold(act);
     __syncthreads();
     const int step = s_step;
     const double dn = (double)n;
@@ -1797,7 +1803,9 @@ __global__ __launch_bounds__(SS_NT) void scalar_small_kernel(const ScalarRec* __
     const float* const* st = reinterpret_cast<const float* const*>(R.d.state);
     float q0 = ld_uniform(st[0]), imp = ld_uniform(st[1]), mq = ld_uniform(st[2]), mp = ld_uniform(st[3]);
     float fr = ld_uniform(st[4]), de = ld_uniform(st[5]), sur = ld_uniform(st[6]), act = ld_uniform(st[7]);
-    const int step = steps[ri] + 1;
+    int step = __builtin_amdgcn_readfirstlane(steps[ri]) + 1;
+    hold(q0); hold(imp); hold(mq); hold(mp); hold(fr); hold(de); hold(sur); hold(act);
+    asm volatile("" : "+s"(step));
     const double dn = (double)n, in = 1.0 / dn;
     const float eps = (float)h.eps, pw = (float)h.energy_power, ipw = (float)fmax(h.instant_metric_power, 0.25);
     const float kappa = nd > 0 ? (float)(h.instant_metric_coupling / ((double)nd * fmax(h.instant_metric_power, 0.25))) : 0.f;
@@ -1956,7 +1964,9 @@ __global__ __launch_bounds__(SS_NT) void micro_small_kernel(const ScalarRec* __r
     }
     const float* const* st = reinterpret_cast<const float* const*>(R.d.state);
     float fr = ld_uniform(st[3]), de = ld_uniform(st[4]), sur = ld_uniform(st[5]);
-    const int step = steps[ri] + 1;
+    int step = __builtin_amdgcn_readfirstlane(steps[ri]) + 1;
+    hold(fr); hold(de); hold(sur);
+    asm volatile("" : "+s"(step));
     const double dn = (double)n, in = 1.0 / dn;
     const float eps = (float)h.eps, pw = (float)h.energy_power;
     const double ipw_d = fmax(h.instant_metric_power, 0.25);

@@ -52,3 +52,37 @@ def test_small_tensor_with_a_bad_gradient_has_no_number_left(bad):
     torch.cuda.synchronize()
     assert not torch.isfinite(opt.state[p]["force_rms"])
     assert not torch.isfinite(p).any()
+
+
+@pytest.mark.parametrize("shape", [(4096, 16), (16, 4096), (2048, 16), (768, 8)])
+def test_scalar_step_beside_another_streams_work_is_bit_identical(shape):
+    """The one-workgroup kernels beside spectral steps on another stream, whose blocks hold some of a workgroup's waves
+    up for microseconds, against the same steps on an idle GPU: no wave may read a state value that another has
+    already written back."""
+    import cresso_amd
+
+    announce(f"scalar {shape} beside a side stream")
+    kw = dict(rank=8, hash_bins=64, hash_tables=2, cuda_ops="required")
+    gen = torch.Generator().manual_seed(44)
+    p0 = [0.02 * torch.randn(shape, generator=gen) for _ in range(4)]
+    grads = [[(1e-3 * torch.randn(shape, generator=gen)).cuda() for _ in p0] for _ in range(4)]
+    quiet = [torch.nn.Parameter(p.cuda()) for p in p0]
+    busy = [torch.nn.Parameter(p.cuda()) for p in p0]
+    opts = [cresso_amd.CRESSO5(quiet, **kw), cresso_amd.CRESSO5(busy, **kw)]
+    other = torch.nn.Parameter(0.02 * torch.randn(256, 512, device="cuda"))
+    other.grad = 1e-3 * torch.randn_like(other)
+    load = cresso_amd.CRESSO5([other], **kw)
+    side = torch.cuda.Stream()
+    for k in range(60):
+        for ps in (quiet, busy):
+            for p, g in zip(ps, grads[k % 4]):
+                p.grad = g
+        opts[0].step()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            for _ in range(3):
+                load.step()
+        opts[1].step()
+        torch.cuda.synchronize()
+        for a, b in zip(quiet, busy):
+            assert torch.equal(a, b), k
