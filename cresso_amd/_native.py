@@ -79,13 +79,14 @@ class SpectralDesc(ctypes.Structure):
     ]
 
 
+class SpectralUnit(ctypes.Structure):
+    _fields_ = [("plan", ctypes.c_void_p), ("workspace", ctypes.c_void_p), ("workspace_bytes", ctypes.c_size_t),
+                ("descs", ctypes.c_void_p), ("count", ctypes.c_int32), ("batched", ctypes.c_int32),
+                ("lane", ctypes.c_int32), ("pad", ctypes.c_int32)]
+
+
 def hyper_from_group(group: dict) -> Hyper:
-    h = Hyper()
-    for n in HYPER_DOUBLES:
-        setattr(h, n, float(group[n]))
-    h.warmup_steps = int(group["warmup_steps"])
-    h.maximize = 1 if bool(group["maximize"]) else 0
-    return h
+    return Hyper(*[float(group[n]) for n in HYPER_DOUBLES], int(group["warmup_steps"]), 1 if bool(group["maximize"]) else 0)
 
 
 _LOCK = threading.Lock()
@@ -142,6 +143,16 @@ def _declare(lib: ctypes.CDLL) -> None:
                                                  c.c_size_t, c.POINTER(Hyper), c.c_void_p]
     lib.cresso_spectral_step_noalloc.restype = c.c_int32
     lib.cresso_spectral_step_noalloc.argtypes = [c.c_void_p, c.POINTER(SpectralDesc), c.POINTER(Hyper), c.c_void_p]
+    lib.cresso_spectral_step_units.restype = c.c_int32
+    lib.cresso_spectral_step_units.argtypes = [c.POINTER(SpectralUnit), c.c_int32, c.POINTER(Hyper),
+                                               c.POINTER(c.c_void_p), c.c_int32]
+    lib.cresso_fork_create.restype = c.c_void_p
+    lib.cresso_fork_create.argtypes = [c.c_int32]
+    lib.cresso_fork_destroy.restype = None
+    lib.cresso_fork_destroy.argtypes = [c.c_void_p]
+    for fork in (lib.cresso_fork_begin, lib.cresso_fork_end):
+        fork.restype = c.c_int32
+        fork.argtypes = [c.c_void_p, c.c_void_p, c.POINTER(c.c_void_p), c.c_int32]
     lib.cresso_spectral_workspace_bins.restype = c.c_int32
     lib.cresso_spectral_workspace_bins.argtypes = [c.c_void_p, c.c_void_p, c.c_size_t, c.c_void_p, c.c_void_p,
                                                    c.c_void_p]

@@ -521,6 +521,70 @@ extern "C" int32_t cresso_spectral_step_batched(const cresso_spectral_plan* P, c
     return fn(*P, descs, count, at<cresso_spectral_desc>(ws, P->o.desc), ls, ws, *hyper, s);
 }
 
+extern "C" int32_t cresso_spectral_step_units(const cresso_spectral_unit* units, int32_t n, const cresso_hyper* hyper,
+                                              void* const* streams, int32_t n_streams) {
+    if (!units || n < 0 || !hyper || !streams) return fail(CRESSO_E_INVALID, "spectral route: null argument");
+    for (int32_t i = 0; i < n; ++i)
+        if (units[i].lane < 0 || units[i].lane >= n_streams || units[i].count < 1 || (!units[i].batched && units[i].count != 1))
+            return fail(CRESSO_E_INVALID, "spectral route: unit %d has lane %d and %d tensors", i, units[i].lane, units[i].count);
+    for (int32_t i = 0; i < n; ++i) {
+        const cresso_spectral_unit& u = units[i];
+        void* s = streams[u.lane];
+        const int32_t rc = u.batched ? cresso_spectral_step_batched(u.plan, u.descs, u.count, u.workspace, u.workspace_bytes, hyper, s)
+                                     : cresso_spectral_step(u.plan, u.descs, u.workspace, u.workspace_bytes, hyper, s);
+        if (rc != CRESSO_OK) return rc;
+    }
+    return CRESSO_OK;
+}
+
+// Events of a fork (first) and of each stream's join.
+struct cresso_fork {
+    std::vector<hipEvent_t> ev;
+};
+
+extern "C" void cresso_fork_destroy(cresso_fork* F) {
+    if (!F) return;
+    for (hipEvent_t e : F->ev) (void)hipEventDestroy(e);
+    delete F;
+}
+
+extern "C" cresso_fork* cresso_fork_create(int32_t lanes) {
+    if (lanes < 1) {
+        fail(CRESSO_E_INVALID, "fork of %d streams", lanes);
+        return nullptr;
+    }
+    cresso_fork* F = new cresso_fork();
+    for (int32_t i = 0; i <= lanes; ++i) {
+        hipEvent_t e = nullptr;
+        const hipError_t rc = hipEventCreateWithFlags(&e, hipEventDisableTiming);
+        if (rc != hipSuccess) {
+            hip_fail(rc, "fork events");
+            cresso_fork_destroy(F);
+            return nullptr;
+        }
+        F->ev.push_back(e);
+    }
+    return F;
+}
+
+extern "C" int32_t cresso_fork_begin(cresso_fork* F, void* caller, void* const* streams, int32_t n) {
+    if (!F || !streams || n < 0 || (size_t)n >= F->ev.size()) return fail(CRESSO_E_INVALID, "fork of %d streams", n);
+    hipError_t e = hipEventRecord(F->ev[0], reinterpret_cast<hipStream_t>(caller));
+    for (int32_t i = 0; i < n && e == hipSuccess; ++i)
+        e = hipStreamWaitEvent(reinterpret_cast<hipStream_t>(streams[i]), F->ev[0], 0);
+    return e == hipSuccess ? CRESSO_OK : hip_fail(e, "fork");
+}
+
+extern "C" int32_t cresso_fork_end(cresso_fork* F, void* caller, void* const* streams, int32_t n) {
+    if (!F || !streams || n < 0 || (size_t)n >= F->ev.size()) return fail(CRESSO_E_INVALID, "join of %d streams", n);
+    hipError_t e = hipSuccess;
+    for (int32_t i = 0; i < n && e == hipSuccess; ++i) {
+        e = hipEventRecord(F->ev[i + 1], reinterpret_cast<hipStream_t>(streams[i]));
+        if (e == hipSuccess) e = hipStreamWaitEvent(reinterpret_cast<hipStream_t>(caller), F->ev[i + 1], 0);
+    }
+    return e == hipSuccess ? CRESSO_OK : hip_fail(e, "join");
+}
+
 // ---------------------------------------------------------------------------
 // cresso_spectral_step_noalloc: the step above with its workspace (carrier
 // tables, bins, tangent field and per-step scratch) in a static device array,

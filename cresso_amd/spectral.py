@@ -17,7 +17,8 @@ that share a workspace run one after another on that lane's stream, so its
 per-step scratch is never used concurrently.  The side streams wait for the
 caller's stream before the first launch and the caller's stream waits for
 all of them after the last, so the step is ordered like any other work on
-the caller's stream.  A single spectral tensor runs on the caller's stream
+the caller's stream; the group's scalar tensors step on the caller's stream
+meanwhile.  A single spectral tensor runs on the caller's stream
 directly.
 
 Device memory held: per (plan, lane) a workspace of the plan's tables (about
@@ -123,13 +124,16 @@ class SpectralEngine:
     def __init__(self):
         self.lib = _native.load()
         self.ws: Dict[tuple, _Workspace] = {}   # (plan key, unit kind, lane) -> workspace
+        self.version = 0                        # changes with every workspace made or dropped
         self.side: Dict[torch.device, List[torch.cuda.Stream]] = {}
+        self.forks: Dict[torch.device, _Fork] = {}
         self.freq_cache: Dict[int, Tuple[int, ...]] = {}
 
     def reset(self) -> None:
         """Forget cached frequency lists and free every workspace."""
         self.freq_cache.clear()
         self.ws.clear()
+        self.version += 1
 
     def retain(self, keys) -> None:
         """Forget cached frequency lists; free the workspaces whose plan key is
@@ -137,6 +141,7 @@ class SpectralEngine:
         self.freq_cache.clear()
         for wkey in [k for k in self.ws if k[0] not in keys]:
             del self.ws[wkey]
+        self.version += 1
 
     def plan_key(self, param: torch.Tensor, st: dict, group: dict) -> tuple:
         """The plan key of a spectral tensor: (device, shape, freqs, hash_bins, hash_tables, work dtype)."""
@@ -163,6 +168,7 @@ class SpectralEngine:
             self.ws.pop(wkey, None)
             ws = _Workspace(self.lib, shape, freqs, rank, bins, tables, group, device, count, work)
             self.ws[wkey] = ws
+            self.version += 1
         return ws
 
     def _prepare(self, param: torch.Tensor, grad: torch.Tensor, st: dict, group: dict):
@@ -206,24 +212,6 @@ class SpectralEngine:
         d.hard = 1 if hard else 0
         return key, rank, d
 
-    def _launch(self, ws: _Workspace, d, hyper, stream: int) -> None:
-        _native.check(self.lib.cresso_spectral_step(ws.plan, ctypes.byref(d), ctypes.c_void_p(ws.buf.data_ptr()),
-                                                    ctypes.c_size_t(ws.buf.numel()), ctypes.byref(hyper),
-                                                    ctypes.c_void_p(stream)), "spectral route step")
-
-    def _launch_batch(self, ws: _Workspace, descs: list, hyper, stream: int) -> None:
-        arr = (_native.SpectralDesc * len(descs))(*descs)
-        _native.check(self.lib.cresso_spectral_step_batched(ws.plan, arr, len(descs), ctypes.c_void_p(ws.buf.data_ptr()),
-                                                            ctypes.c_size_t(ws.buf.numel()), ctypes.byref(hyper),
-                                                            ctypes.c_void_p(stream)), "spectral route batched step")
-
-    def step(self, param: torch.Tensor, grad: torch.Tensor, st: dict, group: dict) -> None:
-        """One tensor on the caller's stream."""
-        key, rank, d = self._prepare(param, grad, st, group)
-        ws = self._workspace(key, 0, rank, group)
-        st["step"] += 1
-        self._launch(ws, d, _native.hyper_from_group(group), _native.stream_handle(param.device))
-
     def _streams(self, device: torch.device, n: int) -> List[torch.cuda.Stream]:
         have = self.side.setdefault(device, [])
         while len(have) < n:
@@ -253,36 +241,141 @@ class SpectralEngine:
                 units.append(((key, True, m), key, rank, [prepared[i][2] for i in sel], [sts[i] for i in sel]))
         return units
 
-    def step_many(self, items: Sequence[Tuple[torch.Tensor, torch.Tensor, dict]], group: dict) -> None:
-        """Every spectral tensor of a param group: (param, grad, state) each."""
+    def step_many(self, items: Sequence[Tuple[torch.Tensor, torch.Tensor, dict]], group: dict, between=None) -> None:
+        """Every spectral tensor of a param group: (param, grad, state) each.
+        between: work for the caller's stream that may run beside the side
+        streams (called once)."""
+        plan = self._plan(items, group)
+        for _, _, sts, _, _ in plan:
+            for st in sts:
+                st["step"] += 1
+        Launch(self, [(ws, (_native.SpectralDesc * len(descs))(*descs), lane, device)
+                      for ws, descs, _, lane, device in plan]).run(_native.hyper_from_group(group), between)
+
+    def _plan(self, items, group: dict) -> list:
+        """The step's units: (workspace, [desc], [state], lane or None, device).
+        lane None: the caller's stream (a single tensor).  Workspaces created
+        here are initialised on the caller's stream, before the lanes fork."""
         if len(items) == 1:
-            self.step(*items[0], group)
-            return
+            p, g, st = items[0]
+            key, rank, d = self._prepare(p, g, st, group)
+            return [(self._workspace(key, 0, rank, group), [d], [st], None, p.device)]
         by_dev: Dict[torch.device, list] = {}
         for it in items:
             by_dev.setdefault(it[0].device, []).append(it)
-        hyper = _native.hyper_from_group(group)
+        plan = []
         for device, its in by_dev.items():
-            # descriptors and workspaces first: a workspace created now is
-            # initialised on the caller's stream, before the lanes fork from it
             prepared = [self._prepare(p, g, st, group) for p, g, st in its]
             units = self._units(prepared, [st for _, _, st in its])
             nl = min(self.LANES, len(units))
             lanes = assign_lanes([u[0][:2] for u in units], nl)
-            plan = []
             for (ukey, key, rank, descs, sts), lane in zip(units, lanes):
                 count = ukey[2] if ukey[1] else None
-                plan.append((self._workspace(key, lane, rank, group, count), descs, sts, lane))
-            cur = torch.cuda.current_stream(device)
-            side = self._streams(device, nl)
-            for s in side:
-                s.wait_stream(cur)
-            for ws, descs, sts, lane in plan:
-                for st in sts:
-                    st["step"] += 1
-                if ws.count is None:
-                    self._launch(ws, descs[0], hyper, int(side[lane].cuda_stream))
+                plan.append((self._workspace(key, lane, rank, group, count), descs, sts, lane, device))
+        return plan
+
+    def _fork(self, device: torch.device, lanes: int) -> "_Fork":
+        fork = self.forks.get(device)
+        if fork is None or len(fork.streams) < lanes:   # (streams are made as they are needed)
+            fork = self.forks[device] = _Fork(self.lib, self._streams(device, lanes), device)
+        return fork
+
+
+class _Fork:
+    """A device's side streams and the library's events that fork them from
+    and join them to the caller's stream."""
+
+    def __init__(self, lib, streams: List[torch.cuda.Stream], device: torch.device):
+        self.lib = lib
+        self.streams = streams
+        self.handles = (ctypes.c_void_p * len(streams))(*[int(s.cuda_stream) for s in streams])
+        with torch.cuda.device(device):
+            self.fork = lib.cresso_fork_create(len(streams))
+        if not self.fork:
+            _native.check(-1, "side streams")
+
+    def __del__(self):
+        if getattr(self, "fork", None):
+            try:
+                self.lib.cresso_fork_destroy(self.fork)
+            except Exception:
+                pass
+
+
+class Launch:
+    """The launches of a step: units (workspace, descriptor array, lane or
+    None, device).  Per device one call steps the units; several units run on
+    the side streams, which fork from the caller's stream before the first
+    launch and join it after the last (a lone tensor: the caller's stream)."""
+
+    def __init__(self, engine: SpectralEngine, units: list):
+        self.engine = engine
+        self.keep = units                 # workspaces and descriptor arrays
+        self.devices = []
+        for device in dict.fromkeys(u[3] for u in units):
+            mine = [u for u in units if u[3] == device]
+            arr = (_native.SpectralUnit * len(mine))()
+            for a, (ws, descs, lane, _) in zip(arr, mine):
+                a.plan, a.workspace, a.workspace_bytes = ws.plan.value, ws.buf.data_ptr(), ws.buf.numel()
+                a.descs, a.count, a.batched = ctypes.addressof(descs), len(descs), 0 if ws.count is None else 1
+                a.lane = 0 if lane is None else lane
+            lanes = 0 if mine[0][2] is None else 1 + max(u[2] for u in mine)
+            self.devices.append((device, arr, len(mine), lanes))
+
+    def run(self, hyper, between=None) -> None:
+        """between: run after the launches, on the caller's stream, beside the
+        side streams."""
+        lib, open_ = self.engine.lib, []
+        try:
+            for device, arr, n, lanes in self.devices:
+                caller = ctypes.c_void_p(_native.stream_handle(device))
+                if lanes == 0:
+                    handles, count = ctypes.pointer(caller), 1
                 else:
-                    self._launch_batch(ws, descs, hyper, int(side[lane].cuda_stream))
-            for s in side:
-                cur.wait_stream(s)
+                    fork = self.engine._fork(device, lanes)
+                    handles, count = fork.handles, lanes
+                    _native.check(lib.cresso_fork_begin(fork.fork, caller, handles, lanes), "side streams")
+                    open_.append((fork, caller, lanes))
+                _native.check(lib.cresso_spectral_step_units(arr, n, ctypes.byref(hyper), handles, count),
+                              "spectral route step")
+            if between is not None:
+                between()
+        finally:
+            for fork, caller, lanes in open_:
+                _native.check(lib.cresso_fork_end(fork.fork, caller, fork.handles, lanes), "side streams")
+
+
+class SteadyStep:
+    """The steady state of a group's spectral tensors: the units of a step that
+    has run, with their workspaces, and the C++ guard that checks every
+    parameter, grad and state tensor again on each step and writes their
+    descriptors.  run() returns False, with nothing launched, when anything
+    differs; the general path then takes the step."""
+
+    def __init__(self, engine: SpectralEngine, items, group: dict, hb):
+        plan = engine._plan(items, group)
+        if any(ws.count is None and len(descs) != 1 for ws, descs, _, _, _ in plan):
+            raise ValueError("a unit without a batched workspace holds one tensor")
+        by_state = {id(st): (p, st) for p, _, st in items}
+        order = [by_state[id(st)] for _, _, sts, _, _ in plan for st in sts]
+        descs = [d for _, ds, _, _, _ in plan for d in ds]
+        self.engine = engine
+        self.version = engine.version
+        self.guard = hb.SpectralGuard([p for p, _ in order], [st["freqs"] for _, st in order],
+                                      [(d.param_dtype, d.grad_dtype) for d in descs], [d.hard for d in descs],
+                                      [1 if d.hash_energy else 0 for d in descs], int(group["hash_bins"]),
+                                      int(group["hash_tables"]))
+        self.descs = (_native.SpectralDesc * len(descs))()
+        units, at, size = [], 0, ctypes.sizeof(_native.SpectralDesc)
+        for ws, ds, _, lane, device in plan:
+            units.append((ws, (_native.SpectralDesc * len(ds)).from_buffer(self.descs, at * size), lane, device))
+            at += len(ds)
+        self.launch = Launch(engine, units)
+
+    def fill(self, state: dict) -> bool:
+        return self.version == self.engine.version and self.guard.fill(state, ctypes.addressof(self.descs))
+
+    def run(self, state: dict, hyper, between=None) -> None:
+        """The step (after fill() returned True)."""
+        self.guard.bump(state)
+        self.launch.run(hyper, between)

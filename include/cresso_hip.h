@@ -214,6 +214,29 @@ int32_t cresso_spectral_batched_workspace_init(const cresso_spectral_plan* plan,
 int32_t cresso_spectral_step_batched(const cresso_spectral_plan* plan, const cresso_spectral_desc* descs, int32_t count,
                                      void* workspace, size_t workspace_bytes, const cresso_hyper* hyper, void* stream);
 
+/* Several steps in one call: unit i steps its `count` descriptors (batched != 0:
+ * cresso_spectral_step_batched on a batched workspace; else count is 1 and
+ * cresso_spectral_step runs) on streams[lane]. */
+typedef struct cresso_spectral_unit {
+    const cresso_spectral_plan* plan;
+    void* workspace;
+    size_t workspace_bytes;
+    const cresso_spectral_desc* descs;
+    int32_t count, batched, lane, pad;
+} cresso_spectral_unit;
+int32_t cresso_spectral_step_units(const cresso_spectral_unit* units, int32_t n, const cresso_hyper* hyper,
+                                   void* const* streams, int32_t n_streams);
+
+/* Fork and join of streams for such a call: begin makes streams[0..n) wait for
+ * what `caller` holds so far, end makes `caller` wait for them.  A handle
+ * keeps the events (for up to `lanes` streams of the current device); calls on
+ * one handle must not overlap. */
+typedef struct cresso_fork cresso_fork;
+cresso_fork* cresso_fork_create(int32_t lanes);
+void cresso_fork_destroy(cresso_fork* fork);
+int32_t cresso_fork_begin(cresso_fork* fork, void* caller, void* const* streams, int32_t n);
+int32_t cresso_fork_end(cresso_fork* fork, void* caller, void* const* streams, int32_t n);
+
 /* cresso_spectral_step without a workspace argument, for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference.

@@ -1,0 +1,97 @@
+"""Steps of mixed groups after the second, which the C++ guards take when
+nothing has changed: the same results as an optimizer whose every step goes
+the general way, over changes that must send a step back there."""
+
+import pytest
+import torch
+
+from gpu_util import announce, needs_gpu
+
+pytestmark = [pytest.mark.gpu, needs_gpu]
+
+SHAPES = [(256, 300), (64, 65), (64, 65), (4096, 16), (1500,), (10,), (24, 6, 3, 3)]
+
+
+def _pair(shapes, **kw):
+    import cresso_amd
+
+    gen = torch.Generator().manual_seed(51)
+    p0 = [0.02 * torch.randn(s, generator=gen) for s in shapes]
+    out = []
+    for _ in range(2):
+        ps = [torch.nn.Parameter(p.cuda()) for p in p0]
+        out.append((ps, cresso_amd.CRESSO5(ps, cuda_ops="required", rank=8, hash_bins=64, hash_tables=2, **kw)))
+    return gen, out
+
+
+def _steps(gen, pair, n, change=None):
+    for k in range(n):
+        grads = [1e-3 * torch.randn(p.shape, generator=gen) for p in pair[0][0]]
+        for i, (ps, opt) in enumerate(pair):
+            for p, g in zip(ps, grads):
+                p.grad = g.cuda()
+            if change is not None:
+                change(k, ps, opt)
+            if i == 1:
+                opt._steady.clear()   # the general way
+            opt.step()
+    torch.cuda.synchronize()
+    (pa, oa), (pb, ob) = pair
+    for a, b in zip(pa, pb):
+        assert torch.equal(a, b)
+        for key, v in oa.state[a].items():
+            w = ob.state[b][key]
+            assert torch.equal(v, w) if torch.is_tensor(v) else v == w, key
+
+
+@pytest.mark.parametrize("shapes", [SHAPES, SHAPES[:1], SHAPES[1:3]], ids=["mixed", "one", "batch"])
+def test_steady_steps_are_the_general_steps(shapes):
+    announce(f"steady steps {len(shapes)}")
+    gen, pair = _pair(shapes)
+    _steps(gen, pair, 6)
+    assert pair[0][1]._steady[0][2] is not None   # the steady step was made
+
+
+def test_steady_steps_follow_changes():
+    """A skipped grad, other layouts and dtypes of grads, new parameter storage, replaced state tensors, another
+    step count, group options and learning rate."""
+    announce("steady steps with changes")
+    gen, pair = _pair(SHAPES)
+
+    def change(k, ps, opt):
+        if k == 3:
+            ps[1].grad = None
+        if k == 5:
+            ps[0].grad = ps[0].grad.t().contiguous().t()
+        if k == 7:
+            ps[2].data = ps[2].data.clone()
+        if k == 9:
+            st = opt.state[ps[0]]
+            st["q_cos"] = st["q_cos"].clone() * 0.5
+            st["step"] = 3
+        if k == 10:
+            opt.param_groups[0]["lr"] = 1e-3
+        if k == 12:
+            opt.param_groups[0]["weight_decay"] = 0.01
+        if k == 14:
+            opt.load_state_dict(opt.state_dict())
+        if k == 16:
+            with torch.no_grad():
+                ps[5].zero_()
+
+    _steps(gen, pair, 19, change)
+
+
+def test_steady_step_refuses_what_the_general_step_refuses():
+    gen, pair = _pair(SHAPES)
+    _steps(gen, pair, 4)
+    ps, opt = pair[0]
+    for p in ps:
+        p.grad = torch.zeros_like(p)
+    ps[1].grad = torch.zeros_like(ps[1]).to_sparse()
+    with pytest.raises(RuntimeError, match="sparse"):
+        opt.step()
+    ps[1].grad = torch.zeros_like(ps[1])
+    opt.state[ps[0]]["hash_energy"] = opt.state[ps[0]]["hash_energy"].t().contiguous()
+    with pytest.raises(RuntimeError, match="shape"):
+        opt.step()
