@@ -20,7 +20,7 @@
 // The kernels:
 //  * scalar_small_kernel: tensors of at most 16 Ki elements (fp32 work), any
 //    shape, every pass from registers; micro_small_kernel the same for the
-//    micro-field route.
+//    micro-field route; scalar_mid_kernel up to 32 Ki, from LDS.
 //  * scalar_resident_kernel: 2D tensors of <= 64 Ki elements whose rows map to
 //    lane groups (LoRA-thin (L,16)) or whose rows are exactly one block wide
 //    ((16,4096)); f, then t, then drive stay on chip (half of each thread's
@@ -1704,9 +1704,16 @@ __device__ __forceinline__ void ss_axis_factors(const ScalarRec& R, const float*
         int P = 1;
         while (P < 64 && 2 * P <= M && D * 2 * P <= nt) P *= 2;
         const int q = tid & (P - 1);
+        // short runs of a power of two, one lane each: the lanes of a wave
+        // start at different elements of their runs, so that they read 64 banks
+        const int rot = contig && P == 1 && M <= 64 && (M & (M - 1)) == 0 ? 6 - (31 - __builtin_clz(M)) : -1;
         for (int e = tid / P; e < D; e += nt / P) {
             double a = 0.0;
-            if (contig) {
+            if (contig && rot >= 0) {
+                const int r0 = e >> rot;
+#pragma unroll 8
+                for (int m = 0; m < M; ++m) a += (double)sd[e * st + ((m + r0) & (M - 1))];
+            } else if (contig) {
                 for (int m = q; m < M; m += P) a += (double)sd[e * st + m];
             } else if (st == 1) {
                 for (int m = q; m < M; m += P) a += (double)sd[m * D + e];
@@ -1932,6 +1939,183 @@ __global__ __launch_bounds__(SS_NT) void scalar_small_kernel(const ScalarRec* __
     }
 }
 
+// Tensors of more than SS_MAX and at most SS_MID elements, as
+// scalar_small_kernel with the elements in LDS: thirty-two a thread in
+// registers spill (2700 of them).  The grads are read again in passes B and C
+// (from L2), the densities, then t, then the drive stay in LDS, each element
+// on its own thread.  The moments' fp64 sums go by DPP (LDS is full).
+// us a step of 132 x (16,2048) fp32: 156 in the wide form's ten launches ->
+// 70 in one (resident shapes: build_plan).
+constexpr int64_t SS_MID = 32 * SS_NT;
+constexpr size_t ss_mid_lds() { return sizeof(float) * ((size_t)SS_MID + 2 * SS_NT + SS_AXES); }
+
+template <typename PT, typename GT>
+__global__ __launch_bounds__(SS_NT) void scalar_mid_kernel(const ScalarRec* __restrict__ recs, int32_t* __restrict__ steps,
+                                                           const void* const* __restrict__ grads, int32_t first,
+                                                           cresso_hyper h) {
+    extern __shared__ __align__(16) float ss_dyn[];
+    __shared__ double pub[2], red[(SS_NT / 64) * 13];
+    __shared__ float s_sM;
+    __shared__ DriveCoef<float> s_dc;
+    constexpr int U = 8;                      // elements whose loads are in flight together
+    float* const sx = ss_dyn;                 // [SS_MID]
+    float* const sy = ss_dyn + SS_MID;        // [2][SS_NT]
+    float* const fac = sy + 2 * SS_NT;        // [SS_AXES]
+    const int tid = threadIdx.x, wave = tid >> 6;
+    const int ri = first + blockIdx.x;
+    const ScalarRec& R = recs[ri];
+    const int n = (int)R.d.numel, nd = R.d.ndim, layout = R.layout;
+    const GT* __restrict__ g = reinterpret_cast<const GT*>(grads[ri]);
+    PT* p = reinterpret_cast<PT*>(R.d.param);
+    const float wd = (float)h.weight_decay;
+    const bool wd_on = h.weight_decay != 0.0;
+    // fn(i, f) for the thread's elements in order
+    auto each = [&](auto&& fn) {
+        for (int ib = tid; ib < n; ib += U * SS_NT) {
+            float f[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int i = ib + u * SS_NT, c = i < n ? i : n - 1;   // (clamped: no branch between the loads)
+                f[u] = to_f(g[c]);
+                if (h.maximize) f[u] = -f[u];
+                if (wd_on) f[u] = f[u] + wd * to_f(p[c]);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (ib + u * SS_NT < n) fn(ib + u * SS_NT, f[u]);
+        }
+    };
+    const float* const* st = reinterpret_cast<const float* const*>(R.d.state);
+    float q0 = ld_uniform(st[0]), imp = ld_uniform(st[1]), mq = ld_uniform(st[2]), mp = ld_uniform(st[3]);
+    float fr = ld_uniform(st[4]), de = ld_uniform(st[5]), sur = ld_uniform(st[6]), act = ld_uniform(st[7]);
+    int step = __builtin_amdgcn_readfirstlane(steps[ri]) + 1;
+    hold(q0); hold(imp); hold(mq); hold(mp); hold(fr); hold(de); hold(sur); hold(act);
+    asm volatile("" : "+s"(step));
+    const double dn = (double)n, in = 1.0 / dn;
+    const float eps = (float)h.eps, pw = (float)h.energy_power, ipw = (float)fmax(h.instant_metric_power, 0.25);
+    const float kappa = nd > 0 ? (float)(h.instant_metric_coupling / ((double)nd * fmax(h.instant_metric_power, 0.25))) : 0.f;
+    const float tq = wave == 0 ? (float)tanh((double)mq) : 0.f;
+    // ---- A ----
+    {
+        float a[1] = {0.f};
+        double v[1];
+        each([&](int, float f) { a[0] += f * f; });
+        block_sum_t<1>(a, v, sy, pub);
+        fr = reservoir(fr, sqrtf((float)(v[0] * in) + eps), h.reservoir_decay, step);
+    }
+    if (tid == 0) steps[ri] = step;   // (every thread read it before the barriers above)
+    const float scale = fmaxf(fr, eps), inv_s = 1.0f / scale;
+    // ---- B ----
+    float gden;
+    {
+        float a[2] = {0.f, 0.f};
+        double v[2];
+        each([&](int i, float f) {
+            const float r = fabsf(f) * inv_s + eps;
+            const float d = ss_density(fminf(r, 1.0e4f), eps, ipw);
+            a[0] += flog1p(fpow(r, pw));
+            a[1] += d;
+            sx[i] = d;
+        });
+        block_sum_t<2>(a, v, sy, pub);
+        gden = (float)fmax(v[1] * in, (double)eps);
+        if (wave == 0) {
+            // scalar metric oscillator (cresso_v5.py:1510-1518)
+            const float mport = (float)(v[0] * in) - tq;
+            mp = mp * (float)fmax(0.0, 1.0 - h.metric_dt * h.metric_friction);
+            mp = mp + (float)h.metric_dt * (mport - mq);
+            mq = mq + (float)h.metric_dt * mp;
+            mq = clampn(mq, -3.0f, 3.0f);
+            const float metric = clampn((float)exp((double)((float)h.metric_coupling * mq)), 0.06f, 16.0f);
+            if (tid == 0) s_sM = scale * metric;
+        }
+        if (layout == L_2D || layout == L_GENERIC) ss_axis_factors(R, sx, fac, gden, kappa, eps, tid, SS_NT);
+    }
+    __syncthreads();
+    const float sM = s_sM;
+    // ---- C ----
+    const float clip = (float)h.drive_clip, iclip = 1.0f / clip, clip2 = clip * clip, k2 = -2.8853900817779268f * iclip;
+    const float ls = (float)h.local_sharpness;
+    const bool ls_on = h.local_sharpness != 0.0;
+    {
+        SSWalk w(R, tid);
+        float m[13] = {0.f};
+        each([&](int i, float f) {
+            float den = sM;
+            if (ls_on) den *= clampn(1.0f + ls * fsqrt(fminf(fabsf(f) * inv_s + eps, 100.0f)), 1.0f, 8.0f);
+            float inst = 1.0f;
+            if (layout == L_1D) {
+                const float d = ss_density(fminf(fabsf(f) * inv_s + eps, 1.0e4f), eps, ipw);
+                inst = fexp2(kappa * flog2(fmaxf(d / gden, eps)));
+            } else if (layout != L_NONE) {
+                inst = fexp2(ss_log_inst(R, fac, w, i));
+            }
+            w.next();
+            if (layout != L_NONE) inst = clampn(inst, 0.08f, 12.0f);
+            const float t = clampn(f * frcp(den * inst + eps), -1.0e4f, 1.0e4f);
+            sx[i] = t;
+            const float e = t - q0, at = fabsf(t);
+            const Shape3A z = shape3a(at, k2, iclip, clip2, eps);
+            m[0] += e; m[1] += e * e; m[2] += t; m[3] += t * t;
+            m[4] += z.rat * z.rat; m[5] += z.th * z.th; m[6] += z.root * z.root;
+            m[7] += z.rat * z.th; m[8] += z.rat * z.root; m[9] += z.th * z.root;
+            m[10] += at * z.rat; m[11] += at * z.th; m[12] += at * z.root;
+        });
+        double M[13];
+#pragma unroll
+        for (int j = 0; j < 13; ++j) M[j] = (double)m[j];
+        block_sum<13>(M, red);
+        if (wave == 0) {
+            // bnd = clip tanh(t / clip)
+            M[5] *= (double)clip * (double)clip;
+            M[7] *= (double)clip; M[9] *= (double)clip; M[11] *= (double)clip;
+            const DriveCoef<float> c = contact_and_coefs<float>(M, dn, h, step, q0, imp, act, sur);
+            if (tid == 0) s_dc = c;
+        }
+        __syncthreads();
+    }
+    // ---- D ----
+    const DriveCoef<float> c = s_dc;
+    {
+        const float cbt = c.cb * clip, cn = c.cN * clip, k2n = -2.8853900817779268f * c.nscale;
+        float a[1] = {0.f};
+        double v[1];
+#pragma unroll 4
+        for (int i = tid; i < n; i += SS_NT) {
+            const float t = sx[i], e = t - c.q1, at = fabsf(t);
+            Shape3A z;
+            const float nov = shape3a_nov(at, e, k2, k2n, iclip, clip2, eps, z);
+            const float core = xorsign(fmaf(c.ct, at, fmaf(c.co, z.root, fmaf(cbt, z.th, c.cr * z.rat))), t);
+            const float d = c.cA * core + c.cB + cn * nov + c.cD * e;
+            sx[i] = d;
+            a[0] += d * d;
+        }
+        block_sum_t<1>(a, v, sy, pub);
+        de = reservoir(de, (float)(v[0] * in), h.reservoir_decay, step);
+    }
+    const float gain = clampn((float)h.target_update_rms / sqrtf(de + eps), (float)h.min_gain, (float)h.max_gain);
+    // ---- E ----
+    const float nlr = (float)update_alpha<PT>(-h.lr);
+    for (int ib = tid; ib < n; ib += U * SS_NT) {
+        float pv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = ib + u * SS_NT;
+            pv[u] = to_f(p[i < n ? i : n - 1]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = ib + u * SS_NT;
+            if (i < n) p[i] = from_w<PT>(pv[u] + nlr * to_f(from_w<PT>(sx[i] * gain)));
+        }
+    }
+    if (tid == 0) {
+        float* const* so = reinterpret_cast<float* const*>(R.d.state);
+        *so[0] = c.q1; *so[1] = imp; *so[2] = mq; *so[3] = mp;
+        *so[4] = fr; *so[5] = de; *so[6] = sur; *so[7] = act;
+    }
+}
+
 // The micro-field route of small tensors (at most SS_MAX elements): as
 // scalar_small_kernel, with the three dense fields in registers too (each is
 // read once and written once).  us a step of a coordinate network's 18
@@ -2108,7 +2292,7 @@ bool is_pow2(int64_t v) { return v > 0 && (v & (v - 1)) == 0; }
 
 struct Variant {
     int pt, gt, kind;   // kind: 0 stream, 1 resident (row-group or column-block layout), 2 wide stream, 3 micro field,
-                        // 4 small, 5 small micro field
+                        // 4 small, 5 small micro field, 6 middle (small, with the elements in LDS)
     bool full;          // resident with numel == SR_RESIDENT_MAX: eligible for the FAST kernel
     bool operator==(const Variant& o) const { return pt == o.pt && gt == o.gt && kind == o.kind && full == o.full; }
 };
@@ -2121,7 +2305,7 @@ bool fast_hyper(const cresso_hyper& h) {
 // Tensors the small kernels take: fp32 work, elements in registers, axis
 // factors in LDS (sum_dims 0: none).
 bool small_ok(const cresso_scalar_desc& d, int64_t sum_dims) {
-    return d.param_dtype != CRESSO_F64 && d.numel <= SS_MAX && sum_dims <= SS_AXES;
+    return d.param_dtype != CRESSO_F64 && d.numel <= (d.route == 1 ? SS_MAX : SS_MID) && sum_dims <= SS_AXES;
 }
 
 int dtype_bytes(int t) { return t == CRESSO_F64 ? 8 : (t == CRESSO_F32 ? 4 : 2); }
@@ -2203,7 +2387,7 @@ int32_t plan_desc(const cresso_scalar_desc& d, const cresso_hyper& h, ScalarRec&
         int64_t dims = 0;
         for (int a = 0; a < d.ndim; ++a) dims += d.shape[a];
         // (the small kernel takes resident shapes too, up to its size)
-        const bool small = small_ok(d, dims);
+        const bool small = n <= SS_MAX && small_ok(d, dims);
         if (!small && res_ok && is_pow2(C0 / 4) && C0 / 4 <= 64 && rg_lds <= SR_LDS_MAX) {
             r.layout = L_ROWGROUP;
             r.group = (int32_t)(C0 / 4);
@@ -2241,7 +2425,7 @@ int32_t plan_desc(const cresso_scalar_desc& d, const cresso_hyper& h, ScalarRec&
         }
     }
     if (kind == 0 && small_ok(d, r.sum_dims)) {
-        kind = 4;
+        kind = n <= SS_MAX ? 4 : 6;
         scratch = 0;
     }
     if (kind == 0 && n >= SR_WIDE_MIN) kind = 2;
@@ -2307,6 +2491,15 @@ hipError_t launch_small_k(bool micro, const ScalarRec* recs, int32_t* steps, con
     return hipGetLastError();
 }
 template <typename PT, typename GT>
+hipError_t launch_mid(const ScalarRec* recs, int32_t* steps, const void* const* grads, int32_t first, int32_t cnt,
+                      const cresso_hyper& h, hipStream_t s) {
+    static const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&scalar_mid_kernel<PT, GT>),
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)ss_mid_lds());
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((scalar_mid_kernel<PT, GT>), dim3(cnt), dim3(SS_NT), ss_mid_lds(), s, recs, steps, grads, first, h);
+    return hipGetLastError();
+}
+template <typename PT, typename GT>
 hipError_t launch_small(bool micro, bool k16, const ScalarRec* recs, int32_t* steps, const void* const* grads, int32_t first,
                         int32_t cnt, const cresso_hyper& h, hipStream_t s) {
     return k16 ? launch_small_k<PT, GT, 16>(micro, recs, steps, grads, first, cnt, h, s)
@@ -2365,7 +2558,9 @@ hipError_t dispatch(const Variant& v, const ScalarRec* recs, int32_t* steps, con
     if (v.kind >= 4) {
 #define CRESSO_SS_CASE(PC, GC, PT, GT)                                                                               \
     if (v.pt == PC && v.gt == GC)                                                                                    \
-        return launch_small<PT, GT>(v.kind == 5, lds > ss_lds(8), recs, steps, grads, first, cnt, h, s);
+        return v.kind == 6 ? launch_mid<PT, GT>(recs, steps, grads, first, cnt, h, s)                                \
+                           : launch_small<PT, GT>(v.kind == 5, lds > ss_lds(8), recs, steps, grads, first, cnt, h, \
+                                                  s);
         CRESSO_SS_CASE(CRESSO_F32, CRESSO_F32, float, float)
         CRESSO_SS_CASE(CRESSO_BF16, CRESSO_BF16, __hip_bfloat16, __hip_bfloat16)
         CRESSO_SS_CASE(CRESSO_F16, CRESSO_F16, __half, __half)
@@ -2445,6 +2640,31 @@ int32_t build_plan(const cresso_scalar_desc* descs, int32_t count, const cresso_
     if (mid > 0 && mid < SR_WIDE_FILL)
         for (int32_t i = 0; i < count; ++i)
             if (var[(size_t)i].kind == 0 && descs[i].numel >= SR_WIDE_MID) var[(size_t)i].kind = 2;
+    // Resident tensors of the middle sizes join the middle kernel's launch when
+    // the plan holds such tensors and all of them fit in one round of 256
+    // workgroups: two launches run one after the other (110 x (2048,16) fp32
+    // 60 us on the resident kernel, 72 on the middle one; with 132 x (16,2048)
+    // 60 + 70 in two launches, 81 in one).
+    auto joins = [&](int32_t i) {
+        return var[(size_t)i].kind == 1 && !var[(size_t)i].full && small_ok(descs[i], descs[i].shape[0] + descs[i].shape[1]);
+    };
+    int32_t middle = 0, joining = 0;
+    for (int32_t i = 0; i < count; ++i) {
+        middle += var[(size_t)i].kind == 6;
+        joining += joins(i);
+    }
+    if (middle > 0 && middle + joining <= 256)
+        for (int32_t i = 0; i < count; ++i)
+            if (joins(i)) {
+                ScalarRec& r = recs[(size_t)i];
+                r.layout = L_2D;
+                r.stride[0] = r.cols;
+                r.stride[1] = 1;
+                r.axis_off[1] = r.rows;
+                r.sum_dims = r.rows + r.cols;
+                r.resident = 0;
+                var[(size_t)i].kind = 6;
+            }
     std::vector<Variant> keys;
     for (const Variant& v : var)
         if (std::find(keys.begin(), keys.end(), v) == keys.end()) keys.push_back(v);

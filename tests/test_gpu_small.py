@@ -13,7 +13,8 @@ pytestmark = [pytest.mark.gpu, needs_gpu]
 KW = dict(lr=2e-3, rank=4, hash_bins=64, hash_tables=2, min_spectral_size=1 << 30)
 OPTIONS = dict(KW, weight_decay=0.02, maximize=True, local_sharpness=0.3, instant_metric_power=0.7, warmup_steps=0)
 SHAPES = [(), (1,), (1, 1), (1, 7), (1023,), (1025,), (64, 16), (33, 31), (8, 1024), (8193,), (16384,), (4, 4096),
-          (16385,), (5, 3276), (1, 4095), (1, 4096), (2, 8192), (3, 5, 7), (2, 4, 1000), (16, 8, 3, 3), (2, 3, 2, 5, 3)]
+          (16385,), (5, 3276), (1, 4095), (1, 4096), (2, 8192), (16, 2000), (16, 2048), (2048, 16),
+          (32768,), (32769,), (40, 700), (7, 40, 100), (3, 5, 7), (2, 4, 1000), (16, 8, 3, 3), (2, 3, 2, 5, 3)]
 
 
 @pytest.mark.parametrize("kw", [KW, OPTIONS, dict(KW, instant_metric_coupling=0.0)], ids=["plain", "options", "no_axes"])
