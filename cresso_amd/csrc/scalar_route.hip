@@ -64,6 +64,7 @@ struct ScalarRec {
     int32_t resident;       // 1: scalar_resident_kernel
     int64_t ctl_off;        // wide form: byte offset of the tensor's StreamCtl in the table
     int32_t blk0, nblk;     // wide form: first block (within its group's launches) and block count
+    int64_t chunk;          // wide form: elements per block
 };
 
 __device__ __forceinline__ float uni(float v) {
@@ -778,7 +779,7 @@ __global__ __launch_bounds__(SR_NT) void scalar_resident_kernel(const ScalarRec*
 //     whole tensor, with block reductions between the passes;
 //   - the wide form (tensors of more than 64 Ki elements, or of 16 Ki and
 //     more when the plan holds fewer than 256 of those): each pass is
-//     one launch over chunks of SR_WIDE_CH elements of every tensor of the
+//     one launch over chunks of wide_chunk() elements of every tensor of the
 //     group, writing block partials; a finish kernel (one workgroup per
 //     tensor) reduces them in block order and carries the tensor's values
 //     (StreamCtl, in the plan table) to the next pass.  Ten launches per
@@ -792,7 +793,13 @@ template <typename W> struct StreamCtl {
     int32_t step;
 };
 constexpr int SR_WIDE_NT = 256;              // threads per block of the wide form
-constexpr int64_t SR_WIDE_CH = 8192;         // elements per block of the wide form
+// Elements per block of the wide form, by the plan's wide elements: few of them
+// fill the GPU with smaller blocks, many pay for every block's partials and
+// atomics.  us a step of fp32 tensors with 8192 / 4096 / 2048 a block: 8 x
+// (8192,16) 111 / 78 / 63, 3 x (20000,7) 134 / 95 / 82, (65536,64) 135 / 125 /
+// 156, 66 x (5632,16) 156 / 134 / 146, 132 x (5632,16) and (16,5632) 208 / 218
+// / 240.
+inline int64_t wide_chunk(int64_t elements) { return elements <= 3 << 19 ? 2048 : (elements <= 1 << 23 ? 4096 : 8192); }
 constexpr int64_t SR_WIDE_MIN = SR_RESIDENT_MAX + 1;   // non-resident tensors this large use the wide form
 constexpr int64_t SR_WIDE_MID = 16384;       // ... and from this size when fewer than SR_WIDE_FILL of them
 constexpr int32_t SR_WIDE_FILL = 256;        //     (one workgroup per tensor would leave CUs idle)
@@ -1288,8 +1295,8 @@ __global__ __launch_bounds__(SR_WIDE_NT) void scalar_wide_pass(const ScalarRec* 
     const int ri = bmap[b];
     const ScalarRec& R = recs[ri];
     const Stream<W, PT, GT> S(R, h, grads[ri], table);
-    const int64_t i0 = (int64_t)(b - R.blk0) * SR_WIDE_CH;
-    const int64_t i1 = S.n < i0 + SR_WIDE_CH ? S.n : i0 + SR_WIDE_CH;
+    const int64_t i0 = (int64_t)(b - R.blk0) * R.chunk;
+    const int64_t i1 = S.n < i0 + R.chunk ? S.n : i0 + R.chunk;
     double* out = part + (size_t)b * 16;
     if constexpr (PH == 0) {
         if (S.axes) {
@@ -2683,6 +2690,9 @@ int32_t build_plan(const cresso_scalar_desc* descs, int32_t count, const cresso_
     P.groups.clear();
     P.bmap.clear();
     int32_t max_blocks = 0;
+    int64_t wide = 0;
+    for (int32_t i = 0; i < count; ++i) wide += var[(size_t)i].kind == 2 ? descs[i].numel : 0;
+    const int64_t chunk = wide_chunk(wide);
     for (int32_t j = 0; j < count; ++j) {
         const int32_t i = P.order[(size_t)j];
         ScalarRec& r = P.recs[(size_t)j];
@@ -2696,9 +2706,10 @@ int32_t build_plan(const cresso_scalar_desc* descs, int32_t count, const cresso_
         G.count += 1;
         G.lds = std::max(G.lds, lds[(size_t)i]);
         if (G.v.kind == 2) {
+            r.chunk = chunk;
             r.ctl_off = (int64_t)off;
             off += SR_CTL_BYTES;
-            const int64_t nb = (r.d.numel + SR_WIDE_CH - 1) / SR_WIDE_CH;
+            const int64_t nb = (r.d.numel + chunk - 1) / chunk;
             if (nb > (int64_t)INT32_MAX - G.nblocks)
                 return fail(CRESSO_E_UNSUPPORTED, "scalar route: wide group of more than 2^31 blocks");
             if (G.nblocks == 0) G.map_off = sizeof(int32_t) * P.bmap.size();   // relative until placed below
