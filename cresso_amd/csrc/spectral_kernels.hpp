@@ -4571,9 +4571,13 @@ int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, 
         v4 = v4 && ((uintptr_t)hd[i].grad % (4 * sizeof(GT))) == 0;
     }
     v4 = v4 && pv4;
-    const bool fast = fast_mode(g, hash_on, axes_on, h);    // MODE 1 tiles of the general sweeps (two tables)
     // the matrix-core sweeps (two or four tables; ranks up to 16: two 16-row projection tiles)
     constexpr bool MX = RM <= 16;
+    // MODE 1 tiles of the general sweeps (two tables): ranks above 16, whose
+    // full tiles the matrix-core sweeps do not take.  (Not instantiated below:
+    // more kernels in the code object slow every launch a little, a lone
+    // (2048,2048) step 93.8 -> 94.7 us with them.)
+    const bool fast = !MX && fast_mode(g, hash_on, axes_on, h);
     const bool mf = MX && mfast_mode(g, hash_on, axes_on, h);
     const bool edge = medge_mode(g, h);
     // with weight decay they read the force that sweep 1 leaves in tbuf
@@ -4627,7 +4631,8 @@ int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, 
                                    hhi, rowfx, colfx, part1, st.force_rms, step, L, h, one_round2, hd2);
             });
     } else if (fast) {
-        hipLaunchKernelGGL((sweep2_kernel<RM, KC, PT, GT, 1>), grid, blk, l2, s, g, grad, param, rowtab, coltab, meta, bins,
+        if constexpr (!MX)
+            hipLaunchKernelGGL((sweep2_kernel<RM, KC, PT, GT, 1>), grid, blk, l2, s, g, grad, param, rowtab, coltab, meta, bins,
                            ctrl, part, hist, rowfx, colfx, hash_on, axes_on, part1, st.force_rms, step, L, h);
     } else {
         hipLaunchKernelGGL((sweep2_kernel<RM, KC, PT, GT, 0>), grid, blk, l2, s, g, grad, param, rowtab, coltab, meta, bins,
@@ -4653,7 +4658,8 @@ int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, 
                                    rowfx, colfx, colfac, tbuf, part, hd3 ? hist : hpart, L, h, one_round3, hd3);
             });
     } else if (fast) {
-        hipLaunchKernelGGL((sweep3_kernel<RM, KC, PT, GT, 1>), grid, blk, l3, s, g, grad, param, rowtab, coltab, meta, bins,
+        if constexpr (!MX)
+            hipLaunchKernelGGL((sweep3_kernel<RM, KC, PT, GT, 1>), grid, blk, l3, s, g, grad, param, rowtab, coltab, meta, bins,
                            ctrl, lt, rowfx, colfx, colfac, tbuf, part, hist, hash_on, L, h);
     } else {
         hipLaunchKernelGGL((sweep3_kernel<RM, KC, PT, GT, 0>), grid, blk, l3, s, g, grad, param, rowtab, coltab, meta, bins,
@@ -4673,10 +4679,11 @@ int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, 
     // sweep 4m runs too, in place, and sweep 5q applies it)
     const bool q4 = m3 && c5c != 0 && !edge;
     if (!MX || c5c == 0) {
-        if (fast)
-            hipLaunchKernelGGL((sweep4_kernel<RM, KC, 1>), grid, blk, l4, s, g, rowtab, coltab, meta, bins, ctrl, imp, tbuf,
+        if (fast) {
+            if constexpr (!MX)
+                hipLaunchKernelGGL((sweep4_kernel<RM, KC, 1>), grid, blk, l4, s, g, rowtab, coltab, meta, bins, ctrl, imp, tbuf,
                                part, hash_on, echo_on, L, h);
-        else
+        } else
             hipLaunchKernelGGL((sweep4_kernel<RM, KC, 0>), grid, blk, l4, s, g, rowtab, coltab, meta, bins, ctrl, imp, tbuf,
                                part, hash_on, echo_on, L, h);
     } else if constexpr (MX) {

@@ -171,9 +171,11 @@ int32_t plan_spectral(const int64_t* shape, int32_t ndim, const int64_t* freqs, 
     // 467.  16 rows up to 640 blocks of them, then 32, and 64 from 256 blocks
     // on: there (2048,2048) alone would gain from 32, but batches of them
     // lose (a transformer's 88 in one group: 2.4 % of its layers' time).
+    // (Four tables skip the 32: the partial histograms of twice the blocks
+    // would take plans past the no-alloc entry's workspace limit.)
     if (mtables(g) && !g.one_d && rank <= 16 && g.rows >= 16 && g.cols >= SP_WCOLS) {
         const int64_t area = g.rows * g.slabs;
-        pr = area <= 16 * 640 ? 16 : area < 64 * 256 ? 32 : 64;
+        pr = area <= 16 * 640 ? 16 : (area < 64 * 256 && g.T == 2) ? 32 : 64;
         while (pr > g.rows) pr /= 2;
     }
     // ranks above 16 run the general sweeps, whose per-block LDS (row
