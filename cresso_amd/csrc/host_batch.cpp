@@ -6,10 +6,12 @@
 // that autograd allocates, advancing every state["step"]) costs about 0.2 us
 // per tensor and per item in CPython, which is as long as the GPU step itself.
 // BatchGuard does the same checks and writes in one pass over the Python
-// objects: gather() verifies each parameter (same object, same storage) and
-// its grad (defined, contiguous, same dtype/device/numel as at plan time) and
-// writes the grad pointers into a host array; bump() adds 1 to state["step"].
-// Any mismatch makes gather() return false and the caller rebuilds the plan.
+// objects: gather() verifies each parameter (same object, storage, shape and
+// dtype, contiguous), its grad (defined, contiguous, the parameter's shape and
+// device, the planned dtype) and its state (the planned dict, tensors, storage
+// and step count: the plan holds their addresses) and writes the grad pointers
+// into a host array; bump() adds 1 to state["step"].  Any mismatch makes
+// gather() return false and the caller rebuilds the plan.
 //
 // SpectralGuard does the same for a group's spectral tensors: fill() verifies
 // each parameter, its grad and every tensor of its state dict again on every
@@ -26,46 +28,184 @@
 
 namespace {
 
-struct BatchGuard {
-    // Strong references: a parameter cannot be freed (and a new object created
-    // at its address) while the guard lives, so the identity test is exact.
-    std::vector<py::object> params;
-    std::vector<const void*> pptr;   // param storage at plan time
-    std::vector<int> gdtype;         // grad dtype at plan time (c10::ScalarType)
-    std::vector<int64_t> numel;
-    std::vector<int> device;
+// The version of a dict's contents: a number that no dict has had before,
+// new with every change of an entry.  0: this Python keeps none.
+uint64_t dict_version(PyObject* d) {
+#if PY_VERSION_HEX < 0x030C0000
+    return reinterpret_cast<PyDictObject*>(d)->ma_version_tag;
+#else
+    (void)d;
+    return 0;
+#endif
+}
 
-    explicit BatchGuard(const py::list& ps) {
+struct BatchGuard {
+    // A planned state tensor and the storage it had at plan time.  The
+    // references keep both alive: no other tensor can take their addresses
+    // while the guard lives, and the plan's pointers stay valid memory.
+    struct Planned {
+        at::Tensor tensor;
+        c10::Storage storage;
+        const void* data;
+    };
+    // Where in the storage it was, if not all of it, and a field's form.
+    struct View {
+        const c10::TensorImpl* x;
+        int64_t offset, numel;
+        caffe2::TypeMeta dtype;
+    };
+    // One (key, value) of a state dict at plan time.
+    struct Entry {
+        py::object key, value;   // value: null unless planned
+        bool step;
+    };
+    struct Item {
+        py::object param, dict;
+        const void* pptr;
+        std::vector<int64_t> sizes;
+        int pdtype, gdtype, device;
+        std::vector<Entry> entries;   // every entry, in the dict's order
+        int64_t step0;                // state["step"] at plan time
+        mutable uint64_t version;     // the dict's, when its entries were last compared (or written by bump)
+    };
+    std::vector<Item> items;
+    std::vector<Planned> planned;
+    std::vector<View> views;
+    bool with_state = false;
+    int64_t ran = 0;                      // steps since plan time (bump)
+    mutable uint64_t state_version = 0;   // the optimizer's state dict's, when its items were last compared
+
+    // states: empty, or one dict per parameter; keys: each state's planned keys.
+    BatchGuard(const py::list& ps, const py::list& states, const py::list& keys) {
         const size_t n = ps.size();
-        params.reserve(n);
+        if ((states.size() != 0 && states.size() != n) || keys.size() != states.size())
+            throw std::invalid_argument("BatchGuard: one state and its keys per parameter");
+        with_state = states.size() != 0;
+        items.reserve(n);
         for (size_t i = 0; i < n; ++i) {
             PyObject* o = ps[i].ptr();
             if (!THPVariable_Check(o)) throw std::invalid_argument("BatchGuard: parameters must be tensors");
             const at::Tensor& t = THPVariable_Unpack(o);
             const at::Tensor& g = t.grad();
             if (!g.defined()) throw std::invalid_argument("BatchGuard: every parameter needs a grad at plan time");
-            params.push_back(py::reinterpret_borrow<py::object>(o));
-            pptr.push_back(t.data_ptr());
-            gdtype.push_back(static_cast<int>(g.scalar_type()));
-            numel.push_back(t.numel());
-            device.push_back(t.device().index());
+            // A strong reference: the parameter cannot be freed (and a new
+            // object created at its address) while the guard lives, so the
+            // identity test is exact.
+            Item it{};
+            it.param = py::reinterpret_borrow<py::object>(o);
+            it.pptr = t.data_ptr();
+            it.sizes = t.sizes().vec();
+            it.pdtype = static_cast<int>(t.scalar_type());
+            it.gdtype = static_cast<int>(g.scalar_type());
+            it.device = t.device().index();
+            if (with_state) plan_state(it, states[i].ptr(), keys[i].ptr());
+            items.push_back(std::move(it));
         }
+    }
+
+    void plan_state(Item& it, PyObject* st, PyObject* want) {
+        if (!PyDict_Check(st)) throw std::invalid_argument("BatchGuard: a state must be a dict");
+        it.dict = py::reinterpret_borrow<py::object>(st);
+        it.step0 = -1;
+        Py_ssize_t missing = PySequence_Size(want);
+        PyObject *k, *v;
+        Py_ssize_t pos = 0;
+        while (PyDict_Next(st, &pos, &k, &v)) {
+            Entry e{py::reinterpret_borrow<py::object>(k), py::object(), false};
+            const int used = PySequence_Contains(want, k);
+            if (used < 0) throw py::error_already_set();
+            if (used) {
+                if (!THPVariable_Check(v)) throw std::invalid_argument("BatchGuard: a planned state must be a tensor");
+                e.value = py::reinterpret_borrow<py::object>(v);
+                const at::Tensor& x = THPVariable_Unpack(v);
+                planned.push_back(Planned{x, x.storage(), x.storage().data()});
+                if (x.numel() != 1 || x.storage().nbytes() != x.itemsize())
+                    views.push_back(View{x.unsafeGetTensorImpl(), x.storage_offset(), x.numel(), x.dtype()});
+                --missing;
+            } else if (PyUnicode_Check(k) && PyUnicode_CompareWithASCIIString(k, "step") == 0 && PyLong_Check(v)) {
+                e.step = true;
+                it.step0 = PyLong_AsLongLong(v);
+            }
+            it.entries.push_back(std::move(e));
+        }
+        if (missing != 0 || it.step0 < 0) throw std::invalid_argument("BatchGuard: a state lacks its 'step' or a planned key");
+        it.version = dict_version(st);
+    }
+
+    // Whether a state dict holds the planned entries and step count.
+    bool entries_hold(const Item& it) const {
+        const uint64_t version = dict_version(it.dict.ptr());
+        if (version != 0 && version == it.version) return true;
+        size_t j = 0;
+        PyObject *k, *v;
+        Py_ssize_t pos = 0;
+        while (PyDict_Next(it.dict.ptr(), &pos, &k, &v)) {
+            if (j == it.entries.size()) return false;
+            const Entry& e = it.entries[j++];
+            if (k != e.key.ptr() || (e.value && v != e.value.ptr())) return false;
+            if (e.step) {
+                if (!PyLong_Check(v)) return false;
+                const long long s = PyLong_AsLongLong(v);
+                if (s == -1) PyErr_Clear();
+                if (s != it.step0 + ran) return false;
+            }
+        }
+        if (j != it.entries.size()) return false;
+        it.version = version;
+        return true;
+    }
+
+    // Whether the optimizer's state holds what the plan was made from.
+    bool states_hold(PyObject* state) const {
+        if (!PyDict_Check(state)) return false;
+        const uint64_t version = dict_version(state);
+        if (version == 0 || version != state_version) {
+            for (const Item& it : items) {
+                PyObject* st = PyDict_GetItemWithError(state, it.param.ptr());   // borrowed
+                if (!st && PyErr_Occurred()) throw py::error_already_set();
+                if (st != it.dict.ptr()) return false;
+            }
+            state_version = version;
+        }
+        for (const Item& it : items)
+            if (!entries_hold(it)) return false;
+        for (const Planned& p : planned)
+            if (p.tensor.unsafeGetTensorImpl()->unsafe_storage().unsafeGetStorageImpl() != p.storage.unsafeGetStorageImpl() ||
+                p.storage.data() != p.data)
+                return false;
+        for (const View& v : views)
+            if (v.x->storage_offset() != v.offset ||
+                (v.numel != 1 && (v.x->numel() != v.numel || v.x->dtype() != v.dtype || !v.x->is_contiguous())))
+                return false;
+        return true;
+    }
+
+    // Whether the parameters and, given the optimizer's state, their states
+    // are those of plan time.
+    bool holds(const py::list& ps, const py::object& state) const {
+        if (ps.size() != items.size()) return false;
+        for (size_t i = 0; i < items.size(); ++i) {
+            const Item& it = items[i];
+            if (PyList_GET_ITEM(ps.ptr(), i) != it.param.ptr()) return false;
+            const at::Tensor& t = THPVariable_Unpack(it.param.ptr());
+            if (t.data_ptr() != it.pptr || static_cast<int>(t.scalar_type()) != it.pdtype ||
+                t.sizes() != c10::IntArrayRef(it.sizes) || !t.is_contiguous())
+                return false;
+        }
+        return !with_state || state.is_none() || states_hold(state.ptr());
     }
 
     // Writes params[i].grad.data_ptr() to out[i]; false if anything differs
     // from plan time (then out is partially written and must not be used).
-    bool gather(const py::list& ps, uintptr_t out_addr) const {
-        const size_t n = params.size();
-        if (ps.size() != n) return false;
+    bool gather(const py::list& ps, uintptr_t out_addr, const py::object& state) const {
+        if (!holds(ps, state)) return false;
         void** out = reinterpret_cast<void**>(out_addr);
-        for (size_t i = 0; i < n; ++i) {
-            PyObject* o = ps[i].ptr();
-            if (o != params[i].ptr()) return false;
-            const at::Tensor& t = THPVariable_Unpack(o);
-            if (t.data_ptr() != pptr[i]) return false;
+        for (size_t i = 0; i < items.size(); ++i) {
+            const Item& it = items[i];
+            const at::Tensor& t = THPVariable_Unpack(it.param.ptr());
             const at::Tensor& g = t.grad();
-            if (!g.defined() || static_cast<int>(g.scalar_type()) != gdtype[i] || g.numel() != numel[i] ||
-                g.device().index() != device[i] || !g.device().is_cuda() || g.is_sparse() || !g.is_contiguous())
+            if (!g.defined() || static_cast<int>(g.scalar_type()) != it.gdtype || g.sizes() != t.sizes() ||
+                g.device().index() != it.device || !g.device().is_cuda() || g.is_sparse() || !g.is_contiguous())
                 return false;
             out[i] = g.data_ptr();
         }
@@ -73,8 +213,10 @@ struct BatchGuard {
     }
 
     // state["step"] += 1 for each state dict (the library advanced its own copy).
-    void bump(const py::list& states) const {
+    void bump(const py::list& states) {
         static PyObject* key = PyUnicode_InternFromString("step");
+        ++ran;
+        size_t i = 0;
         for (const py::handle& h : states) {
             PyObject* d = h.ptr();
             PyObject* v = PyDict_GetItemWithError(d, key);   // borrowed
@@ -86,9 +228,14 @@ struct BatchGuard {
             if (s == -1 && PyErr_Occurred()) throw py::error_already_set();
             PyObject* nv = PyLong_FromLongLong(s + 1);
             if (!nv) throw py::error_already_set();
+            // (the step's own write keeps the entries compared, if they were)
+            const bool known = with_state && i < items.size() && d == items[i].dict.ptr() &&
+                               dict_version(d) == items[i].version && s + 1 == items[i].step0 + ran;
             const int rc = PyDict_SetItem(d, key, nv);
             Py_DECREF(nv);
             if (rc != 0) throw py::error_already_set();
+            if (known) items[i].version = dict_version(d);
+            ++i;
         }
     }
 };
@@ -250,8 +397,10 @@ bool same_objects(const py::list& a, const py::list& b) {
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.doc() = "Per-step host bookkeeping of the CRESSO5 scalar plan";
     py::class_<BatchGuard>(m, "BatchGuard")
-        .def(py::init<const py::list&>())
-        .def("gather", &BatchGuard::gather)
+        .def(py::init<const py::list&, const py::list&, const py::list&>(), py::arg("params"),
+             py::arg("states") = py::list(), py::arg("keys") = py::list())
+        .def("holds", &BatchGuard::holds, py::arg("params"), py::arg("state") = py::none())
+        .def("gather", &BatchGuard::gather, py::arg("params"), py::arg("out"), py::arg("state") = py::none())
         .def("bump", &BatchGuard::bump);
     py::class_<SpectralGuard>(m, "SpectralGuard")
         .def(py::init<const py::list&, const py::list&, const std::vector<std::pair<int, int>>&, const std::vector<int>&,

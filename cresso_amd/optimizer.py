@@ -114,17 +114,23 @@ class _ScalarBatch:
         self.states = states
         self.device = device
         self.pptrs = [p.data_ptr() for p in params]
+        self.shapes = [(p.shape, p.dtype) for p in params]
         self.gdtypes = [g.dtype for g in grads]   # the plan's descriptors fix the grad dtype
         self.hyper_key = self.key_of(group)
+        # the plan holds the state tensors' addresses and step counts: what it
+        # was made from stays referenced here and is compared on every step
+        self.keys = [_MICRO_KEYS if "micro_energy" in st else _SCALAR_KEYS for st in states]
+        self.planned = [[(st[k], st[k].data_ptr()) for k in ks] for st, ks in zip(states, self.keys)]
+        self.step0 = [int(st["step"]) for st in states]
+        self.ran = 0
         descs = (_native.ScalarDesc * len(params))()
         for i, (p, g, st) in enumerate(zip(params, grads, states)):
             d = descs[i]
             d.param = p.data_ptr()
             d.grad = g.data_ptr()
-            micro = "micro_energy" in st
-            for j, k in enumerate(_MICRO_KEYS if micro else _SCALAR_KEYS):
-                d.state[j] = st[k].data_ptr()
-            d.route = _native.ROUTE_MICRO if micro else _native.ROUTE_SCALAR
+            for j, (_, ptr) in enumerate(self.planned[i]):
+                d.state[j] = ptr
+            d.route = _native.ROUTE_MICRO if self.keys[i] is _MICRO_KEYS else _native.ROUTE_SCALAR
             for a, s in enumerate(p.shape):
                 d.shape[a] = int(s)
             d.numel = p.numel()
@@ -151,7 +157,7 @@ class _ScalarBatch:
         hb = _native.host_batch()
         if hb is not None and all(p.grad is not None for p in params):   # (not for contiguous copies)
             try:
-                self.guard = hb.BatchGuard(list(params))
+                self.guard = hb.BatchGuard(list(params), list(states), self.keys)
             except (ValueError, RuntimeError):
                 self.guard = None
 
@@ -159,10 +165,26 @@ class _ScalarBatch:
     def key_of(group: dict):
         return tuple(group[k] for k in _native.HYPER_DOUBLES if k != "lr") + (group["warmup_steps"], group["maximize"])
 
-    def matches(self, params: List[Tensor], gdtypes: List[torch.dtype], group: dict) -> bool:
+    def states_hold(self, states: List[dict]) -> bool:
+        """The states are the dicts the plan was made from, with the planned
+        tensors, storage and step counts."""
+        for st, mine, ks, ts, s0 in zip(states, self.states, self.keys, self.planned, self.step0):
+            if st is not mine or st.get("step") != s0 + self.ran:
+                return False
+            if any(st.get(k) is not t or t.data_ptr() != ptr for k, (t, ptr) in zip(ks, ts)):
+                return False
+        return True
+
+    def matches(self, params: List[Tensor], states: List[dict], gdtypes: List[torch.dtype], group: dict,
+                state: dict) -> bool:
+        """Whether the plan still describes these tensors (state: the optimizer's)."""
+        if self.key_of(group) != self.hyper_key or gdtypes != self.gdtypes:
+            return False
+        if self.guard is not None:
+            return self.guard.holds(params, state)
         return (len(params) == len(self.params) and all(a is b for a, b in zip(params, self.params))
-                and [p.data_ptr() for p in params] == self.pptrs and self.key_of(group) == self.hyper_key
-                and gdtypes == self.gdtypes)
+                and [p.data_ptr() for p in params] == self.pptrs and [(p.shape, p.dtype) for p in params] == self.shapes
+                and all(p.is_contiguous() for p in params) and self.states_hold(states))
 
     @staticmethod
     def grads_ready(params: List[Tensor]) -> bool:
@@ -179,21 +201,18 @@ class _ScalarBatch:
         _native.check(self.lib.cresso_scalar_plan_step(self.plan, ctypes.c_void_p(self.table.data_ptr()), arr,
                                                        ctypes.byref(hyper), ctypes.c_void_p(stream)),
                       "scalar route step")
+        self.ran += 1
         if self.guard is not None:
             self.guard.bump(self.states)
         else:
             for st in self.states:
                 st["step"] += 1
 
-    def fast_step(self, group: dict) -> bool:
-        """Steady state in C++: same params and storage, fresh grads of the
-        planned dtype; False (nothing launched) when anything changed."""
-        if self.guard is None or self.key_of(group) != self.hyper_key:
-            return False
-        if not self.guard.gather(group["params"], ctypes.addressof(self.gbuf)):
-            return False
-        self.run(group, None)
-        return True
+    def gather(self, params: List[Tensor], group: dict, state: dict) -> bool:
+        """Steady state in C++: same params, states and storage, fresh grads of
+        the planned dtype (their pointers then are in self.gbuf)."""
+        return (self.guard is not None and self.key_of(group) == self.hyper_key
+                and self.guard.gather(params, ctypes.addressof(self.gbuf), state))
 
     def __del__(self):
         plan = getattr(self, "plan", None)
@@ -365,12 +384,16 @@ class CRESSO5(Optimizer):
         if batch is None or self._group_other.get(gi, True):
             return False
         if batch.guard is not None:
-            return batch.fast_step(group)
+            if not batch.gather(group["params"], group, self.state):
+                return False
+            batch.run(group, None)
+            return True
         try:
             gptrs = [p.grad.data_ptr() for p in batch.params]
+            states = [self.state[p] for p in batch.params]
         except (AttributeError, RuntimeError):
             return False
-        if (not batch.matches(group["params"], [p.grad.dtype for p in batch.params], group)
+        if (not batch.matches(group["params"], states, [p.grad.dtype for p in batch.params], group, self.state)
                 or not batch.grads_ready(batch.params)):
             return False
         batch.run(group, gptrs)
@@ -399,8 +422,7 @@ class CRESSO5(Optimizer):
             return False
         between = None
         if batch is not None:
-            if (batch is not self._batches.get((gi, "scalar")) or batch.key_of(group) != batch.hyper_key
-                    or not batch.guard.gather(batch.params, ctypes.addressof(batch.gbuf))):
+            if batch is not self._batches.get((gi, "scalar")) or not batch.gather(batch.params, group, self.state):
                 return False
             between = lambda: batch.run(group, None, hyper)   # noqa: E731
         if not step.fill(self.state):
@@ -506,9 +528,12 @@ class CRESSO5(Optimizer):
             scalar_st.append(st)
         self._group_other[gi] = other
 
+        # (before the spectral launches: a refused state leaves every tensor as it was)
+        batch = self._scalar_plan(gi, group, scalar_ps, scalar_gs, scalar_st)
+
         def scalar_step() -> None:
             if scalar_ps:
-                self._step_scalar_batch(gi, group, scalar_ps, scalar_gs, scalar_st)
+                self._step_scalar_batch(gi, group, batch, scalar_ps, scalar_gs, scalar_st)
             else:
                 self._batches.pop((gi, "scalar"), None)
 
@@ -524,17 +549,38 @@ class CRESSO5(Optimizer):
         for p, data in copies:
             p.detach().copy_(data)
 
-    def _step_scalar_batch(self, gi: int, group: dict, scalar_ps: List[Tensor], scalar_gs: List[Tensor],
-                           scalar_st: List[dict]) -> None:
-        devices = {p.device for p in scalar_ps}
-        if len(devices) != 1:
+    def _scalar_plan(self, gi: int, group: dict, scalar_ps: List[Tensor], scalar_gs: List[Tensor],
+                     scalar_st: List[dict]) -> Optional[_ScalarBatch]:
+        """The cached plan if it describes these tensors; None, with their
+        devices and states checked, when a new one is needed."""
+        if not scalar_ps:
+            return None
+        if len({p.device for p in scalar_ps}) != 1:
             raise RuntimeError("CRESSO5 scalar route: all parameters of a group must be on one device")
         batch = self._batches.get((gi, "scalar"))
-        if batch is None or not batch.matches(scalar_ps, [g.dtype for g in scalar_gs], group):
+        if batch is not None and batch.matches(scalar_ps, scalar_st, [g.dtype for g in scalar_gs], group, self.state):
+            return batch
+        for p, st in zip(scalar_ps, scalar_st):
+            if "micro_energy" not in st:
+                self._check_scalar_state(p, st)
+        return None
+
+    def _step_scalar_batch(self, gi: int, group: dict, batch: Optional[_ScalarBatch], scalar_ps: List[Tensor],
+                           scalar_gs: List[Tensor], scalar_st: List[dict]) -> None:
+        if batch is None:
             self._batches[(gi, "scalar")] = None  # drop the old plan first
             batch = _ScalarBatch(scalar_ps, scalar_gs, scalar_st, group, scalar_ps[0].device)
             self._batches[(gi, "scalar")] = batch
         batch.run(group, [g.data_ptr() for g in scalar_gs])
+
+    @staticmethod
+    def _check_scalar_state(p: Tensor, st: dict) -> None:
+        want = _state_dtype(p.dtype)
+        for k in _SCALAR_KEYS:
+            v = st.get(k)
+            if not torch.is_tensor(v) or v.dtype != want or v.device != p.device or v.numel() != 1:
+                got = f"{v.dtype} with {v.numel()} elements on {v.device}" if torch.is_tensor(v) else type(v).__name__
+                raise RuntimeError(f"CRESSO5 scalar route: state {k!r} is {got}, expected one {want} on {p.device}")
 
     @staticmethod
     def _check_micro_state(p: Tensor, st: dict) -> None:
@@ -549,6 +595,9 @@ class CRESSO5(Optimizer):
         for k in _MICRO_KEYS[:3]:
             if st[k].shape != p.shape or not st[k].is_contiguous():
                 raise RuntimeError(f"CRESSO5 micro route: state {k!r} must be contiguous with the parameter's shape")
+        for k in _MICRO_KEYS[3:]:
+            if st[k].numel() != 1:
+                raise RuntimeError(f"CRESSO5 micro route: state {k!r} has {st[k].numel()} elements, expected one")
 
     def _spectral_step(self, items, group: dict, between=None) -> None:
         """Every spectral tensor of the group: (param, grad, state) each;

@@ -284,6 +284,56 @@ def test_host_batch_guard_holds_references_and_refuses_replaced_params():
     assert ref() is None              # released with the guard
 
 
+def test_host_batch_guard_compares_layouts_and_states():
+    # what a scalar plan holds the addresses of: each change, seen; undone, accepted again
+    hb = _native.host_batch()
+    assert hb is not None, "cresso_amd/_hostbatch extension not built"
+    ps = [torch.nn.Parameter(torch.zeros(4, 4)) for _ in range(3)]
+    keys = [("q", "impulse")] * 2 + [("field",)]
+    state = {}
+    for p, ks in zip(ps, keys):
+        p.grad = torch.zeros(4, 4)
+        state[p] = dict(step=5, other="kept", **{k: torch.zeros(4, 4) if k == "field" else torch.zeros(()) for k in ks})
+    pair = torch.zeros(2)
+    state[ps[1]].update(q=pair[0], impulse=pair[1])   # views of one buffer
+    states = [state[p] for p in ps]
+    guard = hb.BatchGuard(ps, states, keys)
+    assert guard.holds(ps, state) and guard.holds(ps, state)
+
+    def seen(change, undo):
+        change()
+        assert not guard.holds(ps, state)
+        undo()
+        assert guard.holds(ps, state)
+
+    data = ps[0].data
+    for other in (data.t(), data.view(2, 8), data.clone()):
+        seen(lambda: setattr(ps[0], "data", other), lambda: setattr(ps[0], "data", data))
+    q = states[0]["q"]
+    seen(lambda: states[0].update(q=q.clone()), lambda: states[0].update(q=q))
+    kept = q.data
+    seen(lambda: setattr(q, "data", torch.ones(())), lambda: setattr(q, "data", kept))
+    view = states[1]["q"]
+    seen(lambda: setattr(view, "data", pair[1]), lambda: setattr(view, "data", pair[0]))
+    field = states[2]["field"].data
+    seen(lambda: setattr(states[2]["field"], "data", field.t()), lambda: setattr(states[2]["field"], "data", field))
+    seen(lambda: setattr(states[2]["field"], "data", field[:2]), lambda: setattr(states[2]["field"], "data", field))
+    seen(lambda: states[1].update(step=4), lambda: states[1].update(step=5))
+    seen(lambda: state.update({ps[2]: dict(states[2])}), lambda: state.update({ps[2]: states[2]}))
+    guard.bump(states)
+    assert [s["step"] for s in states] == [6, 6, 6] and guard.holds(ps, state)
+    states[0]["step"] = 5
+    assert not guard.holds(ps, state)
+    guard.bump(states)   # (a count that was changed is not taken for the plan's after the next step either)
+    assert not guard.holds(ps, state)
+    states[0]["step"] = 7
+    assert guard.holds(ps, state)
+    states[0]["new"] = 1
+    assert not guard.holds(ps, state)
+    with pytest.raises(ValueError):
+        hb.BatchGuard(ps, states, [("q", "missing")] * 3)
+
+
 def test_spectral_lane_assignment():
     # the multi-tensor spectral step: m tensors of one shape use min(4, m)
     # distinct lanes (one workspace each), shapes spread over the lanes

@@ -95,3 +95,109 @@ def test_steady_step_refuses_what_the_general_step_refuses():
     opt.state[ps[0]]["hash_energy"] = opt.state[ps[0]]["hash_energy"].t().contiguous()
     with pytest.raises(RuntimeError, match="shape"):
         opt.step()
+
+
+MICRO = dict(micro_field_max_size=64)
+SCALARS = [(4096, 16), (900,), (16, 64), (10,), (6, 8)]   # the last two: micro fields with MICRO
+GROUPS = {"mixed": SCALARS + [(64, 65)], "scalar": SCALARS}
+KEPT = []   # replaced storage stays alive: a step that still used it would write to live memory
+
+
+def _layout(ps, opt):
+    ps[0].data = ps[0].data.t()   # same storage, other element order
+
+
+def _reshape(ps, opt):
+    ps[2].data = ps[2].data.view(64, 16)
+
+
+def _state_entry(ps, opt):
+    st = opt.state[ps[0]]
+    KEPT.append(st["q"])
+    st["q"] = 0.5 * st["q"]
+
+
+def _state_storage(ps, opt):
+    st = opt.state[ps[1]]
+    KEPT.append(st["impulse"].data)
+    st["impulse"].data = 0.5 * st["impulse"].data
+
+
+def _state_dict(ps, opt):
+    KEPT.append(opt.state[ps[1]])
+    opt.state[ps[1]] = {k: 0.5 * v if torch.is_tensor(v) else v for k, v in opt.state[ps[1]].items()}
+
+
+def _micro_field(ps, opt):
+    st = opt.state[ps[4]]
+    KEPT.append(st["micro_energy"])
+    st["micro_energy"] = 0.5 * st["micro_energy"]
+
+
+def _step_count(ps, opt):
+    opt.state[ps[0]]["step"] = 1
+    opt.state[ps[4]]["step"] = 0
+
+
+CHANGES = [_layout, _reshape, _state_entry, _state_storage, _state_dict, _micro_field, _step_count]
+
+
+@pytest.mark.parametrize("group", sorted(GROUPS))
+@pytest.mark.parametrize("change", CHANGES, ids=[c.__name__[1:] for c in CHANGES])
+def test_planned_scalar_tensors_follow_changes(group, change):
+    """A change to a scalar or micro tensor's layout, shape, state or step count after steady steps, against an
+    optimizer that plans every step anew: the same bits."""
+    announce(f"{group} group, {change.__name__[1:]} changed")
+    gen, pair = _pair(GROUPS[group], **MICRO)
+
+    def at(k, ps, opt):
+        if k == 4:
+            change(ps, opt)
+            for p in ps:
+                p.grad = 1e-3 * torch.arange(p.numel(), device="cuda", dtype=torch.float32).view(p.shape)
+        if opt is pair[1][1]:
+            opt._batches.clear()
+
+    _steps(gen, pair, 7, at)
+    KEPT.clear()
+
+
+def _no_q(ps, opt):
+    del opt.state[ps[0]]["q"]
+
+
+def _wide_q(ps, opt):
+    opt.state[ps[0]]["q"] = opt.state[ps[0]]["q"].double()
+
+
+def _host_impulse(ps, opt):
+    opt.state[ps[0]]["impulse"] = opt.state[ps[0]]["impulse"].cpu()
+
+
+def _long_action(ps, opt):
+    opt.state[ps[1]]["action"] = torch.zeros(2, device="cuda")
+
+
+def _flat_field(ps, opt):
+    opt.state[ps[4]]["micro_energy"] = opt.state[ps[4]]["micro_energy"].view(-1)
+
+
+REFUSED = [_no_q, _wide_q, _host_impulse, _long_action, _flat_field]
+
+
+@pytest.mark.parametrize("group", sorted(GROUPS))
+@pytest.mark.parametrize("change", REFUSED, ids=[c.__name__[1:] for c in REFUSED])
+def test_planned_scalar_tensors_refuse_bad_states(group, change):
+    """A scalar or micro state that no plan can be made of is refused on a steady step too."""
+    gen, pair = _pair(GROUPS[group], **MICRO)
+    _steps(gen, pair, 4)
+    ps, opt = pair[0]
+    for p in ps:
+        p.grad = torch.zeros_like(p)
+    before = [p.detach().clone() for p in ps]
+    change(ps, opt)
+    with pytest.raises(RuntimeError, match="state"):
+        opt.step()
+    torch.cuda.synchronize()
+    for i in (0, 1, 4):
+        assert torch.equal(ps[i], before[i])
