@@ -579,10 +579,11 @@ extern "C" int32_t cresso_fork_begin(cresso_fork* F, void* caller, void* const* 
 
 extern "C" int32_t cresso_fork_end(cresso_fork* F, void* caller, void* const* streams, int32_t n) {
     if (!F || !streams || n < 0 || (size_t)n >= F->ev.size()) return fail(CRESSO_E_INVALID, "join of %d streams", n);
-    hipError_t e = hipSuccess;
-    for (int32_t i = 0; i < n && e == hipSuccess; ++i) {
-        e = hipEventRecord(F->ev[i + 1], reinterpret_cast<hipStream_t>(streams[i]));
-        if (e == hipSuccess) e = hipStreamWaitEvent(reinterpret_cast<hipStream_t>(caller), F->ev[i + 1], 0);
+    hipError_t e = hipSuccess;   // the first error; the other streams join all the same
+    for (int32_t i = 0; i < n; ++i) {
+        hipError_t rc = hipEventRecord(F->ev[i + 1], reinterpret_cast<hipStream_t>(streams[i]));
+        if (rc == hipSuccess) rc = hipStreamWaitEvent(reinterpret_cast<hipStream_t>(caller), F->ev[i + 1], 0);
+        if (e == hipSuccess) e = rc;
     }
     return e == hipSuccess ? CRESSO_OK : hip_fail(e, "join");
 }

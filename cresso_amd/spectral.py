@@ -325,7 +325,7 @@ class Launch:
     def run(self, hyper, between=None) -> None:
         """between: run after the launches, on the caller's stream, beside the
         side streams."""
-        lib, open_ = self.engine.lib, []
+        lib, forked = self.engine.lib, []
         try:
             for device, arr, n, lanes in self.devices:
                 caller = ctypes.c_void_p(_native.stream_handle(device))
@@ -334,15 +334,28 @@ class Launch:
                 else:
                     fork = self.engine._fork(device, lanes)
                     handles, count = fork.handles, lanes
+                    forked.append((fork, caller, lanes))   # (a begin that fails may have forked some)
                     _native.check(lib.cresso_fork_begin(fork.fork, caller, handles, lanes), "side streams")
-                    open_.append((fork, caller, lanes))
                 _native.check(lib.cresso_spectral_step_units(arr, n, ctypes.byref(hyper), handles, count),
                               "spectral route step")
             if between is not None:
                 between()
-        finally:
-            for fork, caller, lanes in open_:
-                _native.check(lib.cresso_fork_end(fork.fork, caller, fork.handles, lanes), "side streams")
+        except BaseException:
+            self._join(forked)   # (the first error is the one to raise)
+            raise
+        failed = self._join(forked)
+        if failed is not None:
+            raise failed
+
+    def _join(self, forked: list):
+        """Every forked stream joins its caller's, whatever happens; -> the first error."""
+        failed = None
+        for fork, caller, lanes in forked:
+            try:
+                _native.check(self.engine.lib.cresso_fork_end(fork.fork, caller, fork.handles, lanes), "side streams")
+            except RuntimeError as err:
+                failed = failed or err
+        return failed
 
 
 class SteadyStep:

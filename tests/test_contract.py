@@ -381,6 +381,51 @@ def test_spectral_batch_units_and_chunks():
     assert [len(u[4]) for u in eng._units(prepared, sts)] == [1] * len(prepared)
 
 
+@pytest.mark.parametrize("fails", ["begin", "step", "between", "end", "step and end"])
+def test_spectral_launch_joins_its_streams_after_an_error(fails, monkeypatch):
+    # whatever fails in a step on side streams, every stream that was forked
+    # joins the caller's again, and the first error is the one raised (a
+    # recording stand-in for the library: nothing is launched)
+    import ctypes
+    import types
+
+    from cresso_amd import spectral
+
+    calls, handles = [], (ctypes.c_void_p * 2)(16, 32)
+
+    def op(name):
+        def call(first, *args):
+            dev = int(first) if not hasattr(first, "_length_") else len(calls)
+            calls.append((name, dev if name != "step" else -1))
+            return -1 if name in fails.split(" and ") else 0
+        return call
+
+    lib = types.SimpleNamespace(cresso_fork_begin=op("begin"), cresso_fork_end=op("end"),
+                                cresso_spectral_step_units=op("step"))
+    forks = {"a": types.SimpleNamespace(fork=1, handles=handles), "b": types.SimpleNamespace(fork=2, handles=handles)}
+    engine = types.SimpleNamespace(lib=lib, _fork=lambda device, lanes: forks[device])
+    launch = spectral.Launch.__new__(spectral.Launch)
+    launch.engine, launch.keep = engine, []
+    launch.devices = [(d, (_native.SpectralUnit * 1)(), 1, 2) for d in ("a", "b")]
+    monkeypatch.setattr(_native, "stream_handle", lambda device: 64)
+
+    def check(rc, what):
+        if rc:
+            raise RuntimeError(f"{what} {calls[-1][0]}")
+
+    monkeypatch.setattr(_native, "check", check)
+
+    def between():
+        calls.append(("between", -1))
+        if fails == "between":
+            raise RuntimeError("between")
+
+    with pytest.raises(RuntimeError, match=fails.split(" and ")[0]):
+        launch.run(_native.Hyper(), between)
+    begun = [d for name, d in calls if name == "begin"]
+    assert begun and [d for name, d in calls if name == "end"] == begun
+
+
 def test_load_state_dict_keeps_same_plan_workspaces():
     """A spectral workspace depends only on its plan key (shape, freqs,
     hash_bins, hash_tables, work dtype): load_state_dict keeps those the
