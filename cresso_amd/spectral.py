@@ -30,6 +30,7 @@ uses (`retain`) and frees the others; `reset()` frees them all.
 from __future__ import annotations
 
 import ctypes
+import weakref
 from typing import Dict, List, Sequence, Tuple
 
 import torch
@@ -362,8 +363,9 @@ class SteadyStep:
     """The steady state of a group's spectral tensors: the units of a step that
     has run, with their workspaces, and the C++ guard that checks every
     parameter, grad and state tensor again on each step and writes their
-    descriptors.  run() returns False, with nothing launched, when anything
-    differs; the general path then takes the step."""
+    descriptors.  fill() returns False when anything differs; the general path
+    then takes the step.  The workspaces stay the engine's: one that it drops
+    is freed, and the steady step is at an end (ready())."""
 
     def __init__(self, engine: SpectralEngine, items, group: dict, hb):
         plan = engine._plan(items, group)
@@ -384,9 +386,14 @@ class SteadyStep:
             units.append((ws, (_native.SpectralDesc * len(ds)).from_buffer(self.descs, at * size), lane, device))
             at += len(ds)
         self.launch = Launch(engine, units)
+        self.launch.keep = [u[1] for u in units]
+        self.workspaces = [weakref.ref(u[0]) for u in units]
+
+    def ready(self) -> bool:
+        return self.version == self.engine.version and all(ws() is not None for ws in self.workspaces)
 
     def fill(self, state: dict) -> bool:
-        return self.version == self.engine.version and self.guard.fill(state, ctypes.addressof(self.descs))
+        return self.ready() and self.guard.fill(state, ctypes.addressof(self.descs))
 
     def run(self, state: dict, hyper, between=None) -> None:
         """The step (after fill() returned True)."""

@@ -381,6 +381,42 @@ def test_spectral_batch_units_and_chunks():
     assert [len(u[4]) for u in eng._units(prepared, sts)] == [1] * len(prepared)
 
 
+def test_steady_step_holds_no_dropped_workspace():
+    # SpectralEngine.reset() frees every workspace; a steady step that was made
+    # before must neither keep one alive nor run with it (stand-ins for the
+    # workspaces: nothing is launched)
+    import gc
+    import types
+    import weakref
+
+    from cresso_amd.spectral import SpectralEngine, SteadyStep
+
+    if not (ROOT / "cresso_amd" / "libcresso_hip.so").exists():
+        pytest.skip("library not built")
+
+    class Workspace:
+        def __init__(self):
+            self.plan, self.buf, self.count = types.SimpleNamespace(value=8), torch.zeros(16), None
+
+    ps = [torch.nn.Parameter(torch.zeros(64, 48)), torch.nn.Parameter(torch.zeros(32, 40))]
+    opt = CRESSO5(ps, cuda_ops="required", rank=8, hash_bins=64, hash_tables=2)
+    group = opt.param_groups[0]
+    eng = SpectralEngine()
+    items = []
+    for lane, p in enumerate(ps):
+        p.grad = torch.zeros_like(p)
+        st = opt._init_spectral(p, group)
+        items.append((p, p.grad, st))
+        eng.ws[(eng.plan_key(p, st, group), False, lane)] = Workspace()
+    step = SteadyStep(eng, items, group, _native.host_batch())
+    refs = [weakref.ref(w) for w in eng.ws.values()]
+    assert step.ready()
+    eng.reset()
+    gc.collect()
+    assert not step.ready() and not step.fill(opt.state)
+    assert all(r() is None for r in refs)
+
+
 @pytest.mark.parametrize("fails", ["begin", "step", "between", "end", "step and end"])
 def test_spectral_launch_joins_its_streams_after_an_error(fails, monkeypatch):
     # whatever fails in a step on side streams, every stream that was forked
