@@ -555,8 +555,16 @@ extern "C" cresso_fork* cresso_fork_create(int32_t lanes) {
         fail(CRESSO_E_INVALID, "fork of %d streams", lanes);
         return nullptr;
     }
-    cresso_fork* F = new cresso_fork();
-    for (int32_t i = 0; i <= lanes; ++i) {
+    cresso_fork* F = nullptr;
+    try {   // (no exception leaves a C entry)
+        F = new cresso_fork();
+        F->ev.reserve((size_t)lanes + 1);
+    } catch (const std::exception&) {
+        delete F;
+        fail(CRESSO_E_INVALID, "fork of %d streams: out of host memory", lanes);
+        return nullptr;
+    }
+    for (size_t i = 0; i <= (size_t)lanes; ++i) {
         hipEvent_t e = nullptr;
         const hipError_t rc = hipEventCreateWithFlags(&e, hipEventDisableTiming);
         if (rc != hipSuccess) {
