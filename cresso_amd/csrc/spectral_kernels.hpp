@@ -21,8 +21,8 @@
 //   Z1_r = sum_rows a1_r x, Z2_r = sum_rows a2_r x over the lane's column,
 //   combined with the lane's b values at the end; reconstruction is
 //   out = alpha_0(row) + sum_k alpha_k(row) b_k(col) with alpha built per row
-//   panel in LDS from the mode coefficients.  On the fast path (MODE 1) sweeps
-//   3 and 4 run both as 16x16x4 fp32 MFMA tiles.
+//   panel in LDS from the mode coefficients.  The matrix-core sweeps 2m to 4m
+//   run both as 16x16x4 fp32 MFMA tiles.
 // * Step = 5 sweeps over the field, each followed by a one-block finalize
 //   (deterministic fixed-order fp64 reductions of per-block partials) that
 //   runs the rank-level recurrences and writes the next sweep's coefficients:
@@ -35,7 +35,7 @@
 //        the basis Gram matrix G, hash impulse, confidence, contact
 //        oscillator, drive coefficients (every RMS in closed form)
 //     S4 drive without the hash term (written over t); sum d^2, sum d h,
-//        sum h^2 -> F4 drive energy, gain.  Fast path: F3 already has the
+//        sum h^2 -> F4 drive energy, gain.  Matrix cores: F3 already has the
 //        hash term's RMS in closed form (bin co-occurrence counts), so S4
 //        writes the full drive and sums drive^2
 //     S5 param -= lr * cast((d + c5 h) * gain), resp. cast(drive * gain)
@@ -1688,137 +1688,21 @@ __device__ __forceinline__ bool hi_block(const Geom& g, const double* __restrict
     return __syncthreads_or(hit) != 0;
 }
 
-// Panel arrays of a full tile as buffer views: one descriptor per array (the
-// panel's first element as base), the lane's column as the VGPR offset and the
-// row as a uniform SGPR offset, so the row loop needs no address arithmetic.
-// Byte sizes stay below 2^31 (the planner keeps PR * cols below 2^29).
-struct PanelBuf {
-    __amdgpu_buffer_rsrc_t r;
-    uint32_t lane;   // byte offset of the lane's column
-    uint32_t row;    // bytes per row
-};
-template <typename T>
-__device__ __forceinline__ PanelBuf panel_buf(const T* panel0, const Geom& g, int nr) {
-    PanelBuf b;
-    b.r = make_rsrc(panel0, (uint32_t)((int64_t)nr * g.cols * (int64_t)sizeof(T)));
-    b.lane = (uint32_t)(threadIdx.x * sizeof(T));
-    b.row = (uint32_t)(g.cols * sizeof(T));
-    return b;
-}
-template <typename T> __device__ __forceinline__ float ldb_lane(const PanelBuf& b, int lr);
-template <> __device__ __forceinline__ float ldb_lane<float>(const PanelBuf& b, int lr) {
-    return bload1(b.r, b.lane, (uint32_t)lr * b.row);
-}
-template <> __device__ __forceinline__ float ldb_lane<__half>(const PanelBuf& b, int lr) {
-    return to_f(__builtin_bit_cast(__half, (unsigned short)bload1u16(b.r, b.lane, (uint32_t)lr * b.row)));
-}
-template <> __device__ __forceinline__ float ldb_lane<__hip_bfloat16>(const PanelBuf& b, int lr) {
-    return to_f(__builtin_bit_cast(__hip_bfloat16, (unsigned short)bload1u16(b.r, b.lane, (uint32_t)lr * b.row)));
-}
-template <> __device__ __forceinline__ float ldb_lane<double>(const PanelBuf& b, int lr) {
-    return (float)__builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(b.r, b.lane, (uint32_t)lr * b.row, 0));
-}
-__device__ __forceinline__ uint32_t ldb_bins16(const PanelBuf& b, int lr) {
-    return bload1u16(b.r, b.lane, (uint32_t)lr * b.row);
-}
-__device__ __forceinline__ void stb_lane(const PanelBuf& b, int lr, float v) {
-    bstore1(b.r, b.lane, (uint32_t)lr * b.row, v);
-}
-
-// Rows of a full panel in batches of U: the loads of batch i+1 are issued
-// before batch i is processed (two register sets, no copies).  nr is a
-// multiple of 2U.  load(lr, x, b) loads row lr's lane values, body(lr, x, b)
-// processes them.
-// The same with a per-batch body: batch(i0, x[U], b[U]) processes rows i0..i0+U-1.
-// xa/ba hold the first batch, loaded by the caller (at the top of the kernel,
-// so that its latency overlaps the block's set-up).
-template <int U, typename Load, typename Batch>
-__device__ __forceinline__ void pipelined_batches(int nr, Load&& load, Batch&& batch, float (&xa)[U],
-                                                  uint32_t (&ba)[U]) {
-    float xb[U];
-    uint32_t bb[U];
-    for (int i0 = 0; i0 < nr; i0 += 2 * U) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) load(i0 + U + u, xb[u], bb[u]);
-        batch(i0, xa, ba);
-        if (i0 + 2 * U < nr) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) load(i0 + 2 * U + u, xa[u], ba[u]);
-        }
-        batch(i0 + U, xb, bb);
-    }
-}
-template <int U, typename Load, typename Body>
-__device__ __forceinline__ void pipelined_rows(int nr, Load&& load, Body&& body, float (&xa)[U], uint32_t (&ba)[U]) {
-    pipelined_batches<U>(
-        nr, load,
-        [&](int i0, const float* x, const uint32_t* b) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) body(i0 + u, x[u], b[u]);
-        },
-        xa, ba);
-}
-
-// Sums of 8 per-lane values (rows i0..i0+7 of the lane's column) over the 16
-// lanes of each DPP row: lane l returns row (l & 7)'s partial (lanes l and
-// l ^ 8 hold the same sum).  Lanes pair xor 1, 2, 4 while the values halve
-// (each lane keeps the rows of its own bit and receives them from its
-// partner), then xor 8: 25 instructions instead of 8 full wave reductions.
-// DPP row_ror:n reads lane (l - n) mod 16, so xor 4 is ror 4 for lanes with
-// bit 2 set and ror 12 for the others.
-template <int CTRL> __device__ __forceinline__ float dpp_mov(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
-}
-__device__ __forceinline__ float rows8_lanesum16(const float (&v)[8]) {
-    const int l = threadIdx.x & 63;
-    const bool b0 = (l & 1) != 0, b1 = (l & 2) != 0, b2 = (l & 4) != 0;
-    float w4[4], w2[2];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const float keep = b0 ? v[2 * j + 1] : v[2 * j], give = b0 ? v[2 * j] : v[2 * j + 1];
-        w4[j] = keep + dpp_mov<0xB1>(give);   // quad_perm [1,0,3,2]: xor 1
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const float keep = b1 ? w4[2 * j + 1] : w4[2 * j], give = b1 ? w4[2 * j] : w4[2 * j + 1];
-        w2[j] = keep + dpp_mov<0x4E>(give);   // quad_perm [2,3,0,1]: xor 2
-    }
-    const float keep = b2 ? w2[1] : w2[0], give = b2 ? w2[0] : w2[1];
-    const float from_below = dpp_mov<0x124>(give);   // row_ror:4  -> lane l - 4
-    const float from_above = dpp_mov<0x12C>(give);   // row_ror:12 -> lane l + 4
-    float w1 = keep + (b2 ? from_below : from_above);
-    w1 += dpp_mov<0x128>(w1);                        // row_ror:8: xor 8
-    return w1;
-}
-
-// Sweep variants: MODE 1 is the common large-matrix case with every option
-// fixed at compile time (2-D tensor, instant metric on, two hash tables of at
-// most 256 bins, no weight decay, no local sharpness); MODE 0 handles every
-// other combination with runtime flags.
+// The general sweeps' options: runtime flags, uniform over the block.  (A form
+// with the common options fixed at compile time and full tiles, as the
+// matrix-core sweeps have, spilled at the only ranks those do not take: rank
+// 24, fp32, two tables, (1024,1024) 1706 us a step against 232, (4096,4096)
+// 11550 against 1170.)
 struct SweepFlags {
     bool hash_on, axes_on, wd_on, ls_on;
     int T, bpb, binbytes;
 };
-template <int MODE>
 __device__ __forceinline__ SweepFlags sweep_flags(const Geom& g, int hash_arg, int axes_arg, const cresso_hyper& h) {
     SweepFlags f;
-    if (MODE == 1) {
-        f.hash_on = true; f.axes_on = true; f.wd_on = false; f.ls_on = false;
-        f.T = 2; f.bpb = 1; f.binbytes = 2;
-    } else {
-        f.hash_on = hash_arg != 0; f.axes_on = axes_arg != 0;
-        f.wd_on = h.weight_decay != 0.0; f.ls_on = h.local_sharpness != 0.0;
-        f.T = g.T; f.bpb = g.bpb; f.binbytes = g.binbytes;
-    }
+    f.hash_on = hash_arg != 0; f.axes_on = axes_arg != 0;
+    f.wd_on = h.weight_decay != 0.0; f.ls_on = h.local_sharpness != 0.0;
+    f.T = g.T; f.bpb = g.bpb; f.binbytes = g.binbytes;
     return f;
-}
-// whether a tensor's step can use MODE 1 (host side)
-// (MODE 1 also needs full tiles: every row of every panel and every lane's
-// column valid, and panels of a multiple of 4 SP_U rows for the row pipelines.)
-inline bool fast_mode(const Geom& g, int hash_on, int axes_on, const cresso_hyper& h) {
-    return hash_on && axes_on && g.T == 2 && g.bpb == 1 && g.binbytes == 2 && !g.one_d && h.weight_decay == 0.0 &&
-           h.local_sharpness == 0.0 && (float)fmax(h.instant_metric_power, 0.25) == 1.0f && g.rows % g.PR == 0 &&
-           g.cols % SP_NT == 0 && g.PR % (4 * SP_U) == 0;
 }
 // tables the matrix-core sweeps take: 2 or 4 tables of one-byte bins, packed
 __host__ __device__ inline bool mtables(const Geom& g) {
@@ -1853,7 +1737,7 @@ inline bool medge_mode(const Geom& g, const cresso_hyper& h) {
 // ---------------------------------------------------------------------------
 // S2: density field
 // ---------------------------------------------------------------------------
-template <int RM, int KC, typename PT, typename GT, int MODE>
+template <int RM, int KC, typename PT, typename GT>
 __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep2_kernel(
     Geom g, const GT* __restrict__ grad, const PT* __restrict__ param, const float* __restrict__ rowtab,
     const float* __restrict__ coltab, const ModeMeta* __restrict__ meta, const unsigned char* __restrict__ bins,
@@ -1869,36 +1753,18 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep2_kernel(
     constexpr int RW = 2 * RM;
     extern __shared__ __align__(16) unsigned char dyn[];
     __shared__ float red[4 * NV2];
-    const SweepFlags F = sweep_flags<MODE>(g, hash_arg, axes_arg, h);
+    const SweepFlags F = sweep_flags(g, hash_arg, axes_arg, h);
     const Tile t = tile_of(g);
     const int B = g.B;
     const int TB = F.T * B;
     const int nr = (int)(t.r1 - t.r0);
     const int64_t base = panel_base(g, t);
     const GT* __restrict__ gb = grad + base;
-    // MODE 1: the first batch's loads go out before the set-up below
-    PanelBuf gbv, bnv;
-    float x0[SP_U];
-    uint32_t b0[SP_U];
-    if constexpr (MODE == 1) {
-        gbv = panel_buf(gb, g, nr);
-        bnv = panel_buf(reinterpret_cast<const uint16_t*>(bins) + base, g, nr);
-#pragma unroll
-        for (int u = 0; u < SP_U; ++u) {
-            x0[u] = ldb_lane<GT>(gbv, u);
-            b0[u] = ldb_bins16(bnv, u);
-        }
-    }
-    // LDS: histogram [T][B] u64 (low words; MODE 1: [T][B][SP_NHIST] copies) |
-    // row-sum partials [16][PR] (MODE 0: [4 waves][PR]; MODE 1: [4 waves][4
-    // DPP rows][PR]) | MODE 1 row factors [PR][RW]
+    // LDS: histogram [T][B] u64 (low words) | row-sum partials [4 waves][PR]
     unsigned long long* s_hist = reinterpret_cast<unsigned long long*>(dyn);
     float* s_wrow = reinterpret_cast<float*>(dyn + sizeof(unsigned long long) * SP_NHIST * (size_t)TB);
-    constexpr int NH = MODE == 1 ? SP_NHIST : 1;   // histogram copies in use
-    float* s_ar = s_wrow + 16 * g.PR;
     if (F.hash_on)
-        for (int i = threadIdx.x; i < NH * TB; i += SP_NT) s_hist[i] = 0ull;
-    if (MODE == 1) stage_rows<RM>(g, rowtab, t.r0, nr, s_ar);
+        for (int i = threadIdx.x; i < TB; i += SP_NT) s_hist[i] = 0ull;
     __syncthreads();
     const PT* __restrict__ pb = param + base;
     const float* __restrict__ rt = rowtab + t.r0 * g.RW;
@@ -1919,48 +1785,6 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep2_kernel(
     float aL = 0.f, aD = 0.f;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     // Sums of log(1 + ds) are kept in log2 units (fin2 scales them by ln 2).
-    if constexpr (MODE == 1) {
-        // full tile: rel >= eps and instant-metric power 1, so the density is rel
-        constexpr int U = SP_U;
-        const int hc = threadIdx.x & (SP_NHIST - 1);
-        pipelined_batches<U>(
-            nr,
-            [&](int lr, float& x, uint32_t& b) {
-                x = ldb_lane<GT>(gbv, lr);
-                b = ldb_bins16(bnv, lr);
-            },
-            [&](int i0, const float* x, const uint32_t* bv) {
-#pragma unroll
-                for (int h8 = 0; h8 < U / 8; ++h8) {
-                    float dn[8];
-#pragma unroll
-                    for (int v8 = 0; v8 < 8; ++v8) {
-                        const int u = 8 * h8 + v8;
-                        const float rel = rel_full(x[u], inv_s, eps);
-                        const float ds = fexp2(pw * flog2(rel));
-                        const float L = flog2(1.0f + ds);
-                        dn[v8] = rel;
-                        aL += L;
-                        aD += rel;
-                        const float* __restrict__ ar = s_ar + (i0 + u) * RW;
-#pragma unroll
-                        for (int q = 0; q < RW; ++q) Z[q] = fmaf(ar[q], L, Z[q]);
-                        const unsigned long long v = to_fixed_u(fminf(ds * hs, yk));   // high words: hi_pass
-                        atomicAdd(&s_hist[bin_of(bv[u], 0, 1) * NH + hc], v);
-                        atomicAdd(&s_hist[(B + bin_of(bv[u], 1, 1)) * NH + hc], v);
-#pragma unroll
-                        for (int q = 0; q < RW; ++q) pin1(Z[q]);
-                        pin1(aL);
-                        pin1(aD);
-                        pin1(dn[v8]);
-                        elem_fence();
-                    }
-                    const float rs = rows8_lanesum16(dn);
-                    if ((lane & 8) == 0) s_wrow[((wave << 2) + (lane >> 4)) * g.PR + i0 + 8 * h8 + (lane & 7)] = rs;
-                }
-            },
-            x0, b0);
-    } else
     for (int i0 = 0; i0 < nr; i0 += SP_U) {
         float gv[SP_U], pv[SP_U];
         uint64_t bv[SP_U];
@@ -2005,7 +1829,7 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep2_kernel(
                 const float ws = wave_total(dens);
                 if (lane == 63) s_wrow[wave * g.PR + lr] = ws;
             }
-            if (MODE == 0) elem_fence();
+            elem_fence();
         }
     }
     if (F.hash_on && hi_on && hi_block(g, part1, base, nr, SP_NT, inv_s, eps, pw, kmf) && t.colok) {
@@ -2013,24 +1837,15 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep2_kernel(
         const unsigned long long lo_k = to_fixed_u(yk);   // what the loop added for y >= 2^k
         for (int lr = 0; lr < nr; ++lr) {
             const uint32_t o = panel_off(g, lr);
-            float ds;
-            if constexpr (MODE == 1) {
-                ds = fexp2(pw * flog2(rel_full(to_f(gb[o]), inv_s, eps)));
-            } else {
-                const float pvv = F.wd_on ? to_f(pb[o]) : 0.f;
-                ds = fpow(rel_gen(force_of(to_f(gb[o]), pvv, sg, wd, F.wd_on), inv_s, eps), pw);
-            }
+            const float pvv = F.wd_on ? to_f(pb[o]) : 0.f;
+            const float ds = fpow(rel_gen(force_of(to_f(gb[o]), pvv, sg, wd, F.wd_on), inv_s, eps), pw);
             if (ds * hs >= yk) {
-                // MODE 1: two tables of one-byte bins, histogram copy threadIdx.x mod SP_NHIST
-                const uint64_t bb = MODE == 1 ? (uint64_t)(reinterpret_cast<const uint16_t*>(bins) + base)[o]
-                                              : load_bins_at(bins, base, o, F.binbytes);
-                const int nt = MODE == 1 ? 2 : F.T, bpb = MODE == 1 ? 1 : F.bpb;
-                const int hcm = MODE == 1 ? (int)(threadIdx.x & (SP_NHIST - 1)) : 0;
+                const uint64_t bb = load_bins_at(bins, base, o, F.binbytes);
                 const HiSplit sp = hi_split(ds, hq, yk, lo_k);
-                for (int tt = 0; tt < nt; ++tt) {
-                    const int bin = tt * B + bin_of(bb, tt, bpb);
+                for (int tt = 0; tt < F.T; ++tt) {
+                    const int bin = tt * B + bin_of(bb, tt, F.bpb);
                     atomicAdd(&hist[(size_t)g.hcopies * TB + bin], sp.hi);   // the high-word table
-                    atomicAdd(&s_hist[bin * NH + hcm], sp.lo);
+                    atomicAdd(&s_hist[bin], sp.lo);
                 }
             }
         }
@@ -2040,16 +1855,14 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep2_kernel(
         // axis density sums: one fixed-point atomic per row of this slab and per column of this panel
         for (int lr = threadIdx.x; lr < nr; lr += SP_NT) {
             float s = 0.f;
-            for (int w = 0; w < (MODE == 1 ? 16 : SP_NT / 64); ++w) s += s_wrow[w * g.PR + lr];
+            for (int w = 0; w < SP_NT / 64; ++w) s += s_wrow[w * g.PR + lr];
             atomicAdd(&rowfx[t.r0 + lr], to_fixed_u(s * (float)g.hs_row));
         }
         if (t.colok) atomicAdd(&colfx[t.col], to_fixed_u(aD * (float)g.hs_col));
     }
     if (F.hash_on)
         for (int i = threadIdx.x; i < TB; i += SP_NT) {
-            unsigned long long v = 0ull;
-#pragma unroll
-            for (int c = 0; c < NH; ++c) v += s_hist[i * NH + c];
+            const unsigned long long v = s_hist[i];
             if (v) atomicAdd(&hist[i], v);
         }
     float b[KC];
@@ -2768,7 +2581,7 @@ __global__ __launch_bounds__(SP_MARG_NT) void marg_fac_kernel(
 // ---------------------------------------------------------------------------
 // S3: tangent force, prediction error, port projection / histograms, t projection
 // ---------------------------------------------------------------------------
-template <int RM, int KC, typename PT, typename GT, int MODE>
+template <int RM, int KC, typename PT, typename GT>
 __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep3_kernel(
     Geom g, const GT* __restrict__ grad, const PT* __restrict__ param, const float* __restrict__ rowtab,
     const float* __restrict__ coltab, const ModeMeta* __restrict__ meta, const unsigned char* __restrict__ bins,
@@ -2784,7 +2597,7 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep3_kernel(
     constexpr int RW = 2 * RM;
     extern __shared__ __align__(16) unsigned char dyn[];
     __shared__ float red[4 * NV3];
-    const SweepFlags F = sweep_flags<MODE>(g, hash_arg, 1, h);
+    const SweepFlags F = sweep_flags(g, hash_arg, 1, h);
     const Tile t = tile_of(g);
     const int B = g.B;
     const int TB = F.T * B;
@@ -2792,35 +2605,18 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep3_kernel(
     const int64_t base = panel_base(g, t);
     const GT* __restrict__ gb = grad + base;
     float* __restrict__ tb = tbuf + base;
-    // MODE 1: the first batch's loads go out before the set-up below
-    PanelBuf gbv, bnv, tbv;
-    float x0[SP_U];
-    uint32_t b0[SP_U];
-    if constexpr (MODE == 1) {
-        gbv = panel_buf(gb, g, nr);
-        bnv = panel_buf(reinterpret_cast<const uint16_t*>(bins) + base, g, nr);
-        tbv = panel_buf(tb, g, nr);
-#pragma unroll
-        for (int u = 0; u < SP_U; ++u) {
-            x0[u] = ldb_lane<GT>(gbv, u);
-            b0[u] = ldb_bins16(bnv, u);
-        }
-    }
     // LDS: histogram [T][B] u64 | log hash metric [T][B] | row metric factor [PR]
     //      | row reconstruction coefficients [PR][2][KP] (16-byte aligned) | row factors [PR][RW]
     unsigned long long* s_hist = reinterpret_cast<unsigned long long*>(dyn);
     float* s_lt = reinterpret_cast<float*>(dyn + sizeof(unsigned long long) * SP_NHIST * (size_t)TB);
-    constexpr int NH = MODE == 1 ? SP_NHIST : 1;   // histogram copies in use
-    const int hc = MODE == 1 ? (int)(threadIdx.x & (SP_NHIST - 1)) : 0;
     float* s_rf = s_lt + TB;
     const float eps = (float)h.eps;
     const float kappa = ctrl->kappa, gden = ctrl->gden;
-    const bool inst_on = MODE == 1 ? true : kappa != 0.0f;
+    const bool inst_on = kappa != 0.0f;
     if (F.hash_on)
         for (int i = threadIdx.x; i < TB; i += SP_NT) {
             s_lt[i] = lt[i];
-#pragma unroll
-            for (int c = 0; c < NH; ++c) s_hist[i * NH + c] = 0ull;
+            s_hist[i] = 0ull;
         }
     for (int lr = threadIdx.x; lr < nr; lr += SP_NT)
         s_rf[lr] = (inst_on && !g.one_d) ? marg_factor(rowfx[t.r0 + lr], 1.0 / (g.hs_row * (double)g.cols), gden, kappa, eps) : 1.0f;
@@ -2864,7 +2660,6 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep3_kernel(
     for (int q = 0; q < RW; ++q) ZT[q] = 0.f;
     float m_ee = 0.f, m_t = 0.f, m_tt = 0.f, m_rr = 0.f, m_bb = 0.f, m_oo = 0.f, m_rb = 0.f, m_ro = 0.f,
           m_bo = 0.f, m_tr = 0.f, m_tb = 0.f, m_to = 0.f;
-    // MODE 1 panel views (full tile)
     // one row of the lane's column: f -> t (stored), moments, projection, histogram
     auto row = [&](int lr, float gval, float pval, uint64_t bval) {
                 float f = sg * gval;
@@ -2884,7 +2679,7 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep3_kernel(
                 }
                 if (inst_on) {
                     float I;
-                    if (MODE == 0 && g.one_d) {
+                    if (g.one_d) {
                         const float rel = fmaxf(fminf(fabsf(f) * inv_s + eps, 1.0e4f), eps);
                         const float dens = fminf(ipw == 1.0f ? rel : fpow(rel, ipw), 1.0e6f);
                         I = fexp(kappa * flog(fmaxf(dens / gden, eps)));
@@ -2903,10 +2698,7 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep3_kernel(
                     den = den * med3f(fexp(lsum * invT), 0.08f, 12.0f);
                 }
                 const float tv = med3f(f * frcp(den + eps), -1.0e4f, 1.0e4f);
-                if (MODE == 1)
-                    stb_lane(tbv, lr, tv);
-                else
-                    tb[panel_off(g, lr)] = tv;
+                tb[panel_off(g, lr)] = tv;
                 float pred = cP;
 #pragma unroll
                 for (int k = 0; k < KC; ++k) pred = fmaf(al[KP + k], bc[k], pred);
@@ -2929,28 +2721,12 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep3_kernel(
 #pragma unroll
                     for (int tt = 0; tt < SP_MAXT; ++tt) {
                         if (tt >= F.T) break;
-                        atomicAdd(&s_hist[(tt * B + bin_of(bval, tt, F.bpb)) * NH + hc], v);
+                        atomicAdd(&s_hist[tt * B + bin_of(bval, tt, F.bpb)], v);
                     }
-                }
-                if (MODE == 1) {
-                    // this row's contributions are complete here
-#pragma unroll
-                    for (int q = 0; q < RW; ++q) pin1(ZT[q]);
-                    pin1(m_ee); pin1(m_t); pin1(m_tt); pin1(m_rr); pin1(m_bb); pin1(m_oo);
-                    pin1(m_rb); pin1(m_ro); pin1(m_bo); pin1(m_tr); pin1(m_tb); pin1(m_to);
                 }
                 elem_fence();
     };
-    if constexpr (MODE == 1) {
-        // full tile: no guards, next rows' loads in flight during these rows
-        pipelined_rows<SP_U>(
-            nr,
-            [&](int lr, float& x, uint32_t& b) {
-                x = ldb_lane<GT>(gbv, lr);
-                b = ldb_bins16(bnv, lr);
-            },
-            [&](int lr, float x, uint32_t b) { row(lr, x, 0.f, b); }, x0, b0);
-    } else if (t.colok) {
+    if (t.colok) {
         for (int i0 = 0; i0 < nr; i0 += SP_U) {
             float gv[SP_U], pv[SP_U];
             uint64_t bv[SP_U];
@@ -2976,9 +2752,7 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep3_kernel(
     __syncthreads();
     if (F.hash_on)
         for (int i = threadIdx.x; i < TB; i += SP_NT) {
-            unsigned long long v = 0ull;
-#pragma unroll
-            for (int c = 0; c < NH; ++c) v += s_hist[i * NH + c];
+            const unsigned long long v = s_hist[i];
             if (v) atomicAdd(&hist[i], v);
         }
     Partials P{red, 15 + 2 * g.R, NV3};
@@ -3785,7 +3559,7 @@ __global__ __launch_bounds__(256) void hh4_kernel(Geom g, const unsigned long lo
 // ---------------------------------------------------------------------------
 // S4: drive without the hash term, written over t; sums for the drive energy
 // ---------------------------------------------------------------------------
-template <int RM, int KC, int MODE>
+template <int RM, int KC>
 __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep4_kernel(
     Geom g, const float* __restrict__ rowtab, const float* __restrict__ coltab, const ModeMeta* __restrict__ meta,
     const unsigned char* __restrict__ bins, const Ctrl* __restrict__ ctrl, const float* __restrict__ imp_tab,
@@ -3793,7 +3567,7 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep4_kernel(
     ctrl = lane_at(ctrl, L); imp_tab = lane_at(imp_tab, L); tbuf = lane_at(tbuf, L); part = lane_at(part, L);
     extern __shared__ __align__(16) unsigned char dyn[];
     __shared__ float red[4 * NV4];
-    const SweepFlags F = sweep_flags<MODE>(g, hash_arg, 1, h);
+    const SweepFlags F = sweep_flags(g, hash_arg, 1, h);
     const Tile t = tile_of(g);
     const int B = g.B;
     const int TB = F.T * B;
@@ -3828,11 +3602,6 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep4_kernel(
     const float k2n = -2.8853900817779268f * ctrl->nscale;    // tanh(err' nscale)
     const float invT = 1.0f / (float)F.T;
     float a_dd = 0.f, a_dh = 0.f, a_hh = 0.f;
-    PanelBuf tbv, bnv;
-    if (MODE == 1) {
-        tbv = panel_buf(tb, g, nr);
-        bnv = panel_buf(reinterpret_cast<const uint16_t*>(bins) + base, g, nr);
-    }
     // one row of the lane's column: t -> drive without the hash term (stored over t)
     auto row = [&](int lr, float tv, uint64_t bval) {
         const float* __restrict__ al = s_al + lr * (2 * KP);
@@ -3848,10 +3617,7 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep4_kernel(
         const Shape3A z = shape3a(at, k2, iclip, clip2, eps);
         const float core = xorsign(fmaf(k_t, at, fmaf(k_root, z.root, fmaf(k_ths, z.th, k_rat * z.rat))), tv);
         const float d = fmaf(k_nov, nov, core + mixed);
-        if (MODE == 1)
-            stb_lane(tbv, lr, d);
-        else
-            tb[panel_off(g, lr)] = d;
+        tb[panel_off(g, lr)] = d;
         a_dd = fmaf(d, d, a_dd);
         if (F.hash_on) {
             float hp = 0.f;
@@ -3864,27 +3630,9 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep4_kernel(
             a_dh = fmaf(d, hp, a_dh);
             a_hh = fmaf(hp, hp, a_hh);
         }
-        if (MODE == 1) {
-            pin1(a_dd); pin1(a_dh); pin1(a_hh);
-        }
         elem_fence();
     };
-    if constexpr (MODE == 1) {
-        float x0[SP_U];
-        uint32_t b0[SP_U];
-#pragma unroll
-        for (int u = 0; u < SP_U; ++u) {
-            x0[u] = ldb_lane<float>(tbv, u);
-            b0[u] = ldb_bins16(bnv, u);
-        }
-        pipelined_rows<SP_U>(
-            nr,
-            [&](int lr, float& x, uint32_t& b) {
-                x = ldb_lane<float>(tbv, lr);
-                b = ldb_bins16(bnv, lr);
-            },
-            [&](int lr, float x, uint32_t b) { row(lr, x, b); }, x0, b0);
-    } else if (t.colok) {
+    if (t.colok) {
         for (int i0 = 0; i0 < nr; i0 += SP_U) {
             float tvs[SP_U];
             uint64_t bv[SP_U];
@@ -3915,7 +3663,7 @@ __global__ __launch_bounds__(SP_NT, RM >= 16 ? 2 : 4) void sweep4_kernel(
 
 
 // ---------------------------------------------------------------------------
-// S4 on the matrix cores (MODE 1 tiles, TT = 2 or 4 tables of one-byte bins).
+// S4 on the matrix cores (TT = 2 or 4 tables of one-byte bins).
 // Each wave owns 64 columns of the panel as 4 x 4 tiles of 16 x 16 elements.
 // A reconstruction of a tile is KCH MFMAs (v_mfma_f32_16x16x4f32, the K = KC
 // carriers in chunks of 4):
@@ -4573,11 +4321,6 @@ int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, 
     v4 = v4 && pv4;
     // the matrix-core sweeps (two or four tables; ranks up to 16: two 16-row projection tiles)
     constexpr bool MX = RM <= 16;
-    // MODE 1 tiles of the general sweeps (two tables): ranks above 16, whose
-    // full tiles the matrix-core sweeps do not take.  (Not instantiated below:
-    // more kernels in the code object slow every launch a little, a lone
-    // (2048,2048) step 93.8 -> 94.7 us with them.)
-    const bool fast = !MX && fast_mode(g, hash_on, axes_on, h);
     const bool mf = MX && mfast_mode(g, hash_on, axes_on, h);
     const bool edge = medge_mode(g, h);
     // with weight decay they read the force that sweep 1 leaves in tbuf
@@ -4630,12 +4373,8 @@ int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, 
                                    blk, l2, s, g, src, fout, rowtab, coltab, meta, bins, ctrl, part, hd2 ? hist : hpart,
                                    hhi, rowfx, colfx, part1, st.force_rms, step, L, h, one_round2, hd2);
             });
-    } else if (fast) {
-        if constexpr (!MX)
-            hipLaunchKernelGGL((sweep2_kernel<RM, KC, PT, GT, 1>), grid, blk, l2, s, g, grad, param, rowtab, coltab, meta, bins,
-                           ctrl, part, hist, rowfx, colfx, hash_on, axes_on, part1, st.force_rms, step, L, h);
     } else {
-        hipLaunchKernelGGL((sweep2_kernel<RM, KC, PT, GT, 0>), grid, blk, l2, s, g, grad, param, rowtab, coltab, meta, bins,
+        hipLaunchKernelGGL((sweep2_kernel<RM, KC, PT, GT>), grid, blk, l2, s, g, grad, param, rowtab, coltab, meta, bins,
                            ctrl, part, hist, rowfx, colfx, hash_on, axes_on, part1, st.force_rms, step, L, h);
     }
     hipLaunchKernelGGL(part_reduce_kernel, dim3(NV2 + (m2 && !hd2 ? pr_hist_blocks(g.T * g.B, g.nblk) : 0), ny), dim3(256), 0, s,
@@ -4657,12 +4396,8 @@ int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, 
                                    blk, lds_sweep3m<KC>(g, 2 * RM), s, g, src, fout ? 1 : 0, rowtab, coltab, meta, bins, ctrl, lt,
                                    rowfx, colfx, colfac, tbuf, part, hd3 ? hist : hpart, L, h, one_round3, hd3);
             });
-    } else if (fast) {
-        if constexpr (!MX)
-            hipLaunchKernelGGL((sweep3_kernel<RM, KC, PT, GT, 1>), grid, blk, l3, s, g, grad, param, rowtab, coltab, meta, bins,
-                           ctrl, lt, rowfx, colfx, colfac, tbuf, part, hist, hash_on, L, h);
     } else {
-        hipLaunchKernelGGL((sweep3_kernel<RM, KC, PT, GT, 0>), grid, blk, l3, s, g, grad, param, rowtab, coltab, meta, bins,
+        hipLaunchKernelGGL((sweep3_kernel<RM, KC, PT, GT>), grid, blk, l3, s, g, grad, param, rowtab, coltab, meta, bins,
                            ctrl, lt, rowfx, colfx, colfac, tbuf, part, hist, hash_on, L, h);
     }
     // the matrix-core sweep 4 writes the full drive: the hash term's RMS comes
@@ -4679,13 +4414,8 @@ int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, 
     // sweep 4m runs too, in place, and sweep 5q applies it)
     const bool q4 = m3 && c5c != 0 && !edge;
     if (!MX || c5c == 0) {
-        if (fast) {
-            if constexpr (!MX)
-                hipLaunchKernelGGL((sweep4_kernel<RM, KC, 1>), grid, blk, l4, s, g, rowtab, coltab, meta, bins, ctrl, imp, tbuf,
-                               part, hash_on, echo_on, L, h);
-        } else
-            hipLaunchKernelGGL((sweep4_kernel<RM, KC, 0>), grid, blk, l4, s, g, rowtab, coltab, meta, bins, ctrl, imp, tbuf,
-                               part, hash_on, echo_on, L, h);
+        hipLaunchKernelGGL((sweep4_kernel<RM, KC>), grid, blk, l4, s, g, rowtab, coltab, meta, bins, ctrl, imp, tbuf,
+                           part, hash_on, echo_on, L, h);
     } else if constexpr (MX) {
         auto sweep4 = [&](auto tt, auto q, auto e) {
             hipLaunchKernelGGL((sweep4m_kernel<RM, KC, decltype(tt)::value, decltype(q)::value, decltype(e)::value>), grid,
