@@ -143,6 +143,8 @@ def _declare(lib: ctypes.CDLL) -> None:
                                                  c.c_size_t, c.POINTER(Hyper), c.c_void_p]
     lib.cresso_spectral_step_noalloc.restype = c.c_int32
     lib.cresso_spectral_step_noalloc.argtypes = [c.c_void_p, c.POINTER(SpectralDesc), c.POINTER(Hyper), c.c_void_p]
+    lib.cresso_spectral_plan_panel_rows.restype = c.c_int32
+    lib.cresso_spectral_plan_panel_rows.argtypes = [c.c_void_p, c.c_int32]
     lib.cresso_spectral_step_units.restype = c.c_int32
     lib.cresso_spectral_step_units.argtypes = [c.POINTER(SpectralUnit), c.c_int32, c.POINTER(Hyper),
                                                c.POINTER(c.c_void_p), c.c_int32]

@@ -4216,7 +4216,8 @@ __global__ __launch_bounds__(SP_NT) void sweep5q_kernel(Geom g, PT* __restrict__
 }  // namespace cresso
 
 struct cresso_spectral_plan {
-    cresso::Geom g;
+    cresso::Geom g;             // its panels: the matrix-core sweeps' where the plan has them, else the general sweeps'
+    int32_t general_rows;       // panel rows of the general sweeps
     cresso::Offs o;
     std::vector<cresso::AxisConst> axc;
     std::vector<cresso::ModeMeta> meta;
@@ -4263,6 +4264,12 @@ size_t lds_sweep4(const Geom& g, int kp, int rw) {
 constexpr size_t SP_LDS_MAX = 64 * 1024;
 constexpr size_t SP_LDS_MAX_M = 96 * 1024;   // dynamic LDS of a matrix-core sweep (gfx950: 160 KB per workgroup)
 
+inline void set_panels(Geom& g, int64_t rows) {
+    g.PR = (int32_t)rows;
+    g.panels = (int32_t)((g.rows + rows - 1) / rows);
+    g.nblk = g.slabs * g.panels;
+}
+
 // One step of `count` tensors of plan P: hd[0..count) are their descriptors
 // on the host; for count > 1, dv is the same array in device memory and each
 // tensor's per-step scratch follows the previous one's at a stride of ls
@@ -4271,7 +4278,7 @@ constexpr size_t SP_LDS_MAX_M = 96 * 1024;   // dynamic LDS of a matrix-core swe
 template <int RM, int KC, typename PT, typename GT>
 int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, int count,
                  const cresso_spectral_desc* dv, size_t ls, void* ws, const cresso_hyper& h, hipStream_t s) {
-    const Geom& g = P.g;
+    Geom g = P.g;
     const Offs& o = P.o;
     const cresso_spectral_desc& d = hd[0];
     const SpecState st = spec_state(d);
@@ -4307,6 +4314,10 @@ int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, 
     double* part1 = at<double>(ws, o.part1);
     const int step = d.step;
     const int axes_on = (hard && h.instant_metric_coupling != 0.0 && !g.one_d) ? 1 : 0;
+    // the matrix-core sweeps (two or four tables; ranks up to 16: two 16-row projection tiles)
+    constexpr bool MX = RM <= 16;
+    const bool mf = MX && mfast_mode(g, hash_on, axes_on, h);
+    if (!mf) set_panels(g, P.general_rows);
     const size_t l2 = lds_sweep2(g, 2 * RM), l3 = lds_sweep3(g, kcp<KC>(), 2 * RM), l4 = lds_sweep4(g, kcp<KC>(), 2 * RM);
     if (l2 > SP_LDS_MAX || l3 > SP_LDS_MAX || l4 > SP_LDS_MAX)
         return fail(CRESSO_E_UNSUPPORTED, "spectral route: hash_tables x hash_bins = %d needs %zu bytes of LDS per block",
@@ -4319,9 +4330,6 @@ int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, 
         v4 = v4 && ((uintptr_t)hd[i].grad % (4 * sizeof(GT))) == 0;
     }
     v4 = v4 && pv4;
-    // the matrix-core sweeps (two or four tables; ranks up to 16: two 16-row projection tiles)
-    constexpr bool MX = RM <= 16;
-    const bool mf = MX && mfast_mode(g, hash_on, axes_on, h);
     const bool edge = medge_mode(g, h);
     // with weight decay they read the force that sweep 1 leaves in tbuf
     float* fout = mf && h.weight_decay != 0.0 ? tbuf : nullptr;

@@ -157,10 +157,21 @@ int32_t plan_spectral(const int64_t* shape, int32_t ndim, const int64_t* freqs, 
         return fail(CRESSO_E_UNSUPPORTED, "spectral route: column carrier table too large (%d x %lld)", g.K, (long long)g.cols);
     g.KA = 2 * P.rmax + 2;
     g.RW = 2 * P.rmax;
-    // tiling: 256 columns per block, PR rows per block
+    // tiling: 256 columns per block, PR rows per block.  The general sweeps
+    // take panels of a multiple of SP_U rows with at most 1024 blocks, one
+    // round at four waves a SIMD (a few blocks more wait for a round of their
+    // own: three tables, (6000,1000), 210 us with 1044 blocks of 23 rows, 190
+    // with 1000 of 24).  Ranks above 16 (two waves a SIMD: 512 blocks) take 32
+    // rows from there on, the most whose row coefficients (2 * 68 + 64 floats
+    // a row) fit in LDS.  us a step, fp32, with panels of 16 / 32 rows: rank
+    // 24, two tables, (1024,1024) 233 / 291, (3072,768) 387 / 348, (2048,2048)
+    // 486 / 367, (2500,1100) 474 / 358; four tables, (1024,1024) 244 / 303,
+    // (3072,768) 464 / 459, (2048,2048) 629 / 470, (3072,2048) 853 / 665.
     g.slabs = (int32_t)((g.cols + SP_NT - 1) / SP_NT);
-    int64_t pr = std::max<int64_t>(16, (g.rows * g.slabs) / 1024);
-    pr = std::min<int64_t>(std::min<int64_t>(pr, 64), g.rows);
+    const int64_t area = g.rows * g.slabs;
+    const int64_t round = SP_U * ((area + 1024 * SP_U - 1) / (1024 * SP_U));
+    int64_t pr = rank > 16 ? (area <= 16 * 512 ? 16 : 32) : std::min<int64_t>(std::max<int64_t>(16, round), 64);
+    pr = std::min<int64_t>(pr, g.rows);
     // The matrix-core sweeps take panels of 16, 32 or 64 rows (a last panel of
     // fewer rows overlaps the one before it).  Fewer rows make more, shorter
     // blocks: each repeats the set-up of its tables, and a lone tensor fills
@@ -173,22 +184,30 @@ int32_t plan_spectral(const int64_t* shape, int32_t ndim, const int64_t* freqs, 
     // lose (a transformer's 88 in one group: 2.4 % of its layers' time).
     // (Four tables skip the 32: the partial histograms of twice the blocks
     // would take plans past the no-alloc entry's workspace limit.)
+    P.general_rows = (int32_t)pr;
     if (mtables(g) && !g.one_d && rank <= 16 && g.rows >= 16 && g.cols >= SP_WCOLS) {
-        const int64_t area = g.rows * g.slabs;
-        pr = area <= 16 * 640 ? 16 : (area < 64 * 256 && g.T == 2) ? 32 : 64;
-        while (pr > g.rows) pr /= 2;
+        int64_t mr = area <= 16 * 640 ? 16 : (area < 64 * 256 && g.T == 2) ? 32 : 64;
+        while (mr > g.rows) mr /= 2;
+        // A step of such a plan that runs the general sweeps (local sharpness,
+        // an instant-metric power, no hard channel) keeps the taller panels
+        // where they tile the rows: a network's matrices, which step in
+        // batches (16 x (2048,2048), rank 8, local sharpness: 1175 us with 64
+        // rows, 1373 with 16; alone 237 and 166).  Ragged ones (embedding
+        // tables, heads) step alone: rank 8, (2500,1100) 165 us with 64 rows,
+        // 154 with 16, (6000,1000) 259 with 64, 193 with 24; rank 16, four
+        // tables, 292 / 256 and 326 / 303.
+        if (g.rows % 32 == 0 || area <= 16 * 640) P.general_rows = (int32_t)mr;
+        pr = mr;
     }
-    // ranks above 16 run the general sweeps, whose per-block LDS (row
-    // coefficients of 2 * 68 + 64 floats per panel row) fits with 32-row panels
-    if (rank > 16) pr = std::min<int64_t>(pr, 32);
     // 32-bit element offsets inside a panel: PR * cols < 2^29
     if (g.cols >= ((int64_t)1 << 29))
         return fail(CRESSO_E_UNSUPPORTED, "spectral route: %lld elements per row exceed this build's panel limit",
                     (long long)g.cols);
-    pr = std::min<int64_t>(pr, ((int64_t)1 << 29) / g.cols);
-    g.PR = (int32_t)std::max<int64_t>(1, pr);
-    g.panels = (int32_t)((g.rows + g.PR - 1) / g.PR);
-    g.nblk = g.slabs * g.panels;
+    const int64_t most = std::max<int64_t>(1, ((int64_t)1 << 29) / g.cols);
+    P.general_rows = (int32_t)std::min<int64_t>(P.general_rows, most);
+    Geom gg = g;
+    set_panels(gg, P.general_rows);
+    set_panels(g, std::min<int64_t>(pr, most));
     // the matrix-core sweeps' histograms: atomic merges (part_reduce's row
     // groups, or every block of a multi-round launch) spread over copies
     g.hcopies = mtables(g) ? SP_HCOPIES : 1;
@@ -220,7 +239,7 @@ int32_t plan_spectral(const int64_t* shape, int32_t ndim, const int64_t* freqs, 
     o.cooc = take(cooc_closed(g) ? sizeof(unsigned long long) * (size_t)cooc_pairs(g) * g.B * g.B : 0);
     o.bins = take((size_t)g.binbytes * (size_t)g.n);
     o.tbuf = take(sizeof(float) * (size_t)g.n);
-    o.part = take(sizeof(double) * (size_t)NVMAX * std::max(g.nblk, g.nblk1));
+    o.part = take(sizeof(double) * (size_t)NVMAX * std::max(std::max(g.nblk, gg.nblk), g.nblk1));
     o.part1 = take(sizeof(double) * 2 * (size_t)g.nblk1);   // sweep 1's sums and maxima, read by every block of sweep 2
     o.sums = take(sizeof(double) * (size_t)NVMAX);
     o.hist = take(sizeof(unsigned long long) * (size_t)hist_words(g));   // low-word copies, then the high words
@@ -521,6 +540,10 @@ extern "C" int32_t cresso_spectral_step_batched(const cresso_spectral_plan* P, c
         hipLaunchKernelGGL(put_descs_kernel, dim3(1), dim3(256), 0, s, c, n, at<unsigned char>(ws, P->o.desc + i0 * ls), ls);
     }
     return fn(*P, descs, count, at<cresso_spectral_desc>(ws, P->o.desc), ls, ws, *hyper, s);
+}
+
+extern "C" int32_t cresso_spectral_plan_panel_rows(const cresso_spectral_plan* P, int32_t general) {
+    return !P ? 0 : (general ? P->general_rows : P->g.PR);
 }
 
 extern "C" int32_t cresso_spectral_step_units(const cresso_spectral_unit* units, int32_t n, const cresso_hyper* hyper,

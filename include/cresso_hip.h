@@ -214,6 +214,10 @@ int32_t cresso_spectral_batched_workspace_init(const cresso_spectral_plan* plan,
 int32_t cresso_spectral_step_batched(const cresso_spectral_plan* plan, const cresso_spectral_desc* descs, int32_t count,
                                      void* workspace, size_t workspace_bytes, const cresso_hyper* hyper, void* stream);
 
+/* Rows of the panels that a step's sweeps are cut into: of the matrix-core
+ * sweeps where the plan has them (general != 0: of the general sweeps). */
+int32_t cresso_spectral_plan_panel_rows(const cresso_spectral_plan* plan, int32_t general);
+
 /* Several steps in one call: unit i steps its `count` descriptors (batched != 0:
  * cresso_spectral_step_batched on a batched workspace; else count is 1 and
  * cresso_spectral_step runs) on streams[lane]. */

@@ -39,7 +39,7 @@ def announce(msg: str) -> None:
     print(f"[gpu-case] {msg}", flush=True)
 
 
-def run_pair(shapes, dtype, kwargs, steps, seed=0, grad_std=1e-2, param_std=0.05, grad_scales=None):
+def run_pair(shapes, dtype, kwargs, steps, seed=0, grad_std=1e-2, param_std=0.05, grad_scales=None, hash_accum="native"):
     """-> (hip params, hip optimizer, oracle params, oracle optimizer) after `steps` steps."""
     import cresso_amd
 
@@ -55,7 +55,7 @@ def run_pair(shapes, dtype, kwargs, steps, seed=0, grad_std=1e-2, param_std=0.05
     hp = [torch.nn.Parameter(p.clone().cuda()) for p in p0]
     op = [p.clone() for p in p0]
     hopt = cresso_amd.CRESSO5(hp, cuda_ops="required", **kwargs)
-    oopt = OracleCRESSO5(op, **kwargs)
+    oopt = OracleCRESSO5(op, hash_accum=hash_accum, **kwargs)
     for k, gs in enumerate(grads):
         if k == len(grads) - 1:
             torch.cuda.synchronize()

@@ -417,6 +417,46 @@ def test_steady_step_holds_no_dropped_workspace():
     assert all(r() is None for r in refs)
 
 
+def _plan(shape, rank, bins, tables):
+    """(panel rows, panel rows of the general sweeps, workspace bytes) of an fp32 plan (no GPU needed)."""
+    import ctypes
+
+    from cresso_amd.modes import freqs_tensor
+
+    lib = _native.load()
+    fr = freqs_tensor(rank, len(shape), 5, "cpu").reshape(-1).tolist()
+    plan = lib.cresso_spectral_plan_create_ex((ctypes.c_int64 * 8)(*shape), len(shape), (ctypes.c_int64 * len(fr))(*fr),
+                                              rank, bins, tables, _native.F32)
+    assert plan
+    plan = ctypes.c_void_p(plan)
+    got = (int(lib.cresso_spectral_plan_panel_rows(plan, 0)), int(lib.cresso_spectral_plan_panel_rows(plan, 1)),
+           int(lib.cresso_spectral_workspace_bytes(plan)))
+    lib.cresso_spectral_plan_destroy(plan)
+    return got
+
+
+PANELS = [
+    # shape, rank, bins, tables, matrix-core (or only) sweeps' rows, general sweeps' rows
+    # ranks above 16: 32 rows from 512 blocks on
+    ((512, 512), 24, 64, 2, 16, 16), ((1024, 2048), 24, 64, 2, 16, 16), ((3072, 768), 24, 64, 2, 32, 32),
+    ((2048, 2048), 24, 256, 4, 32, 32), ((2500, 1100), 20, 64, 2, 32, 32), ((8192, 4096), 32, 64, 2, 32, 32),
+    # matrix-core plans: 16, 32 and 64 rows; the general sweeps as tall where
+    # the rows tile by 32, else multiples of 8 with at most 1024 blocks
+    ((512, 512), 8, 64, 2, 16, 16), ((10, 500), 8, 64, 2, 10, 10), ((1536, 2048), 8, 64, 2, 32, 32),
+    ((2500, 1100), 8, 64, 2, 32, 16), ((2048, 2048), 8, 64, 2, 64, 64), ((6000, 1000), 8, 64, 2, 64, 24),
+    ((9000, 700), 8, 64, 2, 64, 32), ((2500, 1100), 16, 256, 4, 64, 16), ((50257, 768), 8, 64, 2, 64, 64),
+    # one or three tables, two-byte bins, too few columns: the general sweeps only
+    ((2048, 2048), 8, 64, 3, 16, 16), ((2048, 2048), 8, 512, 2, 16, 16), ((30000, 60), 8, 64, 2, 32, 32), ((6000, 1000), 8, 64, 3, 24, 24),
+]
+
+
+@pytest.mark.parametrize("shape,rank,bins,tables,rows,general", PANELS, ids=[f"{c[0]}_r{c[1]}_t{c[3]}" for c in PANELS])
+def test_spectral_plan_panels(shape, rank, bins, tables, rows, general):
+    if not (ROOT / "cresso_amd" / "libcresso_hip.so").exists():
+        pytest.skip("library not built")
+    assert _plan(shape, rank, bins, tables)[:2] == (rows, general)
+
+
 @pytest.mark.parametrize("fails", ["begin", "step", "between", "end", "step and end"])
 def test_spectral_launch_joins_its_streams_after_an_error(fails, monkeypatch):
     # whatever fails in a step on side streams, every stream that was forked

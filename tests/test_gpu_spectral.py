@@ -31,7 +31,7 @@ CASES = [
      1e-3, 0.02),
     ("no_hash_b0", [(96, 80)], dict(rank=8, hash_bins=0), 3, 1e-3, 0.02),
     # ranks above 16: the general sweeps with 32 projection slots (2 x 32
-    # carriers per element), MODE 0 and MODE 1 tiles, 2-D and 3-D
+    # carriers per element), 2-D and 3-D
     ("r24_300x257", [(300, 257)], dict(rank=24, max_frequency=6, hash_bins=64, hash_tables=2), 3, 1e-3, 0.02),
     ("r32_1024x512_fast", [(1024, 512)], dict(rank=32, max_frequency=7, hash_bins=64, hash_tables=2), 3, 1e-3, 0.02),
     ("r20_3d_t4", [(6, 10, 12)], dict(rank=20, max_frequency=7, hash_bins=256, hash_tables=4, min_spectral_size=1),
@@ -40,7 +40,7 @@ CASES = [
     ("r24_variants_40x30", [(40, 30)], dict(rank=24, max_frequency=6, hash_bins=64, hash_tables=3, weight_decay=0.01,
                                             maximize=True, local_sharpness=0.3, min_spectral_size=1, warmup_steps=0),
      4, 1e-2, 0.05),
-    # the matrix-core fast path with 32-row panels and few blocks (1024 rows)
+    # the matrix-core sweeps with few blocks (16-row panels)
     ("fast_1024x768", [(1024, 768)], dict(rank=8, hash_bins=64, hash_tables=2), 3, 1e-3, 0.02),
     ("fast_1024x512_r4_b32", [(1024, 512)], dict(rank=4, max_frequency=3, hash_bins=32, hash_tables=2), 3, 1e-3,
      0.02),
@@ -98,8 +98,8 @@ SPIKE_CASES = [
     # blocks (16384 elements, four rows of 4096, each)
     ("p4_4096sq_clamp", (4096, 4096), 4.0, [((1234, 567), 30.0)]),
     ("p4_4096sq_clamp_x5", (4096, 4096), 4.0, [((100 + 700 * i, 37 * i + 5), 30.0) for i in range(5)]),
-    # the general sweeps (odd column count) and the matrix-core sweeps with
-    # 32-row panels, energy power 6
+    # the matrix-core sweeps of an odd column count, and of full tiles in
+    # 16-row panels at energy power 6
     ("p4_300x257_clamp", (300, 257), 4.0, [((17, 200), 30.0)]),
     ("p6_1024x768_spike", (1024, 768), 6.0, [((700, 3), 10.0)]),
 ]
