@@ -4270,6 +4270,17 @@ inline void set_panels(Geom& g, int64_t rows) {
     g.nblk = g.slabs * g.panels;
 }
 
+// Carrier-count variant of a plan's sweeps (rank and distinct column carriers
+// fixed at compile time), and the LDS its general sweeps need with g's panels.
+inline int sweep_variant(const Geom& g) {
+    return (g.R <= 4 && g.K <= 9) ? 0 : (g.R <= 8 && g.K <= 11) ? 1 : (g.R <= 8) ? 2 : (g.R <= 16) ? 3 : 4;
+}
+inline size_t general_lds(const Geom& g) {
+    constexpr int KP[5] = {kcp<9>(), kcp<11>(), kcp<17>(), kcp<33>(), kcp<65>()}, RM[5] = {4, 8, 8, 16, 32};
+    const int v = sweep_variant(g);
+    return std::max(lds_sweep2(g, 2 * RM[v]), std::max(lds_sweep3(g, KP[v], 2 * RM[v]), lds_sweep4(g, KP[v], 2 * RM[v])));
+}
+
 // One step of `count` tensors of plan P: hd[0..count) are their descriptors
 // on the host; for count > 1, dv is the same array in device memory and each
 // tensor's per-step scratch follows the previous one's at a stride of ls
@@ -4470,9 +4481,7 @@ int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, 
 template <typename PT, typename GT>
 int32_t spectral_run(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, int count,
                      const cresso_spectral_desc* dv, size_t ls, void* ws, const cresso_hyper& h, hipStream_t s) {
-    const int R = P.g.R, K = P.g.K;
-    const int var = (R <= 4 && K <= 9) ? 0 : (R <= 8 && K <= 11) ? 1 : (R <= 8) ? 2 : (R <= 16) ? 3 : 4;
-    switch (var) {
+    switch (sweep_variant(P.g)) {
         case 0: return run_step<4, 9, PT, GT>(P, hd, count, dv, ls, ws, h, s);
         case 1: return run_step<8, 11, PT, GT>(P, hd, count, dv, ls, ws, h, s);
         case 2: return run_step<8, 17, PT, GT>(P, hd, count, dv, ls, ws, h, s);

@@ -28,6 +28,44 @@ double hash_unit_host(int64_t n, int64_t salt) {
 
 size_t al256(size_t v) { return (v + 255) & ~(size_t)255; }
 
+// Workspace layout; part_blocks: blocks whose partial sums it holds.
+void layout_spectral(cresso_spectral_plan& P, int32_t part_blocks) {
+    const Geom& g = P.g;
+    Offs& o = P.o;
+    size_t off = 0;
+    auto take = [&](size_t bytes) { size_t at = off; off = al256(off + bytes); return at; };
+    o.axc = take(sizeof(AxisConst) * P.axc.size());
+    o.meta = take(sizeof(ModeMeta) * P.meta.size());
+    o.csrc = take(sizeof(CarrierSrc) * P.csrc.size());
+    o.rowtab = take(sizeof(float) * (size_t)g.rows * g.RW);
+    o.coltab = take(sizeof(float) * (size_t)(g.KA - 1) * g.cols);   // 2*rmax+1 rows, zero beyond K
+    o.stats = take(sizeof(double) * 4 * g.R);
+    o.bounds = take(sizeof(double) * 2 * g.R);
+    o.gram = take(sizeof(double) * 4 * (size_t)g.R * g.R);
+    o.gpart = take(sizeof(double) * (size_t)g.nblkg * (4 * (size_t)g.R * g.R + (size_t)g.K * g.K));
+    o.counts = take(sizeof(unsigned long long) * (size_t)g.T * g.B);
+    o.cooc = take(cooc_closed(g) ? sizeof(unsigned long long) * (size_t)cooc_pairs(g) * g.B * g.B : 0);
+    o.bins = take((size_t)g.binbytes * (size_t)g.n);
+    o.tbuf = take(sizeof(float) * (size_t)g.n);
+    o.part = take(sizeof(double) * (size_t)NVMAX * std::max(part_blocks, g.nblk1));
+    o.part1 = take(sizeof(double) * 2 * (size_t)g.nblk1);   // sweep 1's sums and maxima, read by every block of sweep 2
+    o.sums = take(sizeof(double) * (size_t)NVMAX);
+    o.hist = take(sizeof(unsigned long long) * (size_t)hist_words(g));   // low-word copies, then the high words
+    // per-block histogram partials of the matrix-core sweeps (two or four tables of one-byte bins)
+    o.hpart = take(mtables(g) ? sizeof(unsigned long long) * (size_t)g.T * g.B * g.nblk : 0);
+    o.lt = take(sizeof(float) * (size_t)g.T * g.B);
+    o.imp = take(sizeof(float) * (size_t)g.T * g.B);
+    o.rowfx = take(sizeof(unsigned long long) * (size_t)g.rows);
+    o.colfx = take(sizeof(unsigned long long) * (size_t)g.cols);
+    o.colfac = take(sizeof(float) * (size_t)g.cols);
+    int64_t sum_trail = 0;
+    for (int a = 0; a < g.ntrail; ++a) sum_trail += g.tdim[a];
+    o.terms = take(sizeof(float) * (size_t)std::max<int64_t>(1, sum_trail));
+    o.ctrl = take(sizeof(Ctrl));
+    o.desc = take(sizeof(cresso_spectral_desc));   // the tensor's descriptor in a batched step
+    o.total = P.work == CRESSO_F64 ? plan_f64_layout(P, off) : off;
+}
+
 int32_t plan_spectral(const int64_t* shape, int32_t ndim, const int64_t* freqs, int32_t rank, int32_t bins,
                       int32_t tables, int32_t work, cresso_spectral_plan& P) {
     if (ndim < 1 || ndim > 8) return fail(CRESSO_E_INVALID, "spectral route: ndim %d outside 1..8", ndim);
@@ -222,40 +260,33 @@ int32_t plan_spectral(const int64_t* shape, int32_t ndim, const int64_t* freqs, 
     g.inv_n = 1.0 / (double)g.n;
     g.hs_row = ldexp(1.0, (int)std::floor(62.0 - std::log2(1.0e6 * (double)g.cols)));
     g.hs_col = ldexp(1.0, (int)std::floor(62.0 - std::log2(1.0e6 * (double)g.rows)));
-    // workspace layout
-    Offs& o = P.o;
-    size_t off = 0;
-    auto take = [&](size_t bytes) { size_t at = off; off = al256(off + bytes); return at; };
-    o.axc = take(sizeof(AxisConst) * P.axc.size());
-    o.meta = take(sizeof(ModeMeta) * P.meta.size());
-    o.csrc = take(sizeof(CarrierSrc) * P.csrc.size());
-    o.rowtab = take(sizeof(float) * (size_t)g.rows * g.RW);
-    o.coltab = take(sizeof(float) * (size_t)(g.KA - 1) * g.cols);   // 2*rmax+1 rows, zero beyond K
-    o.stats = take(sizeof(double) * 4 * g.R);
-    o.bounds = take(sizeof(double) * 2 * g.R);
-    o.gram = take(sizeof(double) * 4 * (size_t)g.R * g.R);
-    o.gpart = take(sizeof(double) * (size_t)g.nblkg * (4 * (size_t)g.R * g.R + (size_t)g.K * g.K));
-    o.counts = take(sizeof(unsigned long long) * (size_t)g.T * g.B);
-    o.cooc = take(cooc_closed(g) ? sizeof(unsigned long long) * (size_t)cooc_pairs(g) * g.B * g.B : 0);
-    o.bins = take((size_t)g.binbytes * (size_t)g.n);
-    o.tbuf = take(sizeof(float) * (size_t)g.n);
-    o.part = take(sizeof(double) * (size_t)NVMAX * std::max(std::max(g.nblk, gg.nblk), g.nblk1));
-    o.part1 = take(sizeof(double) * 2 * (size_t)g.nblk1);   // sweep 1's sums and maxima, read by every block of sweep 2
-    o.sums = take(sizeof(double) * (size_t)NVMAX);
-    o.hist = take(sizeof(unsigned long long) * (size_t)hist_words(g));   // low-word copies, then the high words
-    // per-block histogram partials of the matrix-core sweeps (two or four tables of one-byte bins)
-    o.hpart = take(mtables(g) ? sizeof(unsigned long long) * (size_t)g.T * g.B * g.nblk : 0);
-    o.lt = take(sizeof(float) * (size_t)g.T * g.B);
-    o.imp = take(sizeof(float) * (size_t)g.T * g.B);
-    o.rowfx = take(sizeof(unsigned long long) * (size_t)g.rows);
-    o.colfx = take(sizeof(unsigned long long) * (size_t)g.cols);
-    o.colfac = take(sizeof(float) * (size_t)g.cols);
-    int64_t sum_trail = 0;
-    for (int a = 0; a < g.ntrail; ++a) sum_trail += g.tdim[a];
-    o.terms = take(sizeof(float) * (size_t)std::max<int64_t>(1, sum_trail));
-    o.ctrl = take(sizeof(Ctrl));
-    o.desc = take(sizeof(cresso_spectral_desc));   // the tensor's descriptor in a batched step
-    o.total = work == CRESSO_F64 ? plan_f64_layout(P, off) : off;
+    layout_spectral(P, std::max(g.nblk, gg.nblk));
+    // A plan that fits the no-alloc entry's workspace only with fewer blocks'
+    // partial sums takes taller panels: (704,5824), rank 4, three tables, 32.5
+    // MiB with 16 rows, 32.0 with 64.  First the general sweeps those of the
+    // matrix-core sweeps, then, where all are general, 32 or 64 rows that tile
+    // the tensor's (and whose tables fit in LDS).
+    if (P.o.total > CRESSO_SPECTRAL_NOALLOC_MAX_BYTES) {
+        const int32_t rows = g.PR, general = P.general_rows;
+        auto try_panels = [&](int64_t r) {
+            set_panels(g, r);
+            P.general_rows = g.PR;
+            layout_spectral(P, g.nblk);
+            return P.o.total <= CRESSO_SPECTRAL_NOALLOC_MAX_BYTES;
+        };
+        const int64_t tall = std::min<int64_t>(rank <= 16 && g.rows % 64 == 0 ? 64 : 32, most);
+        bool fits = rows > general && try_panels(rows);
+        if (!fits && rows == general && tall > rows && g.rows >= 256 && g.rows % 32 == 0) {
+            Geom gt = g;
+            set_panels(gt, tall);
+            fits = (work == CRESSO_F64 || general_lds(gt) <= SP_LDS_MAX) && try_panels(tall);
+        }
+        if (!fits) {
+            set_panels(g, rows);
+            P.general_rows = general;
+            layout_spectral(P, std::max(g.nblk, gg.nblk));
+        }
+    }
     return CRESSO_OK;
 }
 

@@ -457,6 +457,27 @@ def test_spectral_plan_panels(shape, rank, bins, tables, rows, general):
     assert _plan(shape, rank, bins, tables)[:2] == (rows, general)
 
 
+@pytest.mark.parametrize("shape,rank,bins,tables", [((704, 5824), 4, 128, 3), ((960, 5632), 4, 512, 1)])
+def test_plans_near_the_noalloc_limit_fit_it_with_taller_panels(shape, rank, bins, tables):
+    # rows that tile by 32: fewer blocks' partial sums where the workspace would
+    # not fit the no-alloc entry's 32 MiB otherwise; ordinary panels well below it
+    if not (ROOT / "cresso_amd" / "libcresso_hip.so").exists():
+        pytest.skip("library not built")
+    rows, general, nbytes = _plan(shape, rank, bins, tables)
+    assert nbytes <= 32 << 20 and rows == general == 64
+    half = (shape[0] // 2,) + shape[1:]
+    assert _plan(half, rank, bins, tables)[0] == 16
+
+
+def test_ragged_plan_near_the_noalloc_limit_fits_it_with_one_panel_height():
+    # the general sweeps then take the matrix-core sweeps' panels
+    if not (ROOT / "cresso_amd" / "libcresso_hip.so").exists():
+        pytest.skip("library not built")
+    rows, general, nbytes = _plan((997, 3775), 16, 128, 4)
+    assert nbytes <= 32 << 20 and rows == general == 64
+    assert _plan((797, 3775), 16, 128, 4)[:2] == (64, 16)
+
+
 @pytest.mark.parametrize("fails", ["begin", "step", "between", "end", "step and end"])
 def test_spectral_launch_joins_its_streams_after_an_error(fails, monkeypatch):
     # whatever fails in a step on side streams, every stream that was forked
