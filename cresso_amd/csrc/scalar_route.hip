@@ -800,6 +800,7 @@ constexpr int SR_WIDE_NT = 256;              // threads per block of the wide fo
 // 156, 66 x (5632,16) 156 / 134 / 146, 132 x (5632,16) and (16,5632) 208 / 218
 // / 240.
 inline int64_t wide_chunk(int64_t elements) { return elements <= 3 << 19 ? 2048 : (elements <= 1 << 23 ? 4096 : 8192); }
+constexpr int64_t SR_MIDDLE_WIDE = 5 << 19;  // elements of middle tensors up to which they join the wide form (build_plan)
 constexpr int64_t SR_WIDE_MIN = SR_RESIDENT_MAX + 1;   // non-resident tensors this large use the wide form
 constexpr int64_t SR_WIDE_MID = 16384;       // ... and from this size when fewer than SR_WIDE_FILL of them
 constexpr int32_t SR_WIDE_FILL = 256;        //     (one workgroup per tensor would leave CUs idle)
@@ -2432,8 +2433,8 @@ int32_t plan_desc(const cresso_scalar_desc& d, const cresso_hyper& h, ScalarRec&
         }
     }
     if (kind == 0 && small_ok(d, r.sum_dims)) {
-        kind = n <= SS_MAX ? 4 : 6;
-        scratch = 0;
+        kind = n <= SS_MAX ? 4 : 6;   // (6: build_plan may choose the wide form, which needs the scratch)
+        if (kind == 4) scratch = 0;
     }
     if (kind == 0 && n >= SR_WIDE_MIN) kind = 2;
     if (kind == 4) lds = ss_lds(n <= 8 * SS_NT ? 8 : 16);
@@ -2655,6 +2656,28 @@ int32_t build_plan(const cresso_scalar_desc* descs, int32_t count, const cresso_
     auto joins = [&](int32_t i) {
         return var[(size_t)i].kind == 1 && !var[(size_t)i].full && small_ok(descs[i], descs[i].shape[0] + descs[i].shape[1]);
     };
+    // Middle tensors without such company go along in the wide form's launches,
+    // if the plan has them (for the same dtypes) and the tensors are few: the
+    // middle launch takes about 50 us whatever it holds, the wide form some 15
+    // us for another million elements.  us a step of bf16 plans in two forms /
+    // all wide (middle elements): 1 x adapters of (734,4502) at rank 33 145 /
+    // 108 (0.27 M), 4 x 171 / 158 (1.07 M), 8 x (1000,4000) at rank 24 168 /
+    // 152 (2.1 M), 12 x 186 / 209 (3.2 M), 12 x (734,4502) 253 / 271 (3.2 M).
+    int64_t elements[4][4] = {}, wide_in[4][4] = {}, join_in[4][4] = {};
+    for (int32_t i = 0; i < count; ++i) {
+        const Variant& v = var[(size_t)i];
+        if (v.kind == 6) elements[v.pt][v.gt] += descs[i].numel;
+        wide_in[v.pt][v.gt] += v.kind == 2;
+        join_in[v.pt][v.gt] += joins(i);
+    }
+    for (int32_t i = 0; i < count; ++i) {
+        Variant& v = var[(size_t)i];
+        if (v.kind != 6) continue;
+        if (wide_in[v.pt][v.gt] > 0 && join_in[v.pt][v.gt] == 0 && elements[v.pt][v.gt] <= SR_MIDDLE_WIDE)
+            v.kind = 2;
+        else
+            scr[(size_t)i] = 0;
+    }
     int32_t middle = 0, joining = 0;
     for (int32_t i = 0; i < count; ++i) {
         middle += var[(size_t)i].kind == 6;

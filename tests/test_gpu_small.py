@@ -40,6 +40,16 @@ def test_small_half_dtypes_first_step(dtype, micro):
     compare(*res, param_tol=BF16_PARAM_TOL, state_tol=F32_TOL)
 
 
+@pytest.mark.parametrize("kw", [KW, OPTIONS, dict(KW, instant_metric_coupling=0.0)], ids=["plain", "options", "no_axes"])
+@pytest.mark.parametrize("extra", [[], [(2048, 16)]], ids=["wide", "middle"])
+def test_middle_tensors_beside_wide_ones_match_oracle(kw, extra):
+    """Tensors of 16 to 32 Ki elements in a plan that has larger ones: in the wide form's launches, or, beside a
+    resident tensor of their size, in the middle kernel's."""
+    announce(f"middle tensors, {len(extra)} resident, {sorted(set(kw) - set(KW))}")
+    shapes = [(16385,), (40, 700), (7, 40, 100), (32768,), (33, 734), (2, 3, 5000), (300, 257), (65537,)] + extra
+    compare(*run_pair(shapes, torch.float32, kw, steps=3, seed=45))
+
+
 @pytest.mark.parametrize("bad", [float("nan"), float("inf")])
 def test_small_tensor_with_a_bad_gradient_has_no_number_left(bad):
     """One NaN or infinite gradient element: the reservoirs and every updated value become NaN, as in the reference."""
