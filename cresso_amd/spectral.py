@@ -7,10 +7,10 @@ workspace (carrier tables, cached coordinate-hash bins, scratch).
 A step of several spectral tensors (`step_many`) first batches the tensors
 that share a plan (and dtypes, hard channel and hash state): one batched C
 call steps a batch, every launch covering all its tensors, with the plan's
-tables held once and per-step scratch (about 4 bytes per element plus a few
-KB) once per tensor.  A batch holds at most BATCH_BYTES of such scratch;
-larger groups are cut into that many chunks.  The units of work (batches and
-single tensors) are spread over up to LANES side streams (default priority),
+tables held once and per-step scratch (about 4 bytes per element plus its
+blocks' partial sums) once per tensor.  A batch holds at most BATCH_BYTES of
+such scratch; larger groups are cut into that many chunks.  The units of work
+(batches and single tensors) are spread over up to LANES side streams (default priority),
 so that one unit's small finish kernels and partly filled sweeps overlap
 with another's work.  Every lane has its own workspace per unit kind: units
 that share a workspace run one after another on that lane's stream, so its
@@ -71,6 +71,15 @@ def assign_lanes(keys: Sequence[tuple], lanes: int) -> List[int]:
     return out
 
 
+def _make_plan(lib, shape, freqs: Tuple[int, ...], rank: int, bins: int, tables: int, work: int) -> ctypes.c_void_p:
+    shp = (ctypes.c_int64 * 8)(*shape)
+    fr = (ctypes.c_int64 * max(1, len(freqs)))(*freqs)
+    plan = lib.cresso_spectral_plan_create_ex(shp, len(shape), fr, rank, bins, tables, work)
+    if not plan:
+        _native.check(-1, "spectral route plan")
+    return ctypes.c_void_p(plan)
+
+
 class _Workspace:
     """A plan with its device workspace: for one tensor (count=None) or for
     batches of up to `count` tensors."""
@@ -79,13 +88,7 @@ class _Workspace:
                  device: torch.device, count=None, work: int = _native.F32):
         self.lib = lib
         self.count = count
-        nd = len(shape)
-        shp = (ctypes.c_int64 * 8)(*shape)
-        fr = (ctypes.c_int64 * max(1, len(freqs_host)))(*freqs_host)
-        plan = lib.cresso_spectral_plan_create_ex(shp, nd, fr, rank, bins, tables, work)
-        if not plan:
-            _native.check(-1, "spectral route plan")
-        self.plan = ctypes.c_void_p(plan)
+        self.plan = _make_plan(lib, shape, freqs_host, rank, bins, tables, work)
         hyper = _native.hyper_from_group(group)
         stream = ctypes.c_void_p(_native.stream_handle(device))
         if count is None:
@@ -110,9 +113,9 @@ class _Workspace:
 
 
 def lane_scratch_bytes(numel: int) -> int:
-    """Per-tensor scratch of a batched step, for sizing chunks: the tangent
-    field (4 bytes per element) dominates; the rest is a few KB per tensor
-    plus small per-row and per-column sums."""
+    """Least per-tensor scratch of a batched step: the tangent field (4 bytes
+    per element), a few KB and small per-row and per-column sums.  (The blocks'
+    partial sums and histograms come on top: SpectralEngine._lane_bytes.)"""
     return 4 * numel + (1 << 16)
 
 
@@ -122,8 +125,11 @@ class SpectralEngine:
     BATCH = True              # batch same-plan tensors into one launch per kernel
     BATCH_BYTES = 512 << 20   # per-tensor scratch held by one batch (C4: 3 % faster than 256 MiB, as fast as 1 GiB)
 
+    lane_bytes: Dict[tuple, int] = {}   # plan key -> per-tensor scratch of its batches (a dict of each engine's own)
+
     def __init__(self):
         self.lib = _native.load()
+        self.lane_bytes = {}
         self.ws: Dict[tuple, _Workspace] = {}   # (plan key, unit kind, lane) -> workspace
         self.version = 0                        # changes with every workspace made or dropped
         self.side: Dict[torch.device, List[torch.cuda.Stream]] = {}
@@ -171,6 +177,22 @@ class SpectralEngine:
             self.ws[wkey] = ws
             self.version += 1
         return ws
+
+    def _lane_bytes(self, key: tuple, rank: int, numel: int) -> int:
+        """Per-tensor scratch of a batched step, for sizing batches: the
+        library's stride between tensors of a batched workspace."""
+        got = self.lane_bytes.get(key)
+        if got is None:
+            if not isinstance(key, tuple):   # (no plan to ask)
+                return lane_scratch_bytes(numel)
+            _, shape, freqs, bins, tables, work = key
+            plan = _make_plan(self.lib, shape, freqs, rank, bins, tables, work)
+            try:
+                one, two = (int(self.lib.cresso_spectral_batched_workspace_bytes(plan, n)) for n in (1, 2))
+            finally:
+                self.lib.cresso_spectral_plan_destroy(plan)
+            got = self.lane_bytes[key] = two - one
+        return got
 
     def _prepare(self, param: torch.Tensor, grad: torch.Tensor, st: dict, group: dict):
         """Validate one tensor's state and build its descriptor; -> (key, rank, desc)."""
@@ -234,7 +256,7 @@ class SpectralEngine:
             if len(idx) == 1:
                 units.append(((key, False), key, rank, [prepared[idx[0]][2]], [sts[idx[0]]]))
                 continue
-            per = lane_scratch_bytes(prepared[idx[0]][2].numel)
+            per = self._lane_bytes(key, rank, prepared[idx[0]][2].numel)
             chunks = -(-len(idx) * per // self.BATCH_BYTES)
             m = -(-len(idx) // chunks)
             for c in range(0, len(idx), m):

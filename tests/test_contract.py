@@ -478,6 +478,33 @@ def test_ragged_plan_near_the_noalloc_limit_fits_it_with_one_panel_height():
     assert _plan((797, 3775), 16, 128, 4)[:2] == (64, 16)
 
 
+def test_spectral_batches_stay_within_their_scratch():
+    # (640,4096) at four tables of 256 bins: 16-row panels, whose histogram
+    # partials take half as much as the tangent field again
+    if not (ROOT / "cresso_amd" / "libcresso_hip.so").exists():
+        pytest.skip("library not built")
+    import ctypes
+
+    from cresso_amd.spectral import SpectralEngine
+
+    shape = (640, 4096)
+    ps = [torch.nn.Parameter(torch.zeros(shape)) for _ in range(8)]
+    opt = CRESSO5(ps, cuda_ops="required", rank=16, max_frequency=7, hash_bins=256, hash_tables=4)
+    group, eng = opt.param_groups[0], SpectralEngine()
+    eng.BATCH_BYTES = 40 << 20
+    sts = [opt._init_spectral(p, group) for p in ps]
+    prepared = [eng._prepare(p, p.data, st, group) for p, st in zip(ps, sts)]
+    units = eng._units(prepared, sts)
+    fr = sts[0]["freqs"].reshape(-1).tolist()
+    plan = eng.lib.cresso_spectral_plan_create_ex((ctypes.c_int64 * 8)(*shape), 2, (ctypes.c_int64 * len(fr))(*fr), 16,
+                                                  256, 4, _native.F32)
+    plan = ctypes.c_void_p(plan)
+    size = [int(eng.lib.cresso_spectral_batched_workspace_bytes(plan, k)) for k in (1, 2)]
+    eng.lib.cresso_spectral_plan_destroy(plan)
+    assert sum(len(u[4]) for u in units) == 8 and len(units) > 1
+    assert max(len(u[4]) for u in units) * (size[1] - size[0]) <= eng.BATCH_BYTES
+
+
 @pytest.mark.parametrize("fails", ["begin", "step", "between", "end", "step and end"])
 def test_spectral_launch_joins_its_streams_after_an_error(fails, monkeypatch):
     # whatever fails in a step on side streams, every stream that was forked
