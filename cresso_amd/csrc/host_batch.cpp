@@ -54,17 +54,12 @@ struct BatchGuard {
         int64_t offset, numel;
         caffe2::TypeMeta dtype;
     };
-    // One (key, value) of a state dict at plan time.
-    struct Entry {
-        py::object key, value;   // value: null unless planned
-        bool step;
-    };
     struct Item {
-        py::object param, dict;
+        py::object param, dict, keys;   // keys: a tuple; the state's planned entries, from planned[first] on
+        size_t first;
         const void* pptr;
         std::vector<int64_t> sizes;
         int pdtype, gdtype, device;
-        std::vector<Entry> entries;   // every entry, in the dict's order
         int64_t step0;                // state["step"] at plan time
         mutable uint64_t version;     // the dict's, when its entries were last compared (or written by bump)
     };
@@ -82,6 +77,7 @@ struct BatchGuard {
             throw std::invalid_argument("BatchGuard: one state and its keys per parameter");
         with_state = states.size() != 0;
         items.reserve(n);
+        planned.reserve(with_state ? 8 * n : 0);
         for (size_t i = 0; i < n; ++i) {
             PyObject* o = ps[i].ptr();
             if (!THPVariable_Check(o)) throw std::invalid_argument("BatchGuard: parameters must be tensors");
@@ -103,54 +99,48 @@ struct BatchGuard {
         }
     }
 
-    void plan_state(Item& it, PyObject* st, PyObject* want) {
-        if (!PyDict_Check(st)) throw std::invalid_argument("BatchGuard: a state must be a dict");
+    static PyObject* step_key() {
+        static PyObject* const key = PyUnicode_InternFromString("step");
+        return key;
+    }
+
+    // state["step"], or -1
+    static int64_t step_of(PyObject* st) {
+        PyObject* v = PyDict_GetItemWithError(st, step_key());   // borrowed
+        const int64_t s = v && PyLong_Check(v) ? PyLong_AsLongLong(v) : -1;
+        if (s == -1) PyErr_Clear();
+        return s;
+    }
+
+    void plan_state(Item& it, PyObject* st, PyObject* keys) {
+        if (!PyDict_Check(st) || !PyTuple_Check(keys)) throw std::invalid_argument("BatchGuard: a state must be a dict, its keys a tuple");
         it.dict = py::reinterpret_borrow<py::object>(st);
-        it.step0 = -1;
-        Py_ssize_t missing = PySequence_Size(want);
-        PyObject *k, *v;
-        Py_ssize_t pos = 0;
-        while (PyDict_Next(st, &pos, &k, &v)) {
-            Entry e{py::reinterpret_borrow<py::object>(k), py::object(), false};
-            const int used = PySequence_Contains(want, k);
-            if (used < 0) throw py::error_already_set();
-            if (used) {
-                if (!THPVariable_Check(v)) throw std::invalid_argument("BatchGuard: a planned state must be a tensor");
-                e.value = py::reinterpret_borrow<py::object>(v);
-                const at::Tensor& x = THPVariable_Unpack(v);
-                planned.push_back(Planned{x, x.storage(), x.storage().data()});
-                if (x.numel() != 1 || x.storage().nbytes() != x.itemsize())
-                    views.push_back(View{x.unsafeGetTensorImpl(), x.storage_offset(), x.numel(), x.dtype()});
-                --missing;
-            } else if (PyUnicode_Check(k) && PyUnicode_CompareWithASCIIString(k, "step") == 0 && PyLong_Check(v)) {
-                e.step = true;
-                it.step0 = PyLong_AsLongLong(v);
-            }
-            it.entries.push_back(std::move(e));
+        it.keys = py::reinterpret_borrow<py::object>(keys);
+        it.first = planned.size();
+        for (Py_ssize_t k = 0; k < PyTuple_GET_SIZE(keys); ++k) {
+            PyObject* v = PyDict_GetItemWithError(st, PyTuple_GET_ITEM(keys, k));   // borrowed
+            if (!v && PyErr_Occurred()) throw py::error_already_set();
+            if (!v || !THPVariable_Check(v)) throw std::invalid_argument("BatchGuard: a state lacks a planned tensor");
+            const at::Tensor& x = THPVariable_Unpack(v);
+            planned.push_back(Planned{x, x.storage(), x.storage().data()});
+            if (x.numel() != 1 || x.storage().nbytes() != x.itemsize())
+                views.push_back(View{x.unsafeGetTensorImpl(), x.storage_offset(), x.numel(), x.dtype()});
         }
-        if (missing != 0 || it.step0 < 0) throw std::invalid_argument("BatchGuard: a state lacks its 'step' or a planned key");
+        it.step0 = step_of(st);
+        if (it.step0 < 0) throw std::invalid_argument("BatchGuard: a state lacks its step count");
         it.version = dict_version(st);
     }
 
-    // Whether a state dict holds the planned entries and step count.
+    // Whether a state dict holds the planned tensors and step count.
     bool entries_hold(const Item& it) const {
         const uint64_t version = dict_version(it.dict.ptr());
         if (version != 0 && version == it.version) return true;
-        size_t j = 0;
-        PyObject *k, *v;
-        Py_ssize_t pos = 0;
-        while (PyDict_Next(it.dict.ptr(), &pos, &k, &v)) {
-            if (j == it.entries.size()) return false;
-            const Entry& e = it.entries[j++];
-            if (k != e.key.ptr() || (e.value && v != e.value.ptr())) return false;
-            if (e.step) {
-                if (!PyLong_Check(v)) return false;
-                const long long s = PyLong_AsLongLong(v);
-                if (s == -1) PyErr_Clear();
-                if (s != it.step0 + ran) return false;
-            }
+        for (Py_ssize_t k = 0; k < PyTuple_GET_SIZE(it.keys.ptr()); ++k) {
+            PyObject* v = PyDict_GetItemWithError(it.dict.ptr(), PyTuple_GET_ITEM(it.keys.ptr(), k));   // borrowed
+            if (!v && PyErr_Occurred()) throw py::error_already_set();
+            if (!v || !THPVariable_Check(v) || !THPVariable_Unpack(v).is_same(planned[it.first + (size_t)k].tensor)) return false;
         }
-        if (j != it.entries.size()) return false;
+        if (step_of(it.dict.ptr()) != it.step0 + ran) return false;
         it.version = version;
         return true;
     }
@@ -214,7 +204,7 @@ struct BatchGuard {
 
     // state["step"] += 1 for each state dict (the library advanced its own copy).
     void bump(const py::list& states) {
-        static PyObject* key = PyUnicode_InternFromString("step");
+        PyObject* const key = step_key();
         ++ran;
         size_t i = 0;
         for (const py::handle& h : states) {
@@ -384,6 +374,61 @@ struct SpectralGuard {
     }
 };
 
+// Dtype code of the C ABI; -1: none.
+int dtype_code(at::ScalarType t) {
+    return t == at::kFloat ? CRESSO_F32 : t == at::kDouble ? CRESSO_F64 : t == at::kHalf ? CRESSO_F16 : t == at::kBFloat16 ? CRESSO_BF16 : -1;
+}
+
+// Writes the scalar plan's descriptors of these tensors to out.  False (out
+// must not be used) unless every state holds, under each of its keys (the
+// descriptor's order), a tensor of the work dtype (fp64 for fp64 parameters,
+// else fp32) on the parameter's device: of one element, or, for the first
+// fields[i] keys (a micro tensor's), contiguous in the parameter's shape; and
+// "step".  (In Python 3 us a tensor, as long again as the rest of a plan.)
+bool scalar_descs(const py::list& ps, const py::list& grads, const py::list& states, const py::list& keys,
+                  const std::vector<int>& fields, uintptr_t out_addr) {
+    const size_t n = ps.size();
+    if (grads.size() != n || states.size() != n || keys.size() != n || fields.size() != n) return false;
+    PyObject* const k_step = PyUnicode_InternFromString("step");
+    const py::object hold = py::reinterpret_steal<py::object>(k_step);
+    cresso_scalar_desc* out = reinterpret_cast<cresso_scalar_desc*>(out_addr);
+    for (size_t i = 0; i < n; ++i) {
+        PyObject *o = PyList_GET_ITEM(ps.ptr(), i), *go = PyList_GET_ITEM(grads.ptr(), i);
+        PyObject *st = PyList_GET_ITEM(states.ptr(), i), *ks = PyList_GET_ITEM(keys.ptr(), i);
+        if (!THPVariable_Check(o) || !THPVariable_Check(go) || !PyDict_Check(st) || !PyTuple_Check(ks)) return false;
+        const at::Tensor &p = THPVariable_Unpack(o), &g = THPVariable_Unpack(go);
+        const at::ScalarType want = p.scalar_type() == at::kDouble ? at::kDouble : at::kFloat;
+        cresso_scalar_desc d{};
+        d.param = p.data_ptr();
+        d.grad = g.data_ptr();
+        d.param_dtype = dtype_code(p.scalar_type());
+        d.grad_dtype = dtype_code(g.scalar_type());
+        d.route = fields[i] > 0 ? 1 : 0;
+        if (p.dim() > 8 || PyTuple_GET_SIZE(ks) > 8 || d.param_dtype < 0 || d.grad_dtype < 0) return false;
+        d.ndim = (int32_t)p.dim();
+        d.numel = p.numel();
+        for (int a = 0; a < d.ndim; ++a) d.shape[a] = p.size(a);
+        for (Py_ssize_t k = 0; k < PyTuple_GET_SIZE(ks); ++k) {
+            PyObject* v = PyDict_GetItemWithError(st, PyTuple_GET_ITEM(ks, k));   // borrowed
+            if (!v && PyErr_Occurred()) throw py::error_already_set();
+            if (!v || !THPVariable_Check(v)) return false;
+            const at::Tensor& x = THPVariable_Unpack(v);
+            if (x.scalar_type() != want || x.device() != p.device()) return false;
+            if (k < fields[i] ? x.sizes() != p.sizes() || !x.is_contiguous() : x.numel() != 1) return false;
+            d.state[k] = x.data_ptr();
+        }
+        PyObject* v = PyDict_GetItemWithError(st, k_step);   // borrowed
+        const long long s = v && PyLong_Check(v) ? PyLong_AsLongLong(v) : -1;
+        if (s < 0 || s >= INT32_MAX) {
+            PyErr_Clear();
+            return false;
+        }
+        d.step = (int32_t)s;
+        out[i] = d;
+    }
+    return true;
+}
+
 // Whether two lists hold the same objects.
 bool same_objects(const py::list& a, const py::list& b) {
     if (a.size() != b.size()) return false;
@@ -408,4 +453,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         .def("fill", &SpectralGuard::fill)
         .def("bump", &SpectralGuard::bump);
     m.def("same_objects", &same_objects);
+    m.def("scalar_descs", &scalar_descs);
 }

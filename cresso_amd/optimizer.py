@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+import operator
 from typing import Dict, Iterable, List, Optional, Sequence, Tuple
 
 import torch
@@ -102,42 +103,51 @@ def theoretical_state_elements(shape: Sequence[int], rank: int, spectral: bool =
     return 8
 
 
+def _check_scalar_state(p: Tensor, st: dict) -> None:
+    want = _state_dtype(p.dtype)
+    for k in _SCALAR_KEYS:
+        v = st.get(k)
+        if not torch.is_tensor(v) or v.dtype != want or v.device != p.device or v.numel() != 1:
+            got = f"{v.dtype} with {v.numel()} elements on {v.device}" if torch.is_tensor(v) else type(v).__name__
+            raise RuntimeError(f"CRESSO5 scalar route: state {k!r} is {got}, expected one {want} on {p.device}")
+
+
+def _check_micro_state(p: Tensor, st: dict) -> None:
+    want = _state_dtype(p.dtype)
+    for k in _MICRO_KEYS:
+        if k not in st:
+            raise RuntimeError(f"CRESSO5 micro route: state {k!r} is missing (the state belongs to another route)")
+        v = st[k]
+        if v.dtype != want or v.device != p.device:
+            raise RuntimeError(f"CRESSO5 micro route: state {k!r} is {v.dtype} on {v.device}, expected {want} on "
+                               f"{p.device}")
+    for k in _MICRO_KEYS[:3]:
+        if st[k].shape != p.shape or not st[k].is_contiguous():
+            raise RuntimeError(f"CRESSO5 micro route: state {k!r} must be contiguous with the parameter's shape")
+    for k in _MICRO_KEYS[3:]:
+        if st[k].numel() != 1:
+            raise RuntimeError(f"CRESSO5 micro route: state {k!r} has {st[k].numel()} elements, expected one")
+
+
 class _ScalarBatch:
     """Cached plan of the scalar-route and micro-route tensors of one param
     group on one device (one library plan; micro tensors carry route 1)."""
 
-    def __init__(self, params: List[Tensor], grads: List[Tensor], states: List[dict], group: dict,
-                 device: torch.device):
+    def __init__(self, params: List[Tensor], grads: List[Tensor], states: List[dict], keys: List[tuple], descs,
+                 group: dict, device: torch.device):
+        """keys: _SCALAR_KEYS or _MICRO_KEYS per tensor; descs: descriptors_of these tensors."""
         lib = _native.load()
         self.lib = lib
         self.params = params
         self.states = states
         self.device = device
-        self.pptrs = [p.data_ptr() for p in params]
-        self.shapes = [(p.shape, p.dtype) for p in params]
         self.gdtypes = [g.dtype for g in grads]   # the plan's descriptors fix the grad dtype
         self.hyper_key = self.key_of(group)
         # the plan holds the state tensors' addresses and step counts: what it
-        # was made from stays referenced here and is compared on every step
-        self.keys = [_MICRO_KEYS if "micro_energy" in st else _SCALAR_KEYS for st in states]
-        self.planned = [[(st[k], st[k].data_ptr()) for k in ks] for st, ks in zip(states, self.keys)]
-        self.step0 = [int(st["step"]) for st in states]
+        # was made from stays referenced (by the guard, or in self.planned) and
+        # is compared on every step
+        self.keys = keys
         self.ran = 0
-        descs = (_native.ScalarDesc * len(params))()
-        for i, (p, g, st) in enumerate(zip(params, grads, states)):
-            d = descs[i]
-            d.param = p.data_ptr()
-            d.grad = g.data_ptr()
-            for j, (_, ptr) in enumerate(self.planned[i]):
-                d.state[j] = ptr
-            d.route = _native.ROUTE_MICRO if self.keys[i] is _MICRO_KEYS else _native.ROUTE_SCALAR
-            for a, s in enumerate(p.shape):
-                d.shape[a] = int(s)
-            d.numel = p.numel()
-            d.ndim = p.ndim
-            d.param_dtype = _native.DTYPE_CODE[p.dtype]
-            d.grad_dtype = _native.DTYPE_CODE[g.dtype]
-            d.step = int(st["step"])
         self.descs = descs
         hyper = _native.hyper_from_group(group)
         plan = lib.cresso_scalar_plan_create(descs, len(params), ctypes.byref(hyper))
@@ -160,10 +170,38 @@ class _ScalarBatch:
                 self.guard = hb.BatchGuard(list(params), list(states), self.keys)
             except (ValueError, RuntimeError):
                 self.guard = None
+        if self.guard is None:
+            self.shapes = [(p.data_ptr(), p.shape, p.dtype) for p in params]
+            self.step0 = [int(st["step"]) for st in states]
+            self.planned = [[(st[k], st[k].data_ptr()) for k in ks] for st, ks in zip(states, self.keys)]
 
     @staticmethod
-    def key_of(group: dict):
-        return tuple(group[k] for k in _native.HYPER_DOUBLES if k != "lr") + (group["warmup_steps"], group["maximize"])
+    def descriptors_of(params: List[Tensor], grads: List[Tensor], states: List[dict], keys: List[tuple]):
+        """The library's descriptors; their states are checked (RuntimeError)."""
+        descs = (_native.ScalarDesc * len(params))()
+        hb = _native.host_batch()
+        if hb is not None and hb.scalar_descs(params, grads, states, keys, [3 if ks is _MICRO_KEYS else 0 for ks in keys],
+                                              ctypes.addressof(descs)):
+            return descs
+        for i, (p, g, st, ks) in enumerate(zip(params, grads, states, keys)):
+            (_check_micro_state if ks is _MICRO_KEYS else _check_scalar_state)(p, st)
+            d = descs[i]
+            d.param = p.data_ptr()
+            d.grad = g.data_ptr()
+            for j, k in enumerate(ks):
+                d.state[j] = st[k].data_ptr()
+            d.route = _native.ROUTE_MICRO if ks is _MICRO_KEYS else _native.ROUTE_SCALAR
+            for a, s in enumerate(p.shape):
+                d.shape[a] = int(s)
+            d.numel = p.numel()
+            d.ndim = p.ndim
+            d.param_dtype = _native.DTYPE_CODE[p.dtype]
+            d.grad_dtype = _native.DTYPE_CODE[g.dtype]
+            d.step = int(st["step"])
+        return descs
+
+    # the group's hyperparameters other than the learning rate, as a tuple
+    key_of = staticmethod(operator.itemgetter(*[k for k in _native.HYPER_DOUBLES if k != "lr"], "warmup_steps", "maximize"))
 
     def states_hold(self, states: List[dict]) -> bool:
         """The states are the dicts the plan was made from, with the planned
@@ -183,7 +221,7 @@ class _ScalarBatch:
         if self.guard is not None:
             return self.guard.holds(params, state)
         return (len(params) == len(self.params) and all(a is b for a, b in zip(params, self.params))
-                and [p.data_ptr() for p in params] == self.pptrs and [(p.shape, p.dtype) for p in params] == self.shapes
+                and [(p.data_ptr(), p.shape, p.dtype) for p in params] == self.shapes
                 and all(p.is_contiguous() for p in params) and self.states_hold(states))
 
     @staticmethod
@@ -404,8 +442,7 @@ class CRESSO5(Optimizer):
                   "hard_channel_min_size", "thin_matrix_hard_cutoff", "thin_matrix_max_width", "thin_matrix_min_aspect",
                   "thin_matrix_route", "cuda_ops")
 
-    def _steady_key(self, group: dict) -> tuple:
-        return tuple(group[k] for k in self._PLAN_KEYS)
+    _steady_key = staticmethod(operator.itemgetter(*_PLAN_KEYS))
 
     def _fast_spectral(self, gi: int, group: dict) -> bool:
         """Steady-state path of a group with spectral tensors: the same
@@ -504,7 +541,7 @@ class CRESSO5(Optimizer):
                 if len(st) == 0:
                     st = self._init_micro(p)
                 else:
-                    self._check_micro_state(p, st)
+                    _check_micro_state(p, st)
                 scalar_ps.append(data)
                 scalar_gs.append(grad)
                 scalar_st.append(st)
@@ -529,11 +566,11 @@ class CRESSO5(Optimizer):
         self._group_other[gi] = other
 
         # (before the spectral launches: a refused state leaves every tensor as it was)
-        batch = self._scalar_plan(gi, group, scalar_ps, scalar_gs, scalar_st)
+        batch, made_of = self._scalar_plan(gi, group, scalar_ps, scalar_gs, scalar_st)
 
         def scalar_step() -> None:
             if scalar_ps:
-                self._step_scalar_batch(gi, group, batch, scalar_ps, scalar_gs, scalar_st)
+                self._step_scalar_batch(gi, group, batch, made_of, scalar_ps, scalar_gs, scalar_st)
             else:
                 self._batches.pop((gi, "scalar"), None)
 
@@ -550,54 +587,26 @@ class CRESSO5(Optimizer):
             p.detach().copy_(data)
 
     def _scalar_plan(self, gi: int, group: dict, scalar_ps: List[Tensor], scalar_gs: List[Tensor],
-                     scalar_st: List[dict]) -> Optional[_ScalarBatch]:
-        """The cached plan if it describes these tensors; None, with their
-        devices and states checked, when a new one is needed."""
+                     scalar_st: List[dict]) -> Tuple[Optional[_ScalarBatch], Optional[tuple]]:
+        """(the cached plan, None) if it describes these tensors; else (None,
+        what a new one is made of), with their devices and states checked."""
         if not scalar_ps:
-            return None
+            return None, None
         if len({p.device for p in scalar_ps}) != 1:
             raise RuntimeError("CRESSO5 scalar route: all parameters of a group must be on one device")
         batch = self._batches.get((gi, "scalar"))
         if batch is not None and batch.matches(scalar_ps, scalar_st, [g.dtype for g in scalar_gs], group, self.state):
-            return batch
-        for p, st in zip(scalar_ps, scalar_st):
-            if "micro_energy" not in st:
-                self._check_scalar_state(p, st)
-        return None
+            return batch, None
+        keys = [_MICRO_KEYS if "micro_energy" in st else _SCALAR_KEYS for st in scalar_st]
+        return None, (keys, _ScalarBatch.descriptors_of(scalar_ps, scalar_gs, scalar_st, keys))
 
-    def _step_scalar_batch(self, gi: int, group: dict, batch: Optional[_ScalarBatch], scalar_ps: List[Tensor],
-                           scalar_gs: List[Tensor], scalar_st: List[dict]) -> None:
+    def _step_scalar_batch(self, gi: int, group: dict, batch: Optional[_ScalarBatch], made_of: Optional[tuple],
+                           scalar_ps: List[Tensor], scalar_gs: List[Tensor], scalar_st: List[dict]) -> None:
         if batch is None:
             self._batches[(gi, "scalar")] = None  # drop the old plan first
-            batch = _ScalarBatch(scalar_ps, scalar_gs, scalar_st, group, scalar_ps[0].device)
+            batch = _ScalarBatch(scalar_ps, scalar_gs, scalar_st, *made_of, group, scalar_ps[0].device)
             self._batches[(gi, "scalar")] = batch
         batch.run(group, [g.data_ptr() for g in scalar_gs])
-
-    @staticmethod
-    def _check_scalar_state(p: Tensor, st: dict) -> None:
-        want = _state_dtype(p.dtype)
-        for k in _SCALAR_KEYS:
-            v = st.get(k)
-            if not torch.is_tensor(v) or v.dtype != want or v.device != p.device or v.numel() != 1:
-                got = f"{v.dtype} with {v.numel()} elements on {v.device}" if torch.is_tensor(v) else type(v).__name__
-                raise RuntimeError(f"CRESSO5 scalar route: state {k!r} is {got}, expected one {want} on {p.device}")
-
-    @staticmethod
-    def _check_micro_state(p: Tensor, st: dict) -> None:
-        want = _state_dtype(p.dtype)
-        for k in _MICRO_KEYS:
-            if k not in st:
-                raise RuntimeError(f"CRESSO5 micro route: state {k!r} is missing (the state belongs to another route)")
-            v = st[k]
-            if v.dtype != want or v.device != p.device:
-                raise RuntimeError(f"CRESSO5 micro route: state {k!r} is {v.dtype} on {v.device}, expected {want} on "
-                                   f"{p.device}")
-        for k in _MICRO_KEYS[:3]:
-            if st[k].shape != p.shape or not st[k].is_contiguous():
-                raise RuntimeError(f"CRESSO5 micro route: state {k!r} must be contiguous with the parameter's shape")
-        for k in _MICRO_KEYS[3:]:
-            if st[k].numel() != 1:
-                raise RuntimeError(f"CRESSO5 micro route: state {k!r} has {st[k].numel()} elements, expected one")
 
     def _spectral_step(self, items, group: dict, between=None) -> None:
         """Every spectral tensor of the group: (param, grad, state) each;

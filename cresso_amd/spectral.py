@@ -412,7 +412,12 @@ class SteadyStep:
         self.workspaces = [weakref.ref(u[0]) for u in units]
 
     def ready(self) -> bool:
-        return self.version == self.engine.version and all(ws() is not None for ws in self.workspaces)
+        if self.version != self.engine.version:
+            return False
+        for ws in self.workspaces:
+            if ws() is None:
+                return False
+        return True
 
     def fill(self, state: dict) -> bool:
         return self.ready() and self.guard.fill(state, ctypes.addressof(self.descs))

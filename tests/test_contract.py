@@ -328,10 +328,40 @@ def test_host_batch_guard_compares_layouts_and_states():
     assert not guard.holds(ps, state)
     states[0]["step"] = 7
     assert guard.holds(ps, state)
-    states[0]["new"] = 1
+    states[0]["other"] = 1   # (no entry of the plan's)
+    assert guard.holds(ps, state)
+    del states[0]["q"]
     assert not guard.holds(ps, state)
     with pytest.raises(ValueError):
         hb.BatchGuard(ps, states, [("q", "missing")] * 3)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.bfloat16, torch.float16])
+def test_scalar_descriptors_are_the_same_from_cpp_and_python(dtype, monkeypatch):
+    import ctypes
+
+    from cresso_amd.optimizer import _MICRO_KEYS, _SCALAR_KEYS, _ScalarBatch
+
+    opt = CRESSO5([torch.nn.Parameter(torch.zeros(1))], micro_field_max_size=20)
+    ps = [torch.nn.Parameter(torch.zeros(s, dtype=dtype)) for s in ((), (7,), (3, 5), (40, 2, 3), (1,) * 8)]
+    micro = [False, True, True, False, False]
+    keys = [_MICRO_KEYS if m else _SCALAR_KEYS for m in micro]
+    sts = [opt._init_micro(p) if m else opt._init_scalar(p) for p, m in zip(ps, micro)]
+    for i, st in enumerate(sts):
+        st["step"] = i
+    gs = [torch.zeros_like(p) for p in ps]
+    out = (_native.ScalarDesc * 5)()
+    assert _native.host_batch().scalar_descs(ps, gs, sts, keys, [3 if m else 0 for m in micro], ctypes.addressof(out))
+    fast = bytes(_ScalarBatch.descriptors_of(ps, gs, sts, keys))
+    monkeypatch.setattr(_native, "host_batch", lambda: None)
+    assert fast == bytes(_ScalarBatch.descriptors_of(ps, gs, sts, keys))
+    monkeypatch.undo()
+    sts[1]["micro_impulse"] = sts[1]["micro_impulse"].view(7, 1)
+    with pytest.raises(RuntimeError, match="micro_impulse"):
+        _ScalarBatch.descriptors_of(ps, gs, sts, keys)
+    sts[0]["q"] = torch.zeros(2)
+    with pytest.raises(RuntimeError, match="state 'q'"):
+        _ScalarBatch.descriptors_of(ps, gs, sts, keys)
 
 
 def test_spectral_lane_assignment():
