@@ -798,7 +798,12 @@ constexpr int SR_WIDE_NT = 256;              // threads per block of the wide fo
 // atomics.  us a step of fp32 tensors with 8192 / 4096 / 2048 a block: 8 x
 // (8192,16) 111 / 78 / 63, 3 x (20000,7) 134 / 95 / 82, (65536,64) 135 / 125 /
 // 156, 66 x (5632,16) 156 / 134 / 146, 132 x (5632,16) and (16,5632) 208 / 218
-// / 240.
+// / 240.  bf16 (fp16 alike), attention adapters by layers of (width, rank):
+// 1 x (2100,64), 1.1 M elements, 116 / 84 / 75, 2 x (3000,40), 1.9 M, 144 / 124
+// / 120, 4 x (4224,33), 4.5 M, 217 / 204 / 217, 7 x (2100,64), 7.5 M, 172 / 156
+// / 169, 10 x (3000,40), 9.6 M, 273 / 278 / 316, 16 x (4224,33), 17.8 M, 423 /
+// 436 / 518.  (At 7 to 9 M elements the two larger chunks change places with
+// the shape: 7 x (4224,33) 247 / 247 in bf16 but 250 / 270 in fp32.)
 inline int64_t wide_chunk(int64_t elements) { return elements <= 3 << 19 ? 2048 : (elements <= 1 << 23 ? 4096 : 8192); }
 constexpr int64_t SR_MIDDLE_WIDE = 5 << 19;  // elements of middle tensors up to which they join the wide form (build_plan)
 constexpr int64_t SR_WIDE_MIN = SR_RESIDENT_MAX + 1;   // non-resident tensors this large use the wide form

@@ -982,7 +982,9 @@ __global__ __launch_bounds__(256) void part_reduce_kernel(
 // columns) for this step's sweep 2.  With weight decay and the matrix-core
 // sweeps it stores the force (fout, the tangent field's place): they then read
 // 4 bytes an element twice, where grad and param together are 4 (16-bit) or 8.
-template <typename PT, typename GT, bool V4>
+// FORCE: a kernel of its own; the stores under a condition of the launch cost
+// every other step too (sweep 1 of a lone (2048,2048) fp32 6.4 -> 7.0 us).
+template <typename PT, typename GT, bool V4, bool FORCE>
 __global__ __launch_bounds__(SP_NT) void sweep1_kernel(
     Geom g, const GT* __restrict__ grad, const PT* __restrict__ param, double* __restrict__ part,
     unsigned long long* __restrict__ rowfx, unsigned long long* __restrict__ colfx, Ctrl* __restrict__ ctrl,
@@ -992,7 +994,7 @@ __global__ __launch_bounds__(SP_NT) void sweep1_kernel(
         grad = (const GT*)d.grad; param = (const PT*)d.param; fr_state = (const float*)d.force_rms;
     }
     part = lane_at(part, L); rowfx = lane_at(rowfx, L); colfx = lane_at(colfx, L); ctrl = lane_at(ctrl, L);
-    if (fout) fout = lane_at(fout, L);
+    if constexpr (FORCE) fout = lane_at(fout, L);
     __shared__ float red[4];
     if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->fr_prev = *fr_state;   // every block of sweep 2 reads the old value
     {
@@ -1031,7 +1033,7 @@ __global__ __launch_bounds__(SP_NT) void sweep1_kernel(
                 for (int u = 0; u < UN; ++u)
 #pragma unroll
                     for (int c = 0; c < VW; ++c) f[u][c] = sg * f[u][c] + wd * pv[u][c];
-                if (fout)
+                if constexpr (FORCE)
 #pragma unroll
                     for (int u = 0; u < UN; ++u)
 #pragma unroll
@@ -1053,7 +1055,7 @@ __global__ __launch_bounds__(SP_NT) void sweep1_kernel(
                 LdV<PT, VW>::go(param, e, pv);
 #pragma unroll
                 for (int c = 0; c < VW; ++c) f[c] = sg * f[c] + wd * pv[c];
-                if (fout)
+                if constexpr (FORCE)
 #pragma unroll
                     for (int c = 0; c < VW; c += 4) St4<float>::go(fout, e + c, f + c);
             }
@@ -1079,7 +1081,7 @@ __global__ __launch_bounds__(SP_NT) void sweep1_kernel(
         float f = sg * ld(grad, i);
         if (wd_on) {
             f = f + wd * ld(param, i);
-            if (fout) fout[i] = f;
+            if constexpr (FORCE) fout[i] = f;
         }
         a += f * f;
         m = fmaxf(m, fabsf(f));
@@ -2217,10 +2219,15 @@ __global__ __launch_bounds__(SP_NT, (occ2m<RM, KC>())) void sweep2m_kernel(
         for (int r = 0; r < 4; ++r) rt[r] = row16_total(rs[r]);
         if (li < 4) s_wrow[wv * g.PR + 16 * tr + 4 * lg + li] = li == 0 ? rt[0] : (li == 1 ? rt[1] : (li == 2 ? rt[2] : rt[3]));
     }
-    // (from the slab's first column, or a wave's width to the left of it)
-    const int64_t slab0 = (int64_t)(blockIdx.x % g.slabs) * SP_NT;
-    if (hi_on && hi_block(g, part1, t.r0 * g.cols + (EDGE && slab0 > 0 ? slab0 - SP_WCOLS : slab0), nr,
-                          EDGE ? SP_NT + SP_WCOLS : SP_NT, inv_s, eps, pw, kmf)) {
+    // EDGE: from the slab's first column, or a wave's width to the left of it.
+    // (Full tiles: their base, held anyway; computed anew it costs registers
+    // that rank 16 does not have, (8192,8192) bf16 197 -> 206 us.)
+    int64_t hbase = base;
+    if constexpr (EDGE) {
+        const int64_t slab0 = (int64_t)(blockIdx.x % g.slabs) * SP_NT;
+        hbase += slab0 > 0 ? slab0 - SP_WCOLS : 0;   // (base: the panel's first element)
+    }
+    if (hi_on && hi_block(g, part1, hbase, nr, EDGE ? SP_NT + SP_WCOLS : SP_NT, inv_s, eps, pw, kmf)) {
         // high-word pass: the lane's elements again
         const unsigned long long lo_k = to_fixed_u(yk);   // what the loop added for y >= 2^k
         for (int tr = tr0; tr < ntr; ++tr)
@@ -3712,11 +3719,11 @@ __global__ __launch_bounds__(SP_NT, (occ4m<RM, KC>())) void sweep4m_kernel(
     // row in flight while one is processed.  Else one set, refilled tile by
     // tile as in sweep 3m (loads three tiles ahead of their use): 40 registers
     // fewer at rank 8, where the edge form spills 10 with two sets (sweep 4m of
-    // (50257,768) 112 -> 104 us), and 16 fewer at rank 16 ((8192,8192): 220 ->
-    // 210 us).  The full tiles of rank 8 keep two sets: a lone (2048,2048)
-    // tensor has one wave a SIMD and nothing else to hide its loads (16.5 us,
-    // 18.2 with one set).  The first row's loads go out before the block's
-    // set-up, so that memory is busy during it.
+    // (50257,768) 112 -> 100 us), and 16 fewer at rank 16 ((8192,8192) bf16
+    // alone: 212 -> 202 us).  The full tiles of rank 8 keep two sets: a lone
+    // (2048,2048) tensor has one wave a SIMD and nothing else to hide its loads
+    // (16.5 us, 18.2 with one set).  The first row's loads go out before the
+    // block's set-up, so that memory is busy during it.
     constexpr bool DB = RM <= 8 && !EDGE;
     float xv[DB ? 2 : 1][16];
     uint32_t bv[DB ? 2 : 1][16];
@@ -3876,7 +3883,7 @@ __global__ __launch_bounds__(SP_NT, (occ4m<RM, KC>())) void sweep4m_kernel(
 
 
 // Sweep 5 after the matrix-core sweeps, whose drive field is 4-row
-// interleaved (q4_base): a thread takes four rows by four columns at a time,
+// interleaved (q4_lane_bytes): a thread takes four rows by four columns at a time,
 // the drive as four float4 (one per column) and the param as four vectors of
 // four (one per row), transposed in registers; params not aligned for vector
 // access take one column of four rows at a time.  Same grid as sweep 5.
@@ -4344,12 +4351,19 @@ int32_t run_step(const cresso_spectral_plan& P, const cresso_spectral_desc* hd, 
     const bool edge = medge_mode(g, h);
     // with weight decay they read the force that sweep 1 leaves in tbuf
     float* fout = mf && h.weight_decay != 0.0 ? tbuf : nullptr;
-    if (v4)
-        hipLaunchKernelGGL((sweep1_kernel<PT, GT, true>), grid1, blk, 0, s, g, grad, param, part1, rowfx, colfx, ctrl,
-                           st.force_rms, fout, L, h);
-    else
-        hipLaunchKernelGGL((sweep1_kernel<PT, GT, false>), grid1, blk, 0, s, g, grad, param, part1, rowfx, colfx, ctrl,
-                           st.force_rms, fout, L, h);
+    auto sweep1 = [&](auto vec, auto force) {
+        hipLaunchKernelGGL((sweep1_kernel<PT, GT, decltype(vec)::value, decltype(force)::value>), grid1, blk, 0, s, g, grad,
+                           param, part1, rowfx, colfx, ctrl, st.force_rms, fout, L, h);
+    };
+    auto form1 = [&](auto force) { v4 ? sweep1(std::true_type{}, force) : sweep1(std::false_type{}, force); };
+    if constexpr (MX) {
+        if (fout)
+            form1(std::true_type{});
+        else
+            form1(std::false_type{});
+    } else {
+        form1(std::false_type{});
+    }
     // the matrix-core sweeps write per-block histogram partials (hpart),
     // which part_reduce sums into hist; the general sweeps add into hist
     const bool m2 = mf;

@@ -213,13 +213,13 @@ int32_t plan_spectral(const int64_t* shape, int32_t ndim, const int64_t* freqs, 
     // The matrix-core sweeps take panels of 16, 32 or 64 rows (a last panel of
     // fewer rows overlaps the one before it).  Fewer rows make more, shorter
     // blocks: each repeats the set-up of its tables, and a lone tensor fills
-    // the chip sooner.  us a step of one fp32 tensor, rank 8, with panels of
-    // 16 / 32 / 64 rows: (512,512) 57 / 66 / 82, (1024,1024) 69 / 75 / 91,
-    // (3072,768) 85 / 87 / 95, (2048,2048) 102 / 96 / 104, (5632,2048)
-    // 183 / 174 / 167, (4096,4096) 233 / 215 / 207, (50257,768) 556 / 480 /
-    // 467.  16 rows up to 640 blocks of them, then 32, and 64 from 256 blocks
-    // on: there (2048,2048) alone would gain from 32, but batches of them
-    // lose (a transformer's 88 in one group: 2.4 % of its layers' time).
+    // the chip sooner.  us a step, fp32, rank 8, two tables of 64 bins, with
+    // panels of 16 / 32 / 64 rows: (512,512) 58 / 67 / 81, (1024,1024) 63 / 70
+    // / 84, (3072,768) 78 / 81 / 88, (2048,2048) 91 / 87 / 96, (5632,2048) 159
+    // / 150 / 143, (4096,4096) 207 / 189 / 179, (50257,768) 487 / 446 / 442.
+    // 16 rows up to 640 blocks of them, then 32, and 64 from 256 blocks on:
+    // there (2048,2048) alone would gain from 32, but batches of it lose (4 of
+    // them 217 / 207 with 32 / 64 rows, 16 of them 699 / 667).
     // (Four tables skip the 32: the partial histograms of twice the blocks
     // would take plans past the no-alloc entry's workspace limit.)
     P.general_rows = (int32_t)pr;
