@@ -165,15 +165,18 @@ class _ScalarBatch:
         self.gbuf = self.gptr_type()
         self.guard = None
         hb = _native.host_batch()
-        if hb is not None and all(p.grad is not None for p in params):   # (not for contiguous copies)
+        self.planned: Optional[List[list]] = None
+        if any(p.grad is None for p in params):   # contiguous copies, which no later step has again
+            return
+        if hb is not None:
             try:
                 self.guard = hb.BatchGuard(list(params), list(states), self.keys)
+                return
             except (ValueError, RuntimeError):
-                self.guard = None
-        if self.guard is None:
-            self.shapes = [(p.data_ptr(), p.shape, p.dtype) for p in params]
-            self.step0 = [int(st["step"]) for st in states]
-            self.planned = [[(st[k], st[k].data_ptr()) for k in ks] for st, ks in zip(states, self.keys)]
+                pass
+        self.shapes = [(p.data_ptr(), p.shape, p.dtype) for p in params]
+        self.step0 = [int(st["step"]) for st in states]
+        self.planned = [[(st[k], st[k].data_ptr()) for k in ks] for st, ks in zip(states, self.keys)]
 
     @staticmethod
     def descriptors_of(params: List[Tensor], grads: List[Tensor], states: List[dict], keys: List[tuple]):
@@ -220,7 +223,7 @@ class _ScalarBatch:
             return False
         if self.guard is not None:
             return self.guard.holds(params, state)
-        return (len(params) == len(self.params) and all(a is b for a, b in zip(params, self.params))
+        return (self.planned is not None and len(params) == len(self.params) and all(a is b for a, b in zip(params, self.params))
                 and [(p.data_ptr(), p.shape, p.dtype) for p in params] == self.shapes
                 and all(p.is_contiguous() for p in params) and self.states_hold(states))
 
@@ -428,7 +431,7 @@ class CRESSO5(Optimizer):
             return True
         try:
             gptrs = [p.grad.data_ptr() for p in batch.params]
-            states = [self.state[p] for p in batch.params]
+            states = [self.state.get(p) for p in batch.params]
         except (AttributeError, RuntimeError):
             return False
         if (not batch.matches(group["params"], states, [p.grad.dtype for p in batch.params], group, self.state)

@@ -162,6 +162,28 @@ def test_planned_scalar_tensors_follow_changes(group, change):
     KEPT.clear()
 
 
+@pytest.mark.parametrize("group", sorted(GROUPS))
+def test_planned_scalar_tensors_follow_changes_without_the_helper(group, monkeypatch):
+    """All of these changes, one after the other, where the C++ helper is not built."""
+    from cresso_amd import _native
+
+    announce(f"{group} group, no helper")
+    monkeypatch.setattr(_native, "host_batch", lambda: None)
+    gen, pair = _pair(GROUPS[group], **MICRO)
+    changes = {2 + 2 * i: c for i, c in enumerate(CHANGES)}
+
+    def at(k, ps, opt):
+        if k in changes:
+            changes[k](ps, opt)
+            for p in ps:
+                p.grad = 1e-3 * torch.arange(p.numel(), device="cuda", dtype=torch.float32).view(p.shape)
+        if opt is pair[1][1]:
+            opt._batches.clear()
+
+    _steps(gen, pair, 2 * len(changes) + 3, at)
+    KEPT.clear()
+
+
 def _no_q(ps, opt):
     del opt.state[ps[0]]["q"]
 
