@@ -1,6 +1,6 @@
 """Benchmark of the CRESSO5 hot path on one MI355X.
 
-    python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload c1|c2|c3|c4|c5|copy] [--no-cpu]
+    python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload c1|c2|c3|c4|c5|forms|middle|edge|decay|copy] [--no-cpu]
 
 With no --workload, the headline configs run first: C2 gives the line's
 `value`, `ms_per_step`, `roofline`, `cpu_baseline` and `parity`; C3 (the
@@ -16,6 +16,8 @@ Workloads:
       rank 4; per-tensor scale 10^U(-4,-1) times N(0,1e-2).
   c4: the 1.2 B-element transformer set (fp32, rank 8; inputs drawn on the device).
   c5: bf16 (8192,8192) and fp32 conv / 3-D tensors at rank 16, F=7, B=256, T=4.
+  forms, middle, edge, decay: for profiles only (PROFILE_ONLY), the kernels that
+      c2 to c5 do not run.
   copy: calibration only -- torch's device copy of a 256 MiB fp32 buffer, the
       plain copy kernel of known size that scales rocprofv3's FETCH_SIZE and
       WRITE_SIZE counters to bytes.
@@ -48,6 +50,7 @@ leg's own inputs (cpu_and_parity).
 from __future__ import annotations
 
 import argparse
+import functools
 import json
 import os
 import subprocess
@@ -80,19 +83,27 @@ def make_c3(device, pool=4, seed=0):
     return params, grads, kwargs, shapes, scales
 
 
-def make_forms(device, pool=1, seed=0):
-    """Profile-only group (not a bench line) for the scalar route's other launch
-    forms: 256 small thin tensors (scalar_stream_kernel), 4 large thin tensors
-    (the wide form's passes and finishes) and 64 micro-route tensors
-    (micro_kernel), one scalar plan."""
+# Profile-only groups (not bench lines): the kernels that C2 to C5 do not run.
+#   forms: 256 small thin tensors (scalar_small_kernel), 4 large ones (the wide
+#     form's passes and finishes), 64 micro tensors (micro_small_kernel)
+#   middle: (16,2048) and (2048,16) in one launch of scalar_mid_kernel, and 300
+#     larger tensors, a workgroup each (scalar_stream_kernel)
+#   edge: the edge form of the matrix-core sweeps (a ragged row count)
+#   decay: the same with a force stored by sweep 1 (weight decay)
+PROFILE_ONLY = {
+    "forms": ([(999, 7)] * 256 + [(262144, 32)] * 4 + [(64, 64)] * 64, torch.float32, dict(rank=4, micro_field_max_size=4096)),
+    "middle": ([(16, 2048)] * 132 + [(2048, 16)] * 110 + [(40, 1000)] * 300, torch.float32, dict(rank=4)),
+    "edge": ([(50257, 768)], torch.float32, dict(rank=8, max_frequency=5)),
+    "decay": ([(5632, 2048)], torch.bfloat16, dict(rank=8, max_frequency=5, weight_decay=0.01)),
+}
+
+
+def make_profile_only(name, device, pool=1, seed=0):
+    shapes, dtype, kw = PROFILE_ONLY[name]
     gen = torch.Generator().manual_seed(seed)
-    shapes = [(999, 7)] * 256 + [(262144, 32)] * 4 + [(64, 64)] * 64
-    params = [torch.nn.Parameter((0.02 * torch.randn(s, generator=gen)).to(device)) for s in shapes]
-    grads = []
-    for _ in range(pool):
-        grads.append([(1e-3 * torch.randn(s, generator=gen)).to(device) for s in shapes])
-    kwargs = dict(lr=2e-3, rank=4, hash_bins=64, hash_tables=2, micro_field_max_size=4096)
-    return params, grads, kwargs, shapes, None
+    params = [torch.nn.Parameter((0.02 * torch.randn(s, generator=gen)).to(device, dtype)) for s in shapes]
+    grads = [[(1e-3 * torch.randn(s, generator=gen)).to(device, dtype) for s in shapes] for _ in range(pool)]
+    return params, grads, dict(lr=2e-3, hash_bins=64, hash_tables=2, **kw), shapes, None
 
 
 def make_c2(device, pool=4, seed=0):
@@ -500,7 +511,8 @@ def rocprof_summary(dirs, calib=None, launches=None):
     print("\n".join(out))
 
 
-MAKERS = {"c1": make_c1, "c2": make_c2, "c3": make_c3, "c4": make_c4, "c5": make_c5, "forms": make_forms}
+MAKERS = {"c1": make_c1, "c2": make_c2, "c3": make_c3, "c4": make_c4, "c5": make_c5,
+          **{k: functools.partial(make_profile_only, k) for k in PROFILE_ONLY}}
 # the timing leg of the full C4 set draws its inputs on the device
 # C3's 840 grads are set once: assigning p.grad for 840 tensors in Python costs
 # ~0.3 us each, more than the GPU step, and is input refresh, not optimizer work
@@ -627,8 +639,10 @@ WORKLOAD_NAMES = {"c1": "C1: (2048,2048) fp32 spectral/hash route, rank 8, F=5, 
                         "(5632,2048), down (2048,5632), two (2048,) norms), rank 8, F=5, B=64, T=2",
                   "c5": "C5: bf16 (8192,8192), fp32 (512,256,3,3), (256,256,3,3), (64,512,512), rank 16, F=7, "
                         "B=256, T=4",
-                  "forms": "profile-only: 256 x (999,7) scalar stream form, 4 x (262144,32) wide form, 64 x (64,64) "
-                           "micro route, fp32"}
+                  "forms": "profile-only: 256 x (999,7) small, 4 x (262144,32) wide form, 64 x (64,64) micro route, fp32",
+                  "middle": "profile-only: 132 x (16,2048) and 110 x (2048,16) middle, 300 x (40,1000) stream form, fp32",
+                  "edge": "profile-only: (50257,768) fp32 spectral/hash route, rank 8, B=64, T=2",
+                  "decay": "profile-only: (5632,2048) bf16, weight decay 0.01, rank 8, B=64, T=2"}
 
 
 def measure(workload, args):
@@ -675,7 +689,7 @@ def main():
     ap.add_argument("--gpus", type=int, default=1)
     ap.add_argument("--steps", type=int, default=20)
     ap.add_argument("--warmup", type=int, default=5)
-    ap.add_argument("--workload", choices=["c1", "c2", "c3", "c4", "c5", "forms", "copy"], default=None)
+    ap.add_argument("--workload", choices=["c1", "c2", "c3", "c4", "c5", *PROFILE_ONLY, "copy"], default=None)
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--rocprof-summary", default=None, nargs="+", metavar="DIR")
     ap.add_argument("--calib", default=None, nargs="+", metavar="DIR")
