@@ -212,6 +212,12 @@ def load() -> ctypes.CDLL:
             ver = int(lib.cresso_hip_abi_version())
             if ver != ABI_VERSION:
                 raise RuntimeError(f"{path} has ABI version {ver}, expected {ABI_VERSION}")
+            # The library's error message is thread-local.  Until a thread has
+            # touched the newest library with thread-local data, each access to
+            # any library's goes the dynamic linker's slow way: torch's host
+            # calls took 10 to 25 % longer (torch.empty(3) 487 -> 547 ns) for
+            # as long as the process ran.
+            lib.cresso_hip_last_error()
         except Exception as exc:  # remembered: later calls fail the same way
             _ERR = exc
             raise RuntimeError(f"CRESSO5 CUDA ops failed to load: {exc}") from exc
